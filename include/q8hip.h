@@ -239,7 +239,8 @@ int q8_pack_weight(const float* W, int64_t rows, int64_t cols, int axis, int gra
  *   bias (may be NULL): fround(y + bias[n]); act: Q8_ACT_*.
  * zpA / zpB must be 0 in this build (Q8_ERR_UNSUPPORTED otherwise).
  * Routes M <= 16 to the GEMV kernel.  K % 16 != 0 or A / B not 16-byte
- * aligned take a generic one-thread-per-output kernel (exact, slow);
+ * aligned take an MFMA kernel that loads its operands through registers
+ * (exact; up to half the rate of the aligned one);
  * q8_generic_gemm_launches counts those launches. */
 int q8_gemm(const int8_t* A, const int8_t* B, int64_t M, int64_t N, int64_t K,
             int32_t zpA, int32_t zpB,
@@ -282,7 +283,7 @@ int q8_gemm_glu(const int8_t* A, const int8_t* B, int64_t M, int64_t F, int64_t 
                 int sA_mode, const double* sB, int sB_mode, const float* bias, float* h, void* workspace,
                 size_t workspace_bytes, void* stream);
 
-/* Launches of the generic (non-MFMA) GEMM kernel since the library was
+/* Launches of the general GEMM kernel since the library was
  * loaded, over all devices and threads: q8_gemm / q8_quantized_dot calls
  * whose K is not a multiple of 16 or whose operands are not 16-byte
  * aligned.  No counterpart in the reference (its CPU kernels have one
@@ -296,11 +297,12 @@ int q8_generic_gemm_launches(int64_t* count);
  *   out[m,n] = ToInt32( sum_k (A[m,k] - zpA) * (B[n,k] - zpB) )
  * with B in the [N,K] layout (rhs_contracting = [1]).  The reference's
  * QuantizationPass sets non-zero zero points for affine schemes
- * (quantization_pass.ts:303-332, :415-425).  Runs the int8 GEMM / GEMV on
+ * (quantization_pass.ts:303-332, :415-425).  Runs the int8 GEMM on
  * operands made signed (ui8 bytes flipped by 128) and adds the exact
- * zero-point correction from row sums; the caller passes a device
- * workspace of q8_quantized_dot_workspace bytes (0 for i8 operands with
- * zero zero points, where this is q8_gemm with Q8_I32 output). */
+ * zero-point correction from row sums, in one launch, or for very large
+ * products as separate passes in the device workspace of
+ * q8_quantized_dot_workspace bytes that the caller passes (0 for i8 operands
+ * with zero zero points, where this is q8_gemm with Q8_I32 output). */
 int q8_quantized_dot_workspace(int64_t M, int64_t N, int64_t K, int a_dtype, int b_dtype,
                                int32_t zpA, int32_t zpB, size_t* bytes);
 int q8_quantized_dot(const void* A, int a_dtype, const void* B, int b_dtype, int64_t M,

@@ -70,6 +70,7 @@ int init_device(int dev) {
   if (cur != dev && (e = hipSetDevice(dev)) != hipSuccess) return hip_fail(e, "hipSetDevice");
   e = q8::setup_kernel_attributes();
   if (e == hipSuccess) e = q8::setup_w4_attributes();
+  if (e == hipSuccess) e = q8::setup_any_attributes();
   (void)q8::cu_count();
   void* sp = nullptr;
   if (e == hipSuccess) e = hipGetSymbolAddress(&sp, HIP_SYMBOL(scratch));
@@ -596,6 +597,24 @@ int q8_quantized_dot(const void* A, int a_dtype, const void* B, int b_dtype, int
   if (rc != Q8_OK) return rc;
   if (M * N == 0) return Q8_OK;
   hipStream_t st = as_stream(stream);
+  // Zero points and ui8 operands: one launch that flips, sums and corrects
+  // on the way through registers (788 x 1000 x 1500: 4350 -> 16.5 us; 256 x
+  // 4096 x 4096, which the tiled GEMM takes too: 34.2 -> 16.8).  Only very
+  // large aligned products gain more from the direct-to-LDS GEMM than its
+  // separate passes over the operands and the result cost: from 2^37
+  // multiply-adds (4096 x 4096 x 11008 takes 267 us here and 222 us in
+  // passes, 2048 x 11008 x 4096 158 and 178).
+  const bool aligned = K % 16 == 0 && ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B)) & 15) == 0;
+  const bool passes = aligned && M > 16 && (double)M * (double)N * (double)K >= 0x1p37;
+  if ((p.a_u8 || p.b_u8 || p.cA != 0 || p.cB != 0) && !passes) {
+    if (!aligned) q8::g_generic_gemm_launches.fetch_add(1, std::memory_order_relaxed);
+    const int flip = (int)0x80808080u;
+    const q8::AffineDot z{p.a_u8 ? flip : 0, p.b_u8 ? flip : 0, p.cA, p.cB,
+                          (uint32_t)(uint64_t)K * (uint32_t)p.cA * (uint32_t)p.cB};
+    return launched(q8::launch_gemm_any(static_cast<const int8_t*>(A), static_cast<const int8_t*>(B), M, N, K, e,
+                                        &z, out, st),
+                    "q8_quantized_dot launch");
+  }
   int8_t* ws = static_cast<int8_t*>(workspace);
   const int8_t* a = static_cast<const int8_t*>(A);
   const int8_t* b = static_cast<const int8_t*>(B);

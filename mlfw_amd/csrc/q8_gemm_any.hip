@@ -1,0 +1,495 @@
+// q8_gemm_any.hip -- the int8 MFMA GEMM for operands the direct-to-LDS GEMM
+// (q8_gemm.hip) cannot copy: any K (not only multiples of 16), any alignment,
+// and the affine quantized_dot (ui8 operands and zero points in the same
+// launch).
+//
+// What bounds it: the copies.  buffer_load ... lds moves 16-byte chunks at
+// 16-byte aligned addresses, so a row pitch that is not a multiple of 16 has
+// no such form.  Here a lane loads its 16-byte chunk of a row into registers
+// (an unaligned global_load_dwordx4), and writes it to the same swizzled LDS
+// layout with ds_write_b128; the loads of the stage after next are in flight
+// while a stage is multiplied.  The contraction's tail never reads past the
+// row: a chunk that would cross the row's end is loaded 16 bytes before the
+// end and shifted down, zeros coming in.  Passing through registers costs
+// VGPRs and LDS write cycles that the direct copies do not pay, so operands
+// those can take stay with them (launch_gemm).
+//
+// The affine form uses the pass through registers: a ui8 operand's bytes are
+// flipped by 0x80 there (a - 128), and v_dot4 against ones adds up the row
+// sums that the zero-point correction needs, so quantized_dot with zero
+// points reads each operand once and writes its result once -- as separate
+// passes the flips, row sums and correction were up to four more launches.
+//
+// Measured (MI355X, whole calls, before: one thread per output with byte
+// loads): quantized_dot 788 x 1000 x 1500 with ui8 activations 4350 -> 16.5
+// us (the host's share of the call is about 12); dynamic linear 42 x 3777 x
+// 7986 5400 -> 51 us, 1183 x 3917 x 3001 59300 -> 79 us.
+#include <type_traits>
+
+#include "q8_device.h"
+#include "q8_epilogue.h"
+#include "q8_internal.h"
+
+namespace q8 {
+
+namespace {
+
+constexpr int AK = 128;   // K bytes per LDS stage
+
+template <int BM, int BN, int KG>
+struct AnyCfg {
+  static constexpr int WM = BM / 2, WN = BN / 2;        // per-wave sub-tile, waves 2 x 2
+  static constexpr int TM = WM / 32, TN = WN / 32;
+  static constexpr int A_BYTES = BM * AK;
+  static constexpr int STAGE = (BM + BN) * AK;
+  static constexpr int RING = 2 * STAGE;                // a group's stages
+  static constexpr int WAVES = 4;                       // per group
+  static constexpr int LDS = KG * RING + 8 * BM + 4 * (BM + BN);   // + row scales, row and column sums
+  static constexpr int CA = BM / 32, CB = BN / 32;      // 16-byte chunks per lane and stage
+  static_assert(TM >= 1 && TN >= 1 && BM % 64 == 0 && BN % 64 == 0, "tile shape");
+};
+
+// v's 16 bytes moved down by sh bytes (sh >= 0), zeros coming in at the top.
+__device__ __forceinline__ v4i shift_down(v4i v, int sh) {
+  if (sh >= 16) return v4i{0, 0, 0, 0};
+  const int dw = sh >> 2;
+  v4i t = (dw & 1) ? v4i{v.y, v.z, v.w, 0} : v;
+  t = (dw & 2) ? v4i{t.z, t.w, 0, 0} : t;
+  const uint32_t b = (uint32_t)(sh & 3);
+  return v4i{(int)__builtin_amdgcn_alignbyte((uint32_t)t.y, (uint32_t)t.x, b),
+             (int)__builtin_amdgcn_alignbyte((uint32_t)t.z, (uint32_t)t.y, b),
+             (int)__builtin_amdgcn_alignbyte((uint32_t)t.w, (uint32_t)t.z, b),
+             (int)__builtin_amdgcn_alignbyte(0u, (uint32_t)t.w, b)};
+}
+
+__device__ __forceinline__ v4i load16_any(const int8_t* p) {
+  v4i v;
+  __builtin_memcpy(&v, p, 16);   // global_load_dwordx4; any byte address
+  return v;
+}
+
+__device__ __forceinline__ int sum16(v4i v, int s) {
+  s = __builtin_amdgcn_sdot4(v.x, 0x01010101, s, false);
+  s = __builtin_amdgcn_sdot4(v.y, 0x01010101, s, false);
+  s = __builtin_amdgcn_sdot4(v.z, 0x01010101, s, false);
+  return __builtin_amdgcn_sdot4(v.w, 0x01010101, s, false);
+}
+
+// One 128-byte stage: the wave's (32 TM) x (32 TN) sub-tile at (wm, wn).
+template <class C>
+__device__ __forceinline__ void mfma_stage(const int8_t* st, int wm, int wn, int lane, v16i (&acc)[C::TM][C::TN]) {
+  const int r32 = lane & 31, kh = lane >> 5;
+#pragma unroll
+  for (int kk = 0; kk < 4; ++kk) {
+    v4i fa[C::TM], fb[C::TN];
+#pragma unroll
+    for (int i = 0; i < C::TM; ++i) {
+      const int row = wm + 32 * i + r32;
+      fa[i] = *reinterpret_cast<const v4i*>(st + row * AK + 16 * ((2 * kk + kh) ^ swz(row)));
+    }
+#pragma unroll
+    for (int j = 0; j < C::TN; ++j) {
+      const int row = wn + 32 * j + r32;
+      fb[j] = *reinterpret_cast<const v4i*>(st + C::A_BYTES + row * AK + 16 * ((2 * kk + kh) ^ swz(row)));
+    }
+#pragma unroll
+    for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+      for (int j = 0; j < C::TN; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[i], fb[j], acc[i][j], 0, 0, 0);
+  }
+}
+
+// The tile's results (every stage buffer free, a barrier passed): KG groups'
+// partial sums in acc, group grp's buffers at lds + grp * C::RING.
+template <class C, int KG, bool ZP>
+__device__ __forceinline__ void any_epilogue(v16i (&acc)[C::TM][C::TN], int8_t* lds, const double* s_rows,
+                                             const int* sum_a, const int* sum_b, int wave, int grp, int lane,
+                                             int m0, int n0, int wm, int wn, int M, int N, int64_t o_base,
+                                             const GemmEpi& e, const AffineDot& z, const AnyPlan& p,
+                                             void* __restrict__ out) {
+  const int r32 = lane & 31, kh = lane >> 5;
+  int8_t* const ring = lds + grp * C::RING;
+  // Epilogue: a 32-row strip of the wave's sub-tile at a time through its
+  // own LDS region (the stages are no longer read), then a rolled loop, one
+  // epilogue's code, over V = 4 columns per lane stored as one 16-byte (int8
+  // out: 4-byte) quad where every quad is aligned and inside, else over
+  // single columns, the lanes of a row taking consecutive ones.
+  constexpr int PITCH = C::WN + 8;
+  static_assert(C::WAVES * 32 * PITCH * 4 <= C::RING, "strips fit in the stage buffers");
+  // group g's strip of sub-tile `wave`; with KG groups each stores 32 / KG of
+  // the strip's rows, adding the groups' sums
+  int* strip = reinterpret_cast<int*>(ring) + wave * 32 * PITCH;
+  const int* strip0 = reinterpret_cast<const int*>(KG > 1 ? lds : ring) + wave * 32 * PITCH;
+  const bool fp = !e.out_i32;
+  auto strips = [&](auto vc) {
+    constexpr int V = decltype(vc)::value;
+    constexpr int LPR = C::WN / V;                     // lanes per strip row
+    constexpr int RPI = 64 / LPR;                      // strip rows per pass
+    constexpr int NIT = 32 / RPI / KG;
+    static_assert(NIT >= 1, "every group has rows to store");
+    const int col = V * (lane % LPR), qrow = lane / LPR;
+    const int n = n0 + wn + col;
+    const bool live = n < N;
+    double sbn[V];
+    float bn[V];
+    uint32_t zc[V];
+#pragma unroll
+    for (int c = 0; c < V; ++c) {
+      const int nc = live ? n + c : N - 1;
+      sbn[c] = fp && e.mode == 1 ? e.sB[(int64_t)nc * e.sB_stride] : 0.0;
+      bn[c] = e.bias ? e.bias[nc] : 0.0f;
+      zc[c] = 0u;
+      if constexpr (ZP) zc[c] = (uint32_t)z.cA * (uint32_t)sum_b[wn + col + c] + z.kcc;
+    }
+    int64_t at0 = o_base + n, ld = N;       // where column n's elements go
+    if (e.col_blk > 0) {                    // n and the block size fit 31 bits
+      const unsigned blk = (unsigned)n / (unsigned)e.col_blk;
+      at0 = o_base + blk * e.blk_stride + (unsigned)n - blk * (unsigned)e.col_blk;
+      ld = e.ld_out;
+    }
+    auto strip_out = [&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      if constexpr (KG > 1 && i > 0) __syncthreads();   // the previous strip's sums have been read
+#pragma unroll
+      for (int j = 0; j < C::TN; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) strip[((r >> 2) * 8 + kh * 4 + (r & 3)) * PITCH + 32 * j + r32] = acc[i][j][r];
+      if constexpr (KG > 1) __syncthreads();
+#pragma unroll 1
+      for (int it = 0; it < NIT; ++it) {
+        const int srow = (grp * NIT + it) * RPI + qrow, trow = wm + 32 * i + srow, m = m0 + trow;
+        uint32_t a[V];
+#pragma unroll
+        for (int c = 0; c < V; ++c) a[c] = 0u;
+#pragma unroll
+        for (int g = 0; g < KG; ++g) {
+          const int* s = strip0 + g * (C::RING / 4) + srow * PITCH + col;
+          if constexpr (V == 4) {
+            const v4i q = *reinterpret_cast<const v4i*>(s);
+#pragma unroll
+            for (int c = 0; c < V; ++c) a[c] += (uint32_t)q[c];
+          } else {
+            a[0] += (uint32_t)s[0];
+          }
+        }
+        if constexpr (ZP) {
+#pragma unroll
+          for (int c = 0; c < V; ++c) a[c] += zc[c] + (uint32_t)z.cB * (uint32_t)sum_a[trow];
+        }
+        if (m >= M || !live) continue;
+        const int64_t at = (int64_t)m * ld + at0;
+        int w[V];
+#pragma unroll
+        for (int c = 0; c < V; ++c) w[c] = (int)a[c];
+        if (fp) {
+          const double sr = s_rows[trow];
+          float y[V];
+#pragma unroll
+          for (int c = 0; c < V; ++c) {
+            y[c] = e.mode == 0 ? (float)((double)w[c] * e.s_out) : mul_acc_f32scale(w[c], (float)(sr * sbn[c]));
+            if (e.bias) y[c] = y[c] + bn[c];
+          }
+          if (e.act == 1) {
+#pragma unroll
+            for (int c = 0; c < V; ++c) y[c] = relu_js(y[c]);
+          } else if (e.act == 2) {
+#pragma unroll
+            for (int c = 0; c < V; ++c) y[c] = silu_js(y[c]);
+          }
+          if (e.out_q8) {
+            int8_t* o = static_cast<int8_t*>(out) + at;
+#pragma unroll
+            for (int c = 0; c < V; ++c) w[c] = requant(y[c], e);
+            if constexpr (V == 4) *reinterpret_cast<int*>(o) = pack4(w[0], w[1], w[2], w[3]);
+            else *o = (int8_t)w[0];
+            continue;
+          }
+#pragma unroll
+          for (int c = 0; c < V; ++c) w[c] = __float_as_int(y[c]);
+        }
+        int* o = static_cast<int*>(out) + at;
+        if constexpr (V == 4) __builtin_nontemporal_store(v4i{w[0], w[1], w[2], w[3]}, reinterpret_cast<v4i*>(o));
+        else *o = w[0];
+      }
+    };
+    strip_out(std::integral_constant<int, 0>{});
+    if constexpr (C::TM > 1) strip_out(std::integral_constant<int, 1>{});
+    static_assert(C::TM <= 2, "strip_out calls cover TM <= 2");
+  };
+  // quads: N, and with column blocks every block's start and pitch, multiples
+  // of 4 elements from an aligned base
+  const bool vec = (N & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0 && (p.o_step & 3) == 0 &&
+                   (e.col_blk == 0 || ((e.col_blk | e.blk_stride | e.ld_out) & 3) == 0);
+  if (vec) strips(std::integral_constant<int, 4>{});
+  else strips(std::integral_constant<int, 1>{});
+}
+
+// out = epilogue(A [M, K] . B [N, K]^T).  ZP: operands flipped by z.xa / z.xb
+// (0 or 0x80808080) and the int32 result corrected by
+// cB * rowsum(a') + cA * rowsum(b') + K * cA * cB (q8_zp.hip states why).
+//
+// KG groups of 4 waves share a tile and take every KG-th K stage, each with
+// a ring of its own; their partial sums meet in LDS (int32 addition does not
+// depend on the order).  A stage costs its load latency whatever the tile, so
+// with a workgroup per CU or less a quarter of the stages in sequence is
+// close to a quarter of the time.
+//
+// CONV: B is a channel-last conv frame (GemmEpi::ConvB); a 16-byte chunk of
+// the contraction lies in one kernel position, and a table in LDS holds every
+// chunk's offset from its column's frame position.
+template <int BM, int BN, int KG, bool ZP, bool CONV>
+__global__ __launch_bounds__(256 * KG, KG == 4 ? 4 : 2)
+void k_qgemm_any(const int8_t* __restrict__ A, const int8_t* __restrict__ B, int M, int N, int K,
+                 int tiles_m, int tiles_n, GemmEpi e, AffineDot z, AnyPlan p, void* __restrict__ out) {
+  using C = AnyCfg<BM, BN, KG>;
+  extern __shared__ __attribute__((aligned(1024))) int8_t lds[];
+  double* s_rows = reinterpret_cast<double*>(lds + KG * C::RING);
+  int* sum_a = reinterpret_cast<int*>(s_rows + BM);
+  int* sum_b = sum_a + BM;
+  int* taps = sum_b + BN;
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = wv & 3, grp = wv >> 2;
+  int8_t* const ring = lds + grp * C::RING;
+  int tm, tn;
+  tile_of((int)blockIdx.x, tiles_m, tiles_n, tm, tn);
+  const int m0 = tm * BM, n0 = tn * BN;
+  const int rows_a = min(BM, M - m0), rows_b = min(BN, N - n0);
+  if (tid < BM)
+    s_rows[tid] = e.mode == 1 && !e.out_i32 && tid < rows_a ? e.sA[(int64_t)(m0 + tid) * e.sA_stride] : 0.0;
+  if (ZP && tid < BM + BN) sum_a[tid] = 0;
+  A += blockIdx.y * p.a_step;
+  B += blockIdx.y * p.b_step;
+  const int64_t o_base = blockIdx.y * p.o_step;
+  if constexpr (CONV) {
+    for (int i = tid; i < (K >> 4); i += 256 * KG) {
+      const uint32_t t = 16u * (uint32_t)i / (uint32_t)p.conv_cg;
+      taps[i] = (int)(convb_tap(e.cb, t) * e.cb.Cg + (16u * (uint32_t)i - t * (uint32_t)p.conv_cg));
+    }
+    __syncthreads();
+  }
+
+  // Copy plan, as k_qgemm's: wave w fills tile rows [w * BM / 4, ...) of A
+  // and its share of B, 8 lanes per row.  A row past the edge repeats the
+  // last one: its results are never stored.
+  const int rl = lane >> 3, c16 = 16 * (lane & 7);
+  const int8_t* pa[C::CA];
+  const int8_t* pb[C::CB];
+  int la[C::CA], lb[C::CB];        // LDS byte offsets within a stage
+#pragma unroll
+  for (int j = 0; j < C::CA; ++j) {
+    const int row = wave * (BM / 4) + 8 * j + rl;
+    pa[j] = A + (m0 + min(row, rows_a - 1)) * p.lda;
+    la[j] = row * AK + 16 * ((lane & 7) ^ swz(row));
+  }
+#pragma unroll
+  for (int j = 0; j < C::CB; ++j) {
+    const int row = wave * (BN / 4) + 8 * j + rl;
+    const int n = n0 + min(row, rows_b - 1);
+    pb[j] = B + (CONV ? (int64_t)convb_row(e.cb, (uint32_t)n) : n * p.ldb);
+    lb[j] = (BM + row) * AK + 16 * ((lane & 7) ^ swz(row));
+  }
+  const int KT = (K + AK - 1) / AK;
+  const int xa = ZP ? z.xa : 0, xb = ZP ? z.xb : 0;
+  int sa[C::CA], sb[C::CB];
+#pragma unroll
+  for (int j = 0; j < C::CA; ++j) sa[j] = 0;
+#pragma unroll
+  for (int j = 0; j < C::CB; ++j) sb[j] = 0;
+  v4i ra[C::CA], rb[C::CB];
+  auto load = [&](int kt) {
+    const int kc = kt * AK + c16;
+    if (CONV || K >= 16) {
+      const int kk = min(kc, K - 16);
+      const int kb = CONV ? taps[kk >> 4] : kk;
+#pragma unroll
+      for (int j = 0; j < C::CA; ++j) ra[j] = load16_any(pa[j] + kk);
+#pragma unroll
+      for (int j = 0; j < C::CB; ++j) rb[j] = load16_any(pb[j] + kb);
+    } else {                       // a row shorter than a chunk: byte by byte
+      auto bytes = [&](const int8_t* q, int x) {
+        uint32_t w[4] = {0u, 0u, 0u, 0u};
+#pragma unroll 1
+        for (int k = 0; k < K; ++k) {
+          const uint32_t b = (uint32_t)(uint8_t)(q[k] ^ (int8_t)x) << (8 * (k & 3));
+          w[0] |= k < 4 ? b : 0u;
+          w[1] |= k >= 4 && k < 8 ? b : 0u;
+          w[2] |= k >= 8 && k < 12 ? b : 0u;
+          w[3] |= k >= 12 ? b : 0u;
+        }
+        return v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]} ^ x;   // undone by put's flip: zeros past K
+      };
+#pragma unroll
+      for (int j = 0; j < C::CA; ++j) ra[j] = bytes(pa[j], xa);
+#pragma unroll
+      for (int j = 0; j < C::CB; ++j) rb[j] = bytes(pb[j], xb);
+    }
+  };
+  // the loaded stage kt into its buffer
+  auto put = [&](int kt) {
+    int8_t* st = ring + (kt / KG & 1) * C::STAGE;
+    if constexpr (ZP) {
+#pragma unroll
+      for (int j = 0; j < C::CA; ++j) ra[j] ^= xa;
+#pragma unroll
+      for (int j = 0; j < C::CB; ++j) rb[j] ^= xb;
+    }
+    if (kt == KT - 1) {            // uniform: only the last stage has a tail to shift
+      // how far below its place load() took the chunk
+      const int kc = kt * AK + c16, sh = CONV || K >= 16 ? kc - min(kc, K - 16) : c16;
+#pragma unroll
+      for (int j = 0; j < C::CA; ++j) ra[j] = shift_down(ra[j], sh);
+#pragma unroll
+      for (int j = 0; j < C::CB; ++j) rb[j] = shift_down(rb[j], sh);
+    }
+#pragma unroll
+    for (int j = 0; j < C::CA; ++j) *reinterpret_cast<v4i*>(st + la[j]) = ra[j];
+#pragma unroll
+    for (int j = 0; j < C::CB; ++j) *reinterpret_cast<v4i*>(st + lb[j]) = rb[j];
+    if constexpr (ZP) {
+#pragma unroll
+      for (int j = 0; j < C::CA; ++j) sa[j] = sum16(ra[j], sa[j]);
+#pragma unroll
+      for (int j = 0; j < C::CB; ++j) sb[j] = sum16(rb[j], sb[j]);
+    }
+  };
+
+  const int wm = (wave >> 1) * C::WM, wn = (wave & 1) * C::WN;
+  v16i acc[C::TM][C::TN];
+#pragma unroll
+  for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+    for (int j = 0; j < C::TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
+
+  if (grp < KT) {
+    load(grp);
+    put(grp);
+    if (grp + KG < KT) load(grp + KG);
+  }
+  __syncthreads();
+  for (int k0 = 0; k0 < KT; k0 += KG) {      // every group runs every iteration: the barriers are the workgroup's
+    const int kt = k0 + grp;
+    const int8_t* st = ring + (kt / KG & 1) * C::STAGE;
+    // the next stage goes into the other buffer, whose last reads ended
+    // before the barrier that closed the previous iteration; then the loads
+    // of the one after it, which have this stage's MFMAs to land (a second
+    // register set, two stages in flight, measured no faster)
+    if (kt + KG < KT) {
+      put(kt + KG);
+      if (kt + 2 * KG < KT) load(kt + 2 * KG);
+    }
+    if (kt < KT) mfma_stage<C>(st, wm, wn, lane, acc);
+    __syncthreads();
+  }
+
+  if constexpr (ZP) {
+    // row sums: the 8 lanes of a row (and the K groups) hold its parts
+#pragma unroll
+    for (int j = 0; j < C::CA; ++j) {
+      int s = sa[j];
+      s += __shfl_xor(s, 1, 64);
+      s += __shfl_xor(s, 2, 64);
+      s += __shfl_xor(s, 4, 64);
+      if ((lane & 7) == 0) atomicAdd(&sum_a[wave * (BM / 4) + 8 * j + rl], s);
+    }
+#pragma unroll
+    for (int j = 0; j < C::CB; ++j) {
+      int s = sb[j];
+      s += __shfl_xor(s, 1, 64);
+      s += __shfl_xor(s, 2, 64);
+      s += __shfl_xor(s, 4, 64);
+      if ((lane & 7) == 0) atomicAdd(&sum_b[wave * (BN / 4) + 8 * j + rl], s);
+    }
+    __syncthreads();
+  }
+
+  any_epilogue<C, KG, ZP>(acc, lds, s_rows, sum_a, sum_b, wave, grp, lane, m0, n0, wm, wn, M, N, o_base, e, z, p, out);
+}
+
+// One thread per output with byte loads: products of a few thousand outputs
+// over a short row are a launch and one load latency either way, and this
+// kernel's few instructions arrive sooner than the tiled kernel's.
+__global__ __launch_bounds__(256) void k_qgemm_tiny(const int8_t* __restrict__ A, const int8_t* __restrict__ B, int M,
+                                                    int N, int K, GemmEpi e, void* __restrict__ out) {
+  const int64_t idx = blockIdx.x * 256LL + threadIdx.x;
+  if (idx >= (int64_t)M * N) return;
+  const int64_t m = idx / N, n = idx % N;
+  uint32_t s = 0;
+  for (int k = 0; k < K; ++k) s += (uint32_t)((int)A[m * K + k] * (int)B[n * K + k]);
+  store_out(out, idx, (int)s, m, n, e);
+}
+
+template <int BM, int BN, int KG>
+hipError_t launch_any_tile(const int8_t* A, const int8_t* B, int M, int N, int K, const GemmEpi& e,
+                           const AffineDot* z, const AnyPlan& p, void* out, hipStream_t st) {
+  const int tm = (M + BM - 1) / BM, tn = (N + BN - 1) / BN;
+  const dim3 grid((unsigned)(tm * tn), (unsigned)p.groups), block(256 * KG);
+  const unsigned lds = AnyCfg<BM, BN, KG>::LDS + (p.conv_cg ? (unsigned)K / 4 : 0u);
+  const AffineDot zz = z ? *z : AffineDot{};
+  if (p.conv_cg) {
+    if (z) hipLaunchKernelGGL((k_qgemm_any<BM, BN, KG, true, true>), grid, block, lds, st, A, B, M, N, K, tm, tn, e, zz, p, out);
+    else hipLaunchKernelGGL((k_qgemm_any<BM, BN, KG, false, true>), grid, block, lds, st, A, B, M, N, K, tm, tn, e, zz, p, out);
+  } else {
+    if (z) hipLaunchKernelGGL((k_qgemm_any<BM, BN, KG, true, false>), grid, block, lds, st, A, B, M, N, K, tm, tn, e, zz, p, out);
+    else hipLaunchKernelGGL((k_qgemm_any<BM, BN, KG, false, false>), grid, block, lds, st, A, B, M, N, K, tm, tn, e, zz, p, out);
+  }
+  return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t launch_gemm_any(const int8_t* A, const int8_t* B, int64_t M, int64_t N, int64_t K,
+                           const GemmEpi& e, const AffineDot* z, const AnyPlan& p, void* out, hipStream_t st) {
+  if (M == 0 || N == 0) return hipSuccess;
+  if (p.conv_cg && (p.conv_cg % 16 != 0 || K % 16 != 0 || K <= 0 || K > ANY_CONV_MAX_K)) return hipErrorInvalidValue;
+  const int64_t cus = cu_count() > 0 ? cu_count() : 256;
+  const int64_t t128 = p.groups * ((M + 127) / 128) * ((N + 127) / 128);
+  const int64_t t64 = p.groups * ((M + 63) / 64) * ((N + 63) / 64);
+  if (t64 > INT32_MAX || p.groups > 65535) return hipErrorInvalidValue;
+  const int m = (int)M, n = (int)N, k = (int)K;
+  // (355 x 10 x 33, the last layer of a small MLP: 2 us less than a tile)
+  if (!z && !p.conv_cg && p.groups == 1 && p.lda == K && p.ldb == K && K < 64 && M * N <= (1 << 16)) {
+    hipLaunchKernelGGL(k_qgemm_tiny, dim3((unsigned)((M * N + 255) / 256)), dim3(256), 0, st, A, B, m, n, k, e, out);
+    return hipGetLastError();
+  }
+  // Up to one 64 x 64 tile per CU: four K groups each (512 x 7 x 7 conv, 200
+  // tiles of 36 stages: 35 us with one group, 26 with two, 22 with four); up
+  // to two per CU: two (392 tiles, 18 stages: 25 / 21 / 25 us).  Above that
+  // the tiles fill the chip, and 128 x 128 halves the bytes per operation
+  // (4096 x 4096 x 1001: 43 us, 64 x 64 60 us) where the product has the
+  // rows for it and stages enough to cover its longer fill (1183 x 3917 x
+  // 319, three stages: 22 against 19 us), in two K groups while a CU gets at
+  // most one (2048 x 2048 x 8192: 76 -> 60 us).
+  const int KT = (k + AK - 1) / AK;
+  const bool big = M > 64 && N > 64 && KT >= 6;
+  if (KT > 2) {
+    if (t64 <= cus) return launch_any_tile<64, 64, 4>(A, B, m, n, k, e, z, p, out, st);
+    if (t64 <= 2 * cus) return launch_any_tile<64, 64, 2>(A, B, m, n, k, e, z, p, out, st);
+  }
+  if (big && t128 > cus) return launch_any_tile<128, 128, 1>(A, B, m, n, k, e, z, p, out, st);
+  if (big && 2 * t128 > cus) return launch_any_tile<128, 128, 2>(A, B, m, n, k, e, z, p, out, st);
+  return launch_any_tile<64, 64, 1>(A, B, m, n, k, e, z, p, out, st);
+}
+
+hipError_t setup_any_attributes() {
+  hipError_t err = hipSuccess;
+  auto set = [&](const void* k, int bytes) {
+    if (err == hipSuccess) err = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  };
+#define Q8_SET_ANY(BM, BN, KG)                                                                          \
+  set(reinterpret_cast<const void*>(k_qgemm_any<BM, BN, KG, false, false>), AnyCfg<BM, BN, KG>::LDS);   \
+  set(reinterpret_cast<const void*>(k_qgemm_any<BM, BN, KG, true, false>), AnyCfg<BM, BN, KG>::LDS);    \
+  set(reinterpret_cast<const void*>(k_qgemm_any<BM, BN, KG, false, true>), AnyCfg<BM, BN, KG>::LDS + ANY_CONV_MAX_K / 4); \
+  set(reinterpret_cast<const void*>(k_qgemm_any<BM, BN, KG, true, true>), AnyCfg<BM, BN, KG>::LDS + ANY_CONV_MAX_K / 4);
+  Q8_SET_ANY(128, 128, 1)
+  Q8_SET_ANY(128, 128, 2)
+  Q8_SET_ANY(64, 64, 1)
+  Q8_SET_ANY(64, 64, 2)
+  Q8_SET_ANY(64, 64, 4)
+#undef Q8_SET_ANY
+  return err;
+}
+
+}  // namespace q8

@@ -123,6 +123,34 @@ extern std::atomic<long long> g_ewise_jit_compiled, g_ewise_jit_launches;
 // Copies why the last failed ewise compile failed into buf (truncated,
 // NUL-terminated; "" if none has) and returns the message's full length.
 size_t ewise_jit_error(char* buf, size_t cap);
+// The GEMM for any K and alignment (q8_gemm_any.hip); with `z` the affine
+// form: operand bytes flipped by xa / xb (0, or 0x80808080 for a ui8
+// operand), the int32 result corrected by cB * rowsum(A) + cA * rowsum(B) +
+// kcc, kcc = K * cA * cB modulo 2^32.
+struct AffineDot {
+  int32_t xa, xb;
+  int32_t cA, cB;
+  uint32_t kcc;
+};
+// Row pitches, and the steps from one group to the next (blockIdx.y) of a
+// grouped conv.  conv_cg != 0: B is a conv frame (e.cb, whose Cg is the
+// frame's row pitch) and conv_cg the channels per group, a multiple of 16.
+constexpr int64_t ANY_CONV_MAX_K = 65536;   // chunk table of 16 KiB
+struct AnyPlan {
+  int64_t lda, ldb;
+  int groups = 1;
+  int64_t a_step = 0, b_step = 0, o_step = 0;   // bytes, bytes, output elements
+  int conv_cg = 0;
+};
+hipError_t launch_gemm_any(const int8_t* A, const int8_t* B, int64_t M, int64_t N, int64_t K,
+                           const GemmEpi& e, const AffineDot* z, const AnyPlan& p, void* out, hipStream_t st);
+inline hipError_t launch_gemm_any(const int8_t* A, const int8_t* B, int64_t M, int64_t N, int64_t K,
+                                  const GemmEpi& e, const AffineDot* z, void* out, hipStream_t st) {
+  AnyPlan p;
+  p.lda = p.ldb = K;
+  return launch_gemm_any(A, B, M, N, K, e, z, p, out, st);
+}
+hipError_t setup_any_attributes();   // its dynamic LDS limits
 bool gemm_dq_fits(int64_t M, int64_t N);
 size_t gemm_dq_ws_bytes(int64_t M);
 hipError_t launch_gemm_dq(const int8_t* A, const int8_t* B, int64_t M, int64_t N, int64_t K,

@@ -440,8 +440,8 @@ def qlinear_requant(A: torch.Tensor, sA: torch.Tensor | None, B: torch.Tensor,
 
 
 def generic_gemm_launches() -> int:
-    """Launches of the generic (non-MFMA) GEMM kernel so far in this process:
-    GEMMs whose K is not a multiple of 16 or whose operands are not 16-byte
+    """Launches of the general GEMM kernel so far in this process: GEMMs
+    whose K is not a multiple of 16 or whose operands are not 16-byte
     aligned take it."""
     n = C.c_int64(0)
     L.call("q8_generic_gemm_launches", C.byref(n))

@@ -1,0 +1,95 @@
+"""The GEMM for any K and alignment and the affine quantized_dot of the same
+kernel (csrc/q8_gemm_any.hip) against the oracle, at the sizes where they can
+go wrong: rows shorter than a 16-byte chunk, the chunk and stage remainders
+of K, tile edges, the three groupings of a tile's K stages, misaligned
+operands, every output form.  Integer and fp32 results bit for bit."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+@pytest.fixture(scope="module")
+def ops():
+    if not torch.cuda.is_available():
+        pytest.skip("no HIP device")
+    from mlfw_amd import ops as O
+    from mlfw_amd import _lib
+    _lib.call("q8_init", 0)
+    return O
+
+
+def dev(a, shift=0):
+    """On the device, `shift` bytes past an aligned address."""
+    flat = torch.zeros(a.size + 64, dtype=torch.uint8, device=DEV)
+    flat[shift:shift + a.size] = torch.from_numpy(np.ascontiguousarray(a).view(np.uint8).reshape(-1)).to(DEV)
+    t = flat[shift:shift + a.size].view(a.shape)
+    return t.view(torch.int8) if a.dtype == np.int8 else t
+
+
+def host(t):
+    torch.cuda.synchronize()
+    return t.cpu().numpy()
+
+
+# K: below a chunk, a chunk and one past, stage edges, several stages with a remainder
+KS = [1, 3, 15, 17, 31, 127, 129, 255, 300, 1001]
+# M, N: one element, tile edges, one tile column; 17 x 17 tiles of 64 take the
+# two-group form, 33 x 17 the 128-wide tile
+MNS = [(1, 1), (16, 65), (17, 64), (63, 129), (130, 68)]
+
+
+@pytest.mark.parametrize("K", KS)
+@pytest.mark.parametrize("M,N", MNS)
+def test_any_k(ops, oracle, M, N, K):
+    rng = np.random.default_rng(M * 7 + N * 3 + K)
+    A = rng.integers(-128, 128, (M, K)).astype(np.int8)
+    B = rng.integers(-128, 128, (N, K)).astype(np.int8)
+    print(f"any M={M} N={N} K={K}", flush=True)
+    acc = oracle.quantized_dot(A, B, 1)
+    np.testing.assert_array_equal(host(ops.quantized_dot(dev(A), dev(B))), acc)
+    sA, sB = rng.uniform(1e-3, 0.05, M), rng.uniform(1e-4, 0.02, N)
+    bias = rng.uniform(-1, 1, N).astype(np.float32)
+    want = oracle.epilogue(acc, "rowcol", sA, sB, bias=bias, act="silu")
+    d = [torch.from_numpy(v).to(DEV) for v in (sA, sB, bias)]
+    got = host(ops.qlinear(dev(A), d[0], dev(B), d[1], bias=d[2], act="silu"))
+    np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("M,N,K", [(1030, 1070, 1001), (2100, 1070, 901), (2100, 2300, 900), (70, 3000, 250)])
+@pytest.mark.parametrize("u8,zpA,zpB", [(False, 0, 0), (True, 121, 0), (True, 3, -5)])
+def test_large_tiles(ops, oracle, M, N, K, u8, zpA, zpB):
+    rng = np.random.default_rng(M + N + K)
+    A = rng.integers(0, 256, (M, K)).astype(np.uint8)
+    A = A if u8 else A.view(np.int8)
+    B = rng.integers(-128, 128, (N, K)).astype(np.int8)
+    np.testing.assert_array_equal(host(ops.quantized_dot(dev(A), dev(B), zpA, zpB)),
+                                  oracle.quantized_dot(A, B, 1, zpA, zpB))
+
+
+@pytest.mark.parametrize("M,N,K", [(5, 70, 64), (100, 70, 256), (1, 33, 10)])
+@pytest.mark.parametrize("shift", [1, 2, 8])
+def test_misaligned_operands(ops, oracle, M, N, K, shift):
+    rng = np.random.default_rng(shift + K)
+    A = rng.integers(0, 256, (M, K)).astype(np.uint8)
+    B = rng.integers(-128, 128, (N, K)).astype(np.int8)
+    for a, zp in ((A.view(np.int8), 0), (A, 0), (A, 77)):
+        got = host(ops.quantized_dot(dev(a, shift), dev(B, 16 - shift), zp, 0))
+        np.testing.assert_array_equal(got, oracle.quantized_dot(a, B, 1, zp, 0))
+
+
+@pytest.mark.parametrize("M,N,K", [(20, 30, 7), (100, 129, 130), (3, 64, 33)])
+def test_int8_output(ops, oracle, M, N, K):
+    rng = np.random.default_rng(K)
+    A = rng.integers(-128, 128, (M, K)).astype(np.int8)
+    B = rng.integers(-128, 128, (N, K)).astype(np.int8)
+    sA, sB = rng.uniform(1e-3, 0.05, M), rng.uniform(1e-4, 0.02, N)
+    y = oracle.epilogue(oracle.quantized_dot(A, B, 1), "rowcol", sA, sB, act="relu")
+    s_next = float(np.abs(y).max() / 127.0) or 1.0
+    got = host(ops.qlinear_requant(dev(A), torch.from_numpy(sA).to(DEV), dev(B), torch.from_numpy(sB).to(DEV),
+                                   s_next, act="relu"))
+    np.testing.assert_array_equal(got, oracle.quantize(y.reshape(-1), s_next).reshape(M, N))
