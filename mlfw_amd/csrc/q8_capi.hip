@@ -953,7 +953,7 @@ static int conv_impl(const char* who, const void* x, int x_dtype, const void* w,
   G.w_u8 = w_dtype == Q8_U8;
   const bool empty = G.N * G.O * G.Pn == 0;
   Q8_REQUIRE(empty || (x && w && out), "%s: NULL pointer", who);
-  const size_t need = q8::conv_direct(G) ? 0 : q8::conv_workspace_bytes(G);
+  const size_t need = q8::conv_direct(G, workspace ? workspace_bytes : 0) ? 0 : q8::conv_workspace_need(G);
   Q8_REQUIRE(empty || workspace_bytes >= need,
              "%s: workspace of %zu bytes is smaller than the %zu bytes required "
              "(q8_quantized_conv_workspace)", who, workspace_bytes, need);
@@ -969,7 +969,7 @@ static int conv_impl(const char* who, const void* x, int x_dtype, const void* w,
     Q8_REQUIRE((reinterpret_cast<uintptr_t>(w_taps) & 15) == 0, "%s: w_taps must be 16-byte aligned", who);
   }
   return launched(q8::launch_conv(static_cast<const int8_t*>(x), static_cast<const int8_t*>(w), w_taps, G,
-                                  e, workspace, out, as_stream(stream)),
+                                  e, workspace, workspace_bytes, out, as_stream(stream)),
                   "quantized_conv launch");
 }
 

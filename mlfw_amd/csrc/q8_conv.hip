@@ -8,31 +8,34 @@
 // coordinate lies in the padding adds 0.
 //
 // Paths, all exact:
-//   * GEMM form for contractions of 64 or more (Kc = Cg * prod(K)): the
-//     [P, Kc] int8 matrix of a group's receptive fields (im2col) is built in
-//     the caller's workspace and the int8 MFMA GEMM computes
-//     out[n, g*Og : (g+1)*Og, :] = W_g [Og, Kc] x col^T -- the weight is the
-//     A operand, so the [Og, P] result is already the NC(spatial) output
-//     block and the dequant epilogue is fused as in q8_gemm.  With more than
-//     16 output channels per group the images go in batches: the matrix of
-//     nb images is [nb * P, Kc] and one GEMM computes [Og, nb * P], its
+//   * GEMM form for contractions of 64 or more (Kc = Cg * prod(K)), and for
+//     large products over shorter ones:
+//     out[n, g*Og : (g+1)*Og, :] = W_g [Og, Kc] x (receptive fields)^T -- the
+//     weight is the A operand, so the [Og, P] result is already the
+//     NC(spatial) output block and the dequant epilogue is fused as in
+//     q8_gemm.  Images go in batches: one GEMM computes [Og, nb * P], its
 //     epilogue storing column n * P + p of the product at image n, position
-//     p (column-blocked output), so a batch is one GEMM large enough to fill
-//     the chip instead of nb small ones.  The matrix is built one of two ways:
-//       - channels per group a multiple of 16: the group's input is first
-//         transposed to a zero-padded channel-last frame, and the
-//         contraction is taken tap-major (k = tap * Cg + c, the weight
-//         permuted to match), so each row of the matrix is a run of
-//         16-byte copies, one per tap; for a 1 x 1 kernel at stride 1 the
-//         frame is the matrix and no copy is made.  Integer addition does
-//         not depend on the order of the taps, so the sums are the same;
-//       - otherwise a byte gather in the OI(spatial) order (ic-major, then
-//         kernel positions), the contraction padded with zeros to a
-//         multiple of 16 (the weight rows copied to that pitch).
-//   * a direct kernel (one thread per output element) for short
-//     contractions -- depthwise and other small-group convolutions, where a
-//     GEMM per group would be launch-bound -- and for zero points and ui8
-//     operands.
+//     p (column-blocked output), and the groups are a second grid dimension,
+//     so a grouped conv is two launches, not two per group.  The receptive
+//     fields come one of two ways:
+//       - channels per group a multiple of 16: the input is transposed to a
+//         padded channel-last frame and the contraction is taken tap-major
+//         (k = tap * Cg + c, the weight permuted to match, in the same launch
+//         as the frame where it was not prepacked): each 16 bytes of a
+//         column are 16 channels of one frame position, which the GEMM reads
+//         where they lie.  Integer addition does not depend on the order of
+//         the taps, so the sums are the same;
+//       - otherwise a matrix (im2col) by a byte gather in the OI(spatial)
+//         order (ic-major, then kernel positions).
+//     Zero points and ui8 operands run the same paths: bytes are flipped on
+//     the way (u - 128), padding holds the input's zero point, and the GEMM
+//     corrects its sums with the operands' row sums (q8_zp.hip states the
+//     identity).  28 x 28 x 128 at batch 32 with ui8 input: 2700 us one
+//     thread per output, 23.6 us here.
+//   * a direct kernel (one thread per output element) for other short
+//     contractions -- depthwise and other small-group convolutions -- for an
+//     input zero point outside its type, and for affine calls that bring
+//     less workspace than the GEMM needs.
 // Spatial ranks 1..3 share the code: unused trailing dimensions have size 1,
 // stride 1, no padding and dilation 1.
 #include "q8_device.h"
@@ -47,14 +50,21 @@ namespace q8 {
 // indices per wave, so each byte load of a wave reads neighbouring input
 // bytes (with stride 1, consecutive bytes of a row); the tile is transposed
 // through LDS so that the stores are 128-byte row segments of the matrix.
+// Affine operands: ui8 bytes are flipped (`flip` = 0x80), and a tap in the
+// padding holds `fill`, the input's zero point as an int8 code, so that its
+// (x - zp) is 0; both 0 in the symmetric scheme.
 constexpr int I2C_TP = 64, I2C_TK = 128, I2C_PITCH = I2C_TK + 16;
 
+template <bool AFFINE>
 __global__ __launch_bounds__(256) void k_im2col(const int8_t* __restrict__ x, ConvGeom G,
-                                                int64_t n0, int64_t g, int8_t* __restrict__ col) {
+                                                int64_t n0, int64_t g, uint32_t flip, uint32_t fill,
+                                                int8_t* __restrict__ col) {
   __shared__ __align__(16) uint32_t tile[I2C_TP * I2C_PITCH / 4];
   // blockIdx.y: image n0 + y of a batch, written at matrix rows y * P ..
+  // blockIdx.z: group g + z, a matrix of its own
   const int64_t n = n0 + blockIdx.y;
-  col += (int64_t)blockIdx.y * G.Pn * G.Kc16;
+  g += blockIdx.z;
+  col += ((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * G.Pn * G.Kc16;
   const int tk = (G.Kc16 + I2C_TK - 1) / I2C_TK;
   const int64_t pt = blockIdx.x / tk;
   const int k0 = (int)(blockIdx.x - pt * tk) * I2C_TK;
@@ -99,7 +109,7 @@ __global__ __launch_bounds__(256) void k_im2col(const int8_t* __restrict__ x, Co
       const uint32_t sp = ((uint32_t)s0 * (uint32_t)G.S[1] + (uint32_t)s1) * (uint32_t)G.S[2] + (uint32_t)s2;
       const int8_t* plane = xg + (int64_t)(kin ? ic : 0) * G.Sn;
       const uint32_t raw = (uint8_t)plane[in ? sp : 0u];   // in bounds either way
-      v[b] = in ? raw : 0u;
+      v[b] = AFFINE ? (in ? raw ^ flip : (kin ? fill : 0u)) : (in ? raw : 0u);
       ++k2;
       const bool c2 = k2 == G.K[2];
       k2 = c2 ? 0 : k2;
@@ -153,72 +163,67 @@ __global__ __launch_bounds__(256) void k_pad_rows(const int8_t* __restrict__ w, 
 // For Cg a multiple of 16 the contraction is taken tap-major, k = t * Cg + c
 // (t: kernel position in row-major order, c: input channel of the group):
 // the same products summed in another order, and int32 wrap-around addition
-// does not depend on the order.  Each group's input goes once to a
-// zero-padded channel-last frame xp[y][e][c], e over E0 x E1 x E2 with
+// does not depend on the order.  The input goes once to a padded
+// channel-last frame xp[y][e][c], e over E0 x E1 x E2 with
 // E_i = (P_i - 1) * st_i + (K_i - 1) * dl_i + 1 (input coordinate e_i - lo_i),
 // so that the receptive field of output p at tap t is the Cg contiguous
-// bytes xp[y][e(p) + off(t)][:] and im2col copies 16-byte chunks.  With a
-// 1 x 1 kernel at stride 1 (E = P, off = 0) xp is the GEMM's B matrix itself.
+// bytes xp[y][e(p) + off(t)][:] and the GEMM reads them as they lie.
 struct ConvFrame {
   int E[3];
   int64_t Ep;   // E0 * E1 * E2
 };
 
-// xp[y][e][c] = x[n0 + y][g * Cg + c][e - lo] (0 outside the image), the nb
-// images of a batch along blockIdx.y, 64-channel tiles along blockIdx.z.  A
-// workgroup transposes 64 frame positions x 64 channels through LDS: in the
-// gather each thread takes one position and 16 channels, the lanes of a
-// wave consecutive positions, so each byte load of a wave reads
-// neighbouring bytes of one channel plane; in the store the lanes take
-// consecutive 16-byte chunks of the frame rows.
+// The frame of nb images and Cb channels from channel c0 on:
+// xp[y][e][c] = x[n0 + y][c0 + c][e - lo], `fill` outside the image, bytes
+// flipped by `flip` (see k_im2col).  A workgroup transposes 64 frame
+// positions x 64 channels through LDS: in the gather each thread takes one
+// position and 16 channels, the lanes of a wave consecutive positions, so
+// each byte load of a wave reads neighbouring bytes of one channel plane; in
+// the store the lanes take consecutive 16-byte chunks of the frame rows.
 constexpr int FR_PITCH = 64 + 16;   // LDS row: 64 channel bytes + pad
-__global__ __launch_bounds__(256) void k_conv_to_frame(const int8_t* __restrict__ x, ConvGeom G,
-                                                       ConvFrame F, int64_t n0, int64_t g,
-                                                       int8_t* __restrict__ xp) {
-  __shared__ __align__(16) uint32_t tile[64 * FR_PITCH / 4];
-  const int64_t y = blockIdx.y;
-  const int64_t eb = blockIdx.x * 64LL;
-  const int64_t e = eb + (threadIdx.x & 63);
+struct FrameJob {
+  int64_t n0;
+  int c0, Cb;
+  uint32_t flip, fill;
+};
+template <bool AFFINE>
+__device__ __forceinline__ void frame_tile(const int8_t* __restrict__ x, const ConvGeom& G, const ConvFrame& F,
+                                           const FrameJob& J, uint32_t* tile, int64_t y, int eb, int ct,
+                                           int8_t* __restrict__ xp) {
+  const int el = (int)(threadIdx.x & 63), e = eb + el, Ep = (int)F.Ep;
   const int cs = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // the wave's 16-channel slice
-  const int el = (int)(threadIdx.x & 63);
   bool in = false;
   uint32_t sp = 0u;
-  if (e < F.Ep) {
-    const int e2 = (int)(e % F.E[2]);
-    const int64_t q = e / F.E[2];
-    const int e1 = (int)(q % F.E[1]);
-    const int e0 = (int)(q / F.E[1]);
+  if (e < Ep) {
+    const int q = e / F.E[2], e2 = e - q * F.E[2];
+    const int e0 = q / F.E[1], e1 = q - e0 * F.E[1];
     const int s0 = e0 - (int)G.lo[0], s1 = e1 - (int)G.lo[1], s2 = e2 - (int)G.lo[2];
     in = (unsigned)s0 < (unsigned)G.S[0] && (unsigned)s1 < (unsigned)G.S[1] &&
          (unsigned)s2 < (unsigned)G.S[2];
     // a position in the padding (or past the frame) reads the plane's
-    // first byte and keeps 0
+    // first byte and keeps the fill
     sp = in ? ((uint32_t)s0 * (uint32_t)G.S[1] + (uint32_t)s1) * (uint32_t)G.S[2] + (uint32_t)s2 : 0u;
   }
-  const int8_t* src = x + ((n0 + y) * G.C + g * G.Cg) * G.Sn + sp;
-  for (int64_t ct = 64LL * blockIdx.z; ct < G.Cg; ct += 64LL * gridDim.z) {   // uniform
-    const int64_t c = ct + 16 * cs;
-    uint32_t w4[4] = {0u, 0u, 0u, 0u};
-    if (c < G.Cg) {
-      const int8_t* sc = src + c * G.Sn;
-      uint32_t v[16];
+  const int c = ct + 16 * cs;
+  uint32_t w4[4] = {0u, 0u, 0u, 0u};
+  if (c < J.Cb) {
+    const int8_t* sc = x + ((J.n0 + y) * G.C + J.c0 + c) * G.Sn + sp;
+    uint32_t v[16];
 #pragma unroll
-      for (int b = 0; b < 16; ++b) v[b] = (uint8_t)sc[(int64_t)b * G.Sn];
+    for (int b = 0; b < 16; ++b) v[b] = (uint8_t)sc[(int64_t)b * G.Sn];
 #pragma unroll
-      for (int b = 0; b < 16; ++b) w4[b >> 2] |= (in ? v[b] : 0u) << (8 * (b & 3));
-    }
-    reinterpret_cast<v4i*>(tile + (el * FR_PITCH + 16 * cs) / 4)[0] =
-        v4i{(int)w4[0], (int)w4[1], (int)w4[2], (int)w4[3]};
-    __syncthreads();
-    // store: chunk ch of row r; 4 chunks per row of this channel tile
-    const int cw = G.Cg - ct < 64 ? (int)((G.Cg - ct) >> 4) : 4;   // chunks in this tile
-    for (int i = threadIdx.x; i < 64 * cw; i += 256) {
-      const int r = i / cw, ch = i - r * cw;
-      if (eb + r < F.Ep)
-        *reinterpret_cast<v4i*>(xp + (y * F.Ep + eb + r) * G.Cg + ct + 16 * ch) =
-            *reinterpret_cast<const v4i*>(tile + (r * FR_PITCH + 16 * ch) / 4);
-    }
-    __syncthreads();
+    for (int b = 0; b < 16; ++b) w4[b >> 2] |= (AFFINE ? (in ? v[b] ^ J.flip : J.fill) : (in ? v[b] : 0u)) << (8 * (b & 3));
+  }
+  reinterpret_cast<v4i*>(tile + (el * FR_PITCH + 16 * cs) / 4)[0] =
+      v4i{(int)w4[0], (int)w4[1], (int)w4[2], (int)w4[3]};
+  __syncthreads();
+  // store: chunk ch of row r; 4 chunks per row of this channel tile
+  const int cw = J.Cb - ct < 64 ? (J.Cb - ct) >> 4 : 4;   // chunks in this tile
+  for (int i = threadIdx.x; i < 64 * cw; i += 256) {
+    const int r = i / cw, ch = i - r * cw;
+    if (eb + r < Ep)
+      *reinterpret_cast<v4i*>(xp + (y * F.Ep + eb + r) * J.Cb + ct + 16 * ch) =
+          *reinterpret_cast<const v4i*>(tile + (r * FR_PITCH + 16 * ch) / 4);
   }
 }
 
@@ -230,13 +235,11 @@ __global__ __launch_bounds__(256) void k_conv_to_frame(const int8_t* __restrict_
 // ns * Kn 16-byte chunks wt[o][t * Cg + c0 .. + 16], tap-major so that
 // neighbouring lanes write neighbouring chunks.  ns * Kn <= WT_CHUNKS.
 constexpr int WT_CHUNKS = 1024;
-__global__ __launch_bounds__(256) void k_conv_weight_taps(const int8_t* __restrict__ w, int64_t nslices,
-                                                          int Cg, int Kn, int ns,
-                                                          int8_t* __restrict__ wt) {
-  __shared__ __align__(16) uint8_t buf[16 * WT_CHUNKS];
+__device__ __forceinline__ void weight_taps(const int8_t* __restrict__ w, int64_t nslices, int Cg, int Kn,
+                                            int ns, int64_t blk, uint8_t* buf, int8_t* __restrict__ wt) {
   const int64_t Kc = (int64_t)Cg * Kn;
   const int slices = Cg >> 4;
-  const int64_t s0 = (int64_t)blockIdx.x * ns;
+  const int64_t s0 = blk * ns;
   const int n = (int)(nslices - s0 < ns ? nslices - s0 : ns);      // slices of this workgroup
   const v4i* src = reinterpret_cast<const v4i*>(w + s0 * 16 * Kn);   // 16-byte aligned
   for (int i = threadIdx.x; i < n * Kn; i += 256) reinterpret_cast<v4i*>(buf)[i] = src[i];
@@ -254,55 +257,37 @@ __global__ __launch_bounds__(256) void k_conv_weight_taps(const int8_t* __restri
   }
 }
 
-// col[y * Pn + p][t * Cg + c] = xp[y][e(p) + off(t)][c] with the frame
-// position of output p, e(p) = row-major index of (o_i * st_i), and the
-// offset of tap t, off(t) = row-major index of (k_i * dl_i), both over E.
-// A thread copies one 16-byte channel chunk of output p for a group of four
-// consecutive taps at a time (four loads in flight); the groups are spread
-// over blockIdx.z.  Tap coordinates are uniform.
-__global__ __launch_bounds__(256) void k_im2col_taps(const int8_t* __restrict__ xp, ConvGeom G,
-                                                     ConvFrame F, int8_t* __restrict__ col) {
-  const int64_t y = blockIdx.y;
-  const int cpr = G.Cg >> 4;
-  const int64_t idx = blockIdx.x * 256LL + threadIdx.x;
-  if (idx >= G.Pn * cpr) return;
-  const int64_t p = idx / cpr;
-  const int c = (int)(idx - p * cpr) * 16;
-  const int o2 = (int)(p % G.P[2]);
-  const int64_t q = p / G.P[2];
-  const int o1 = (int)(q % G.P[1]);
-  const int o0 = (int)(q / G.P[1]);
-  const int64_t ep = ((int64_t)o0 * G.st[0] * F.E[1] + (int64_t)o1 * G.st[1]) * F.E[2] +
-                     (int64_t)o2 * G.st[2];
-  const int64_t Cg = G.Cg;
-  const int8_t* src = xp + (y * F.Ep + ep) * Cg + c;
-  int8_t* dst = col + (y * G.Pn + p) * G.Kc + c;
-  for (int t0 = 4 * blockIdx.z; t0 < G.Kn; t0 += 4 * gridDim.z) {
-    int k2 = t0 % G.K[2];
-    const int r = t0 / G.K[2];
-    int k1 = r % G.K[1];
-    int k0 = r / G.K[1];
-    int64_t o4[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      // a tap past Kn repeats tap t0: the same bytes, stored again at t0
-      o4[j] = t0 + j < G.Kn ? (((int64_t)k0 * G.dl[0] * F.E[1] + (int64_t)k1 * G.dl[1]) * F.E[2] +
-                               (int64_t)k2 * G.dl[2])
-                            : o4[0];
-      const bool c2 = ++k2 == G.K[2];
-      k2 = c2 ? 0 : k2;
-      k1 += c2;
-      const bool c1 = k1 == G.K[1];
-      k1 = c1 ? 0 : k1;
-      k0 += c1;
-    }
-    v4i a[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) a[j] = *reinterpret_cast<const v4i*>(src + o4[j] * Cg);
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      *reinterpret_cast<v4i*>(dst + (int64_t)(t0 + j < G.Kn ? t0 + j : t0) * Cg) = a[j];
+__global__ __launch_bounds__(256) void k_conv_weight_taps(const int8_t* __restrict__ w, int64_t nslices,
+                                                          int Cg, int Kn, int ns,
+                                                          int8_t* __restrict__ wt) {
+  __shared__ __align__(16) uint8_t buf[16 * WT_CHUNKS];
+  weight_taps(w, nslices, Cg, Kn, ns, blockIdx.x, buf, wt);
+}
+
+// The frame of a batch and, for a weight that was not prepacked, its
+// tap-major form in one launch: the first nb * etiles * ctiles workgroups
+// transpose the frame, the rest the weight.  The two do not depend on each
+// other and each alone is a launch's fixed cost.
+template <bool AFFINE>
+__global__ __launch_bounds__(256) void k_conv_prep(const int8_t* __restrict__ x, ConvGeom G, ConvFrame F,
+                                                   FrameJob J, int64_t nb, int etiles, int8_t* __restrict__ xp,
+                                                   const int8_t* __restrict__ w, int64_t nslices, int ns,
+                                                   int8_t* __restrict__ wt) {
+  __shared__ __align__(16) uint8_t buf[16 * WT_CHUNKS];
+  const int64_t nfr = nb * etiles * ((J.Cb + 63) / 64), id = blockIdx.x;
+  if (id >= nfr) {   // uniform
+    weight_taps(w, nslices, G.Cg, G.Kn, ns, id - nfr, buf, wt);
+    return;
   }
+  const unsigned q = (unsigned)id / (unsigned)etiles, ct = q / (unsigned)nb;
+  frame_tile<AFFINE>(x, G, F, J, reinterpret_cast<uint32_t*>(buf), q - ct * (unsigned)nb,
+                     64 * (int)((unsigned)id - q * (unsigned)etiles), 64 * (int)ct, xp);
+}
+template <bool AFFINE>
+__global__ __launch_bounds__(256) void k_conv_to_frame(const int8_t* __restrict__ x, ConvGeom G, ConvFrame F,
+                                                       FrameJob J, int8_t* __restrict__ xp) {
+  __shared__ __align__(16) uint32_t tile[64 * FR_PITCH / 4];
+  frame_tile<AFFINE>(x, G, F, J, tile, blockIdx.y, 64 * (int)blockIdx.x, 64 * (int)blockIdx.z, xp);
 }
 
 // Direct form: one thread per output element, taps in the reference's
@@ -353,15 +338,35 @@ __global__ __launch_bounds__(256) void k_conv_direct(const int8_t* __restrict__ 
 
 // k_im2col computes input coordinates and offsets within one channel plane
 // in 32 bits: every coordinate lies in [-lo, (P - 1) * st + (K - 1) * dl].
-bool conv_uses_gemm(const ConvGeom& G) {
-  if (G.Kc < 64 || G.Sn >= ((int64_t)1 << 31)) return false;
+static bool conv_gemm_fits(const ConvGeom& G) {
+  if (G.Sn >= ((int64_t)1 << 31)) return false;
   for (int i = 0; i < 3; ++i)
     if ((int64_t)(G.P[i] - 1) * G.st[i] + (int64_t)(G.K[i] - 1) * G.dl[i] >= ((int64_t)1 << 31)) return false;
   return true;
 }
+bool conv_uses_gemm(const ConvGeom& G) { return G.Kc >= 64 && conv_gemm_fits(G); }
 
-bool conv_direct(const ConvGeom& G) {
-  return !conv_uses_gemm(G) || G.zpx != 0 || G.zpw != 0 || G.x_u8 || G.w_u8;
+// Short contractions (Cg * prod(K) < 64) that the GEMM still serves better
+// than one thread per output: from 2^24 multiply-adds on (the direct kernel
+// does about 1.2e12 a second: 32 x 3 x 112 x 112 -> 32, 3 x 3, takes 299 us
+// direct and 44 us as im2col + GEMM; 8 x 3 x 56 x 56 -> 32 26 and 13 us)
+// with at least 8 output channels per group in a 64-row tile.
+static bool conv_short_gemm(const ConvGeom& G) {
+  return G.Kc < 64 && G.Og >= 8 && conv_gemm_fits(G) &&
+         (double)G.N * (double)G.O * (double)G.Pn * (double)G.Kc >= 0x1p24;
+}
+
+// The input zero point as an int8 code, zpx - 128 for ui8 operands: what a
+// tap in the padding holds.  Zero points outside the type's range have none.
+static int64_t conv_fill(const ConvGeom& G) { return (int64_t)G.zpx - (G.x_u8 ? 128 : 0); }
+
+static bool conv_affine(const ConvGeom& G) { return G.zpx != 0 || G.zpw != 0 || G.x_u8 || G.w_u8; }
+
+bool conv_direct(const ConvGeom& G, size_t workspace_bytes) {
+  if (conv_uses_gemm(G) && !conv_affine(G)) return false;
+  if (conv_fill(G) < -128 || conv_fill(G) > 127) return true;
+  if (conv_uses_gemm(G)) return workspace_bytes < conv_workspace_need(G);
+  return !conv_short_gemm(G) || workspace_bytes < conv_workspace_bytes(G);
 }
 
 constexpr size_t CONV_BATCH_BYTES = (size_t)128 << 20;   // workspace per batch of images
@@ -399,134 +404,251 @@ static bool conv_pointwise(const ConvGeom& G) {
   return G.Kn == 1 && G.st[0] == 1 && G.st[1] == 1 && G.st[2] == 1;
 }
 
-// Implicit GEMM (launch_gemm_conv: the GEMM reads the frame itself, no
-// im2col matrix): channels per group a multiple of 64, a contraction of at
-// most 16384, more than 16 output channels per group (the GEMM, not the
-// GEMV); a pointwise conv needs no im2col in any case.
-static bool conv_implicit(const ConvGeom& G) {
-  return !conv_pointwise(G) && G.Cg % 64 == 0 && G.Kc <= 16384 && G.Og > 16;
+// The frame path: the GEMM reads the frame itself.
+static bool conv_frame_path(const ConvGeom& G, ConvFrame* F) {
+  return conv_frame_of(G, F) && G.Kc <= ANY_CONV_MAX_K;
+}
+static size_t conv_wt_bytes(const ConvGeom& G) {   // 1 x 1: the weight as given
+  return G.Kn == 1 ? 0 : round256((size_t)G.O * (size_t)G.Kc);
 }
 
-// channel-last workspace: [col: nb * Pn * Kc, unless pointwise or implicit] [frame:
-// nb * Ep * Cg] [tap-major weight: O * Kc, unless 1 x 1] [split-K partial
-// sums of the implicit GEMM], each rounded up to 256 bytes
-struct ClLayout {
-  int64_t nb;
-  size_t col, frame, wt, part;   // part: split-K partial sums of the implicit GEMM
-};
-static ClLayout cl_layout(const ConvGeom& G, const ConvFrame& F) {
-  const bool no_col = conv_pointwise(G) || conv_implicit(G);
-  const size_t col1 = no_col ? 0 : (size_t)G.Pn * (size_t)G.Kc;
-  const size_t fr1 = (size_t)F.Ep * (size_t)G.Cg;
-  ClLayout L;
-  L.nb = conv_batch_of(G, col1 + fr1);
-  L.col = round256((size_t)L.nb * col1);
-  L.frame = round256((size_t)L.nb * fr1);
-  L.wt = G.Kn == 1 ? 0 : round256((size_t)G.O * (size_t)G.Kc);   // 1 x 1: the weight as given
-  L.part = 0;
-  if (conv_implicit(G)) {
-    const ConvGemmPlan pl = conv_gemm_plan(G.Og, L.nb * G.Pn, G.Kc, (size_t)1 << 30);
-    if (pl.splits > 1) L.part = round256((size_t)pl.splits * (size_t)G.Og * (size_t)(L.nb * G.Pn) * 4);
+// What split partial sums of the GEMM took (conv_workspace_need counts them).
+static size_t conv_split_bytes(int64_t M, int64_t N, int64_t K) {
+  const int64_t cus = cu_count() > 0 ? cu_count() : 256;
+  const int64_t tiles64 = ((M + 63) / 64) * ((N + 63) / 64);
+  const int64_t bm = M >= 128 && tiles64 >= 2 * cus ? 128 : 64;
+  const int64_t tiles = ((M + bm - 1) / bm) * ((N + bm - 1) / bm), KT = (K + 127) / 128;
+  int64_t splits = 1;
+  if (tiles < cus && K >= 4096) {
+    splits = (2 * cus + tiles - 1) / tiles;
+    splits = splits < 8 ? splits : 8;
+    splits = splits < KT / 8 ? splits : KT / 8;
+    splits = splits > 1 ? splits : 1;
   }
-  return L;
+  while (splits > 1 && splits * M * N * 4 > ((int64_t)1 << 30)) --splits;
+  const int64_t kps = (KT + splits - 1) / splits;
+  splits = (KT + kps - 1) / kps;
+  return splits > 1 ? round256((size_t)(splits * M * N * 4)) : 0;
 }
 
-size_t conv_workspace_bytes(const ConvGeom& G) {
+// The least workspace a symmetric int8 conv is accepted with.  (What each
+// path below needs for one image and one group is no more; it runs as many
+// at once as fit the workspace it is given.)
+size_t conv_workspace_need(const ConvGeom& G) {
   if (!conv_uses_gemm(G)) return 0;
   // the im2col form: batched matrices, then padded weight rows
   size_t b = round256((size_t)conv_batch_of(G, (size_t)G.Pn * (size_t)G.Kc16) * (size_t)G.Pn *
                       (size_t)G.Kc16);
   if (G.Kc16 != G.Kc) b += (size_t)G.O * (size_t)G.Kc16;
   ConvFrame F;
-  if (conv_frame_of(G, &F)) {   // also enough for the im2col form it falls back to
-    const ClLayout L = cl_layout(G, F);
-    const size_t cl = L.col + L.frame + L.wt + L.part;
+  if (conv_frame_of(G, &F)) {
+    // frames of a batch; receptive fields too where the GEMM once needed them
+    const bool impl = !conv_pointwise(G) && G.Cg % 64 == 0 && G.Kc <= 16384 && G.Og > 16;
+    const size_t col1 = conv_pointwise(G) || impl ? 0 : (size_t)G.Pn * (size_t)G.Kc;
+    const size_t fr1 = (size_t)F.Ep * (size_t)G.Cg;
+    const int64_t nb = conv_batch_of(G, col1 + fr1);
+    size_t cl = round256((size_t)nb * col1) + round256((size_t)nb * fr1) + conv_wt_bytes(G);
+    if (impl) {
+      cl += conv_split_bytes(G.Og, nb * G.Pn, G.Kc);
+    }
     b = cl > b ? cl : b;
   }
   return b;
 }
 
+// What q8_quantized_conv_workspace asks for: every group of as many images
+// as fit CONV_BATCH_BYTES.
+size_t conv_workspace_bytes(const ConvGeom& G) {
+  const size_t need = conv_workspace_need(G);
+  if (need == 0 && !conv_short_gemm(G)) return 0;
+  ConvFrame F;
+  const bool fr = conv_frame_path(G, &F);
+  const size_t per = (size_t)G.groups * (fr ? (size_t)F.Ep * (size_t)G.Cg : (size_t)G.Pn * (size_t)G.Kc16);
+  size_t nb = per ? CONV_BATCH_BYTES / per : 1;
+  nb = nb < 1 ? 1 : nb > (size_t)G.N ? (size_t)G.N : nb;
+  const size_t want = round256(nb * per) + (fr ? conv_wt_bytes(G) : (size_t)G.O * (size_t)G.Kc16);
+  return want > need ? want : need;
+}
+
+// Images and groups of one pass: `unit` bytes each, within `avail` and the
+// launch limits.
+struct ConvBatch {
+  int64_t nb;
+  int gc;
+};
+static ConvBatch conv_batch(const ConvGeom& G, size_t unit, size_t avail) {
+  int64_t units = unit ? (int64_t)(avail / unit) : 1;
+  ConvBatch b;
+  const int64_t fit = unit ? (((int64_t)1 << 31) - 1) / (int64_t)unit : units;   // one image's offsets in 31 bits
+  int64_t gc = units < G.groups ? units : G.groups;
+  gc = gc < fit ? gc : fit;
+  gc = gc < 65535 ? gc : 65535;
+  b.gc = (int)(gc < 1 ? 1 : gc);
+  b.nb = b.gc == G.groups ? units / b.gc : 1;
+  b.nb = b.nb > G.N ? G.N : b.nb;
+  b.nb = b.nb > 65535 ? 65535 : b.nb;                                     // grid.y of k_im2col
+  const int64_t cap = ((int64_t)1 << 31) / (G.Pn > 0 ? G.Pn : 1) - 1;     // GEMM N = nb * P in an int
+  b.nb = b.nb > cap ? cap : b.nb;
+  b.nb = b.nb > fit / b.gc ? fit / b.gc : b.nb;
+  b.nb = b.nb < 1 ? 1 : b.nb;
+  return b;
+}
+
+// The affine correction of the conv's GEMM (A: weights, B: input).
+static AffineDot conv_zp(const ConvGeom& G) {
+  AffineDot z{};
+  z.xa = G.w_u8 ? (int)0x80808080u : 0;
+  z.cA = (G.w_u8 ? 128 : 0) - G.zpw;
+  z.cB = (int32_t)-conv_fill(G);
+  z.kcc = (uint32_t)G.Kc * (uint32_t)z.cA * (uint32_t)z.cB;
+  return z;
+}
+
 static hipError_t launch_conv_channel_last(const int8_t* x, const int8_t* w, const int8_t* w_taps,
                                            const ConvGeom& G, const ConvFrame& F, const GemmEpi& e,
-                                           void* workspace, void* out, hipStream_t st) {
-  const ClLayout L = cl_layout(G, F);
-  const bool pw = conv_pointwise(G);
-  int8_t* col = static_cast<int8_t*>(workspace);
-  int8_t* xp = col + L.col;
+                                           void* workspace, size_t ws_bytes, void* out, hipStream_t st) {
+  const size_t wt_bytes = w_taps ? 0 : conv_wt_bytes(G);
+  int8_t* wt_ws = static_cast<int8_t*>(workspace);
+  int8_t* xp = wt_ws + wt_bytes;
+  const ConvBatch cb = conv_batch(G, (size_t)F.Ep * (size_t)G.Cg, ws_bytes - wt_bytes);
   // a 1 x 1 kernel's weight is its own tap-major form; a prepacked one
   // (q8_conv_weight_taps) is used as given
-  int8_t* wt = G.Kn == 1 ? const_cast<int8_t*>(w) : w_taps ? const_cast<int8_t*>(w_taps) : xp + L.frame;
-  int32_t* part = reinterpret_cast<int32_t*>(xp + L.frame + L.wt);
+  const int8_t* wt = G.Kn == 1 ? w : w_taps ? w_taps : wt_ws;
+  const bool affine = conv_affine(G);
+  const AffineDot z = conv_zp(G);
+  const AffineDot* zp = z.xa || z.cA || z.cB ? &z : nullptr;
   const int64_t nsl = G.O * (G.Cg >> 4);                   // weight slices
   const int wns = G.Kn >= 256 ? WT_CHUNKS / G.Kn : 256 / G.Kn;   // slices per workgroup
-  const int64_t wblk = (nsl + wns - 1) / wns;
-  const int64_t xch = G.Pn * (G.Cg >> 4);
-  const int64_t ctiles = (G.Cg + 63) / 64, tgroups = (G.Kn + 3) / 4;
-  if (wblk >= ((int64_t)1 << 24) || (F.Ep + 63) / 64 >= ((int64_t)1 << 24) ||
-      (xch + 255) / 256 >= ((int64_t)1 << 24))
-    return hipErrorInvalidValue;
-  const unsigned fz = (unsigned)(ctiles < 65535 ? ctiles : 65535);   // strided loops cover the rest
-  const unsigned tz = (unsigned)(tgroups < 65535 ? tgroups : 65535);
-  hipError_t err = hipSuccess;
-  if (G.Kn > 1 && !w_taps) {
-    hipLaunchKernelGGL(k_conv_weight_taps, dim3((unsigned)wblk), dim3(256), 0, st, w, nsl, G.Cg, G.Kn,
-                       wns, wt);
-    err = hipGetLastError();
-    if (err != hipSuccess) return err;
+  bool weight_todo = G.Kn > 1 && !w_taps;
+  const int etiles = (int)((F.Ep + 63) / 64);
+  const size_t osz = e.out_i32 ? sizeof(int32_t) : sizeof(float);
+  for (int64_t n0 = 0; n0 < G.N; n0 += cb.nb) {
+    const int64_t nb = G.N - n0 < cb.nb ? G.N - n0 : cb.nb;
+    for (int64_t g = 0; g < G.groups; g += cb.gc) {
+      const int gc = (int)(G.groups - g < cb.gc ? G.groups - g : cb.gc);
+      const int Cb = gc * G.Cg;
+      const FrameJob J{n0, (int)(g * G.Cg), Cb, G.x_u8 ? 0x80u : 0u, (uint32_t)conv_fill(G) & 0xffu};
+      const int64_t nfr = nb * etiles * ((Cb + 63) / 64), nw = weight_todo ? (nsl + wns - 1) / wns : 0;
+      if (nfr + nw >= ((int64_t)1 << 24) || (Cb + 63) / 64 > 65535) return hipErrorInvalidValue;
+      if (weight_todo) {
+        const dim3 grid((unsigned)(nfr + nw));
+        if (affine) hipLaunchKernelGGL(k_conv_prep<true>, grid, dim3(256), 0, st, x, G, F, J, nb, etiles, xp, w, nsl, wns, wt_ws);
+        else hipLaunchKernelGGL(k_conv_prep<false>, grid, dim3(256), 0, st, x, G, F, J, nb, etiles, xp, w, nsl, wns, wt_ws);
+      } else {
+        const dim3 grid((unsigned)etiles, (unsigned)nb, (unsigned)((Cb + 63) / 64));
+        if (affine) hipLaunchKernelGGL(k_conv_to_frame<true>, grid, dim3(256), 0, st, x, G, F, J, xp);
+        else hipLaunchKernelGGL(k_conv_to_frame<false>, grid, dim3(256), 0, st, x, G, F, J, xp);
+      }
+      hipError_t err = hipGetLastError();
+      if (err != hipSuccess) return err;
+      weight_todo = false;
+      GemmEpi eb = e;
+      eb.col_blk = G.Pn;
+      eb.blk_stride = G.O * G.Pn;
+      eb.ld_out = G.Pn;
+      GemmEpi::ConvB& c = eb.cb;
+      c.Pn = (uint32_t)G.Pn;
+      c.P1 = (uint32_t)G.P[1];
+      c.P2 = (uint32_t)G.P[2];
+      c.st0 = (uint32_t)G.st[0];
+      c.st1 = (uint32_t)G.st[1];
+      c.st2 = (uint32_t)G.st[2];
+      c.E1 = (uint32_t)F.E[1];
+      c.E2 = (uint32_t)F.E[2];
+      c.Ep = (uint32_t)F.Ep;
+      c.Cg = (uint32_t)Cb;
+      c.K1 = (uint32_t)G.K[1];
+      c.K2 = (uint32_t)G.K[2];
+      c.Kn = (uint32_t)G.Kn;
+      c.dl0 = (uint32_t)G.dl[0];
+      c.dl1 = (uint32_t)G.dl[1];
+      c.dl2 = (uint32_t)G.dl[2];
+      c.frame_bytes = (uint32_t)(nb * F.Ep * Cb);
+      const int8_t* A = wt + g * G.Og * G.Kc;
+      void* o = static_cast<char*>(out) + (size_t)((n0 * G.O + g * G.Og) * G.Pn) * osz;
+      // With more than one 64 x 64 tile per CU the direct-to-LDS GEMM's
+      // cheaper copies win (56 x 56 x 64: 24.3 against 25.7 us; 1 x 1 14 x
+      // 14 x 1024 -> 256: 16.6 against 18.9); with fewer, K groups do (7 x 7 x
+      // 512: 25.1, split over K in two launches, against 21.6 us).
+      const int64_t t64 = ((G.Og + 63) / 64) * ((nb * G.Pn + 63) / 64);
+      const bool many = !affine && G.groups == 1 && t64 > (cu_count() > 0 ? cu_count() : 256);
+      if (many && !conv_pointwise(G) && G.Cg % 64 == 0 && G.Kc <= 16384) {
+        err = launch_gemm_conv(A, xp, G.Og, nb * G.Pn, G.Kc, eb, o, st);
+      } else if (many && conv_pointwise(G) && (reinterpret_cast<uintptr_t>(A) & 15) == 0) {
+        err = launch_gemm(A, xp, G.Og, nb * G.Pn, G.Kc, eb, o, st);
+      } else {
+        AnyPlan p;
+        p.lda = G.Kc;
+        p.ldb = 0;
+        p.groups = gc;
+        p.a_step = (int64_t)G.Og * G.Kc;
+        p.b_step = G.Cg;
+        p.o_step = (int64_t)G.Og * G.Pn;
+        p.conv_cg = G.Cg;
+        err = launch_gemm_any(A, xp, G.Og, nb * G.Pn, G.Kc, eb, zp, p, o, st);
+      }
+      if (err != hipSuccess) return err;
+    }
   }
+  return hipSuccess;
+}
+
+// Receptive fields as a matrix (k_im2col), every group of a batch of images
+// at once; the GEMM takes the weight rows at their own pitch.
+static hipError_t launch_conv_im2col(const int8_t* x, const int8_t* w, const ConvGeom& G, const GemmEpi& e,
+                                     void* workspace, size_t ws_bytes, void* out, hipStream_t st) {
+  int8_t* col = static_cast<int8_t*>(workspace);
+  // symmetric int8 with more than two tiles per CU: weight rows padded to the
+  // matrix's pitch for the direct-to-LDS GEMM (32 x 3 x 112 x 112, 7 x 7 at
+  // stride 2: 48.4 us against 53.5 with the weight at its own pitch)
+  const int64_t t64 = ((G.Og + 63) / 64) * ((G.N * G.Pn + 63) / 64);
+  const bool many = !conv_affine(G) && G.groups == 1 && t64 > 2 * (cu_count() > 0 ? cu_count() : 256) &&
+                    (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 && (int64_t)G.Kc16 * 256 < ((int64_t)1 << 31);
+  const size_t wp_bytes = many && G.Kc16 != G.Kc ? (size_t)G.O * (size_t)G.Kc16 : 0;
+  const ConvBatch cb = conv_batch(G, (size_t)G.Pn * (size_t)G.Kc16, ws_bytes - wp_bytes);
+  const int8_t* wmat = w;
+  if (wp_bytes) {
+    int8_t* wp = col + (size_t)cb.nb * (size_t)G.Pn * (size_t)G.Kc16;   // Kc16 % 16 == 0: stays aligned
+    const int64_t n = G.O * G.Kc16;
+    hipLaunchKernelGGL(k_pad_rows, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, w, G.O, (int64_t)G.Kc,
+                       (int64_t)G.Kc16, wp);
+    hipError_t err = hipGetLastError();
+    if (err != hipSuccess) return err;
+    wmat = wp;
+  }
+  const AffineDot z = conv_zp(G);
+  const AffineDot* zp = z.xa || z.cA || z.cB ? &z : nullptr;
   const size_t osz = e.out_i32 ? sizeof(int32_t) : sizeof(float);
   GemmEpi eb = e;
   eb.col_blk = G.Pn;
   eb.blk_stride = G.O * G.Pn;
   eb.ld_out = G.Pn;
-  const bool impl = conv_implicit(G);
-  if (impl) {
-    GemmEpi::ConvB& c = eb.cb;
-    c.Pn = (uint32_t)G.Pn;
-    c.P1 = (uint32_t)G.P[1];
-    c.P2 = (uint32_t)G.P[2];
-    c.st0 = (uint32_t)G.st[0];
-    c.st1 = (uint32_t)G.st[1];
-    c.st2 = (uint32_t)G.st[2];
-    c.E1 = (uint32_t)F.E[1];
-    c.E2 = (uint32_t)F.E[2];
-    c.Ep = (uint32_t)F.Ep;
-    c.Cg = (uint32_t)G.Cg;
-    c.K1 = (uint32_t)G.K[1];
-    c.K2 = (uint32_t)G.K[2];
-    c.Kn = (uint32_t)G.Kn;
-    c.dl0 = (uint32_t)G.dl[0];
-    c.dl1 = (uint32_t)G.dl[1];
-    c.dl2 = (uint32_t)G.dl[2];
-  }
-  for (int64_t n0 = 0; n0 < G.N; n0 += L.nb) {
-    const int64_t nb = G.N - n0 < L.nb ? G.N - n0 : L.nb;
-    for (int64_t g = 0; g < G.groups; ++g) {
-      hipLaunchKernelGGL(k_conv_to_frame, dim3((unsigned)((F.Ep + 63) / 64), (unsigned)nb, fz),
-                         dim3(256), 0, st, x, G, F, n0, g, xp);
-      err = hipGetLastError();
+  for (int64_t n0 = 0; n0 < G.N; n0 += cb.nb) {
+    const int64_t nb = G.N - n0 < cb.nb ? G.N - n0 : cb.nb;
+    for (int64_t g = 0; g < G.groups; g += cb.gc) {
+      const int gc = (int)(G.groups - g < cb.gc ? G.groups - g : cb.gc);
+      dim3 grid;
+      if (!im2col_grid(G, nb, &grid)) return hipErrorInvalidValue;
+      grid.z = (unsigned)gc;
+      const uint32_t flip = G.x_u8 ? 0x80u : 0u, fill = (uint32_t)conv_fill(G) & 0xffu;
+      if (conv_affine(G)) hipLaunchKernelGGL(k_im2col<true>, grid, dim3(256), 0, st, x, G, n0, g, flip, fill, col);
+      else hipLaunchKernelGGL(k_im2col<false>, grid, dim3(256), 0, st, x, G, n0, g, flip, fill, col);
+      hipError_t err = hipGetLastError();
       if (err != hipSuccess) return err;
-      const int8_t* A = wt + g * G.Og * G.Kc;
       void* o = static_cast<char*>(out) + (size_t)((n0 * G.O + g * G.Og) * G.Pn) * osz;
-      if (impl) {
-        GemmEpi ei = eb;
-        ei.cb.frame_bytes = (uint32_t)(nb * F.Ep * G.Cg);
-        const ConvGemmPlan pl = conv_gemm_plan(G.Og, nb * G.Pn, G.Kc, L.part);
-        err = launch_gemm_conv(A, xp, G.Og, nb * G.Pn, G.Kc, ei, pl, part, o, st);
+      if (many && (reinterpret_cast<uintptr_t>(wmat) & 15) == 0) {
+        err = launch_gemm(wmat, col, G.Og, nb * G.Pn, G.Kc16, eb, o, st);
         if (err != hipSuccess) return err;
         continue;
       }
-      const int8_t* B = xp;
-      if (!pw) {
-        hipLaunchKernelGGL(k_im2col_taps, dim3((unsigned)((xch + 255) / 256), (unsigned)nb, tz),
-                           dim3(256), 0, st, xp, G, F, col);
-        err = hipGetLastError();
-        if (err != hipSuccess) return err;
-        B = col;
-      }
-      if (nb > 1) err = launch_gemm(A, B, G.Og, nb * G.Pn, G.Kc, eb, o, st);
-      else if (G.Og <= 16) err = launch_gemv(A, B, G.Og, G.Pn, G.Kc, e, o, st);
-      else err = launch_gemm(A, B, G.Og, G.Pn, G.Kc, e, o, st);
+      AnyPlan p;
+      p.lda = G.Kc;
+      p.ldb = G.Kc16;
+      p.groups = gc;
+      p.a_step = (int64_t)G.Og * G.Kc;
+      p.b_step = nb * G.Pn * G.Kc16;
+      p.o_step = (int64_t)G.Og * G.Pn;
+      err = launch_gemm_any(w + g * G.Og * G.Kc, col, G.Og, nb * G.Pn, G.Kc, eb, zp, p, o, st);
       if (err != hipSuccess) return err;
     }
   }
@@ -546,69 +668,19 @@ hipError_t launch_conv_weight_taps(const int8_t* w, const ConvGeom& G, int8_t* w
 }
 
 hipError_t launch_conv(const int8_t* x, const int8_t* w, const int8_t* w_taps, const ConvGeom& G,
-                       const GemmEpi& e, void* workspace, void* out, hipStream_t st) {
+                       const GemmEpi& e, void* workspace, size_t ws_bytes, void* out, hipStream_t st) {
   if (G.N * G.O * G.Pn == 0) return hipSuccess;
-  if (conv_direct(G)) {
+  if (conv_direct(G, workspace ? ws_bytes : 0)) {
     const int64_t total = G.N * G.O * G.Pn;
     hipLaunchKernelGGL(k_conv_direct, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, x,
                        w, G, e, out);
     return hipGetLastError();
   }
   ConvFrame F;
-  if (conv_frame_of(G, &F) && ((reinterpret_cast<uintptr_t>(workspace) | reinterpret_cast<uintptr_t>(w)) & 15) == 0)
-    return launch_conv_channel_last(x, w, w_taps, G, F, e, workspace, out, st);
-  int8_t* col = static_cast<int8_t*>(workspace);
-  const int64_t NB = conv_batch_of(G, (size_t)G.Pn * (size_t)G.Kc16);
-  const size_t col_bytes = ((size_t)NB * (size_t)G.Pn * (size_t)G.Kc16 + 255) & ~(size_t)255;
-  const int8_t* wmat = w;
-  if (G.Kc16 != G.Kc) {
-    int8_t* wp = col + col_bytes;
-    const int64_t n = G.O * G.Kc16;
-    hipLaunchKernelGGL(k_pad_rows, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, w, G.O,
-                       (int64_t)G.Kc, (int64_t)G.Kc16, wp);
-    hipError_t err = hipGetLastError();
-    if (err != hipSuccess) return err;
-    wmat = wp;
-  }
-  const size_t osz = e.out_i32 ? sizeof(int32_t) : sizeof(float);
-  // batched form: the GEMM's MFMA path needs 16-byte-aligned operands (the
-  // weight rows and the workspace); otherwise one image at a time
-  const bool aligned = ((reinterpret_cast<uintptr_t>(wmat) | reinterpret_cast<uintptr_t>(col)) & 15) == 0;
-  if (NB > 1 && aligned && (int64_t)G.Kc16 * 256 < ((int64_t)1 << 31)) {
-    GemmEpi eb = e;
-    eb.col_blk = G.Pn;
-    eb.blk_stride = G.O * G.Pn;
-    eb.ld_out = G.Pn;
-    for (int64_t n0 = 0; n0 < G.N; n0 += NB) {
-      const int64_t nb = G.N - n0 < NB ? G.N - n0 : NB;
-      for (int64_t g = 0; g < G.groups; ++g) {
-        dim3 grid;
-        if (!im2col_grid(G, nb, &grid)) return hipErrorInvalidValue;
-        hipLaunchKernelGGL(k_im2col, grid, dim3(256), 0, st, x, G, n0, g, col);
-        hipError_t err = hipGetLastError();
-        if (err != hipSuccess) return err;
-        const int8_t* A = wmat + g * G.Og * G.Kc16;
-        void* o = static_cast<char*>(out) + (size_t)((n0 * G.O + g * G.Og) * G.Pn) * osz;
-        err = launch_gemm(A, col, G.Og, nb * G.Pn, G.Kc16, eb, o, st);
-        if (err != hipSuccess) return err;
-      }
-    }
-    return hipSuccess;
-  }
-  for (int64_t n = 0; n < G.N; ++n)
-    for (int64_t g = 0; g < G.groups; ++g) {
-      dim3 grid;
-      if (!im2col_grid(G, 1, &grid)) return hipErrorInvalidValue;
-      hipLaunchKernelGGL(k_im2col, grid, dim3(256), 0, st, x, G, n, g, col);
-      hipError_t err = hipGetLastError();
-      if (err != hipSuccess) return err;
-      const int8_t* A = wmat + g * G.Og * G.Kc16;
-      void* o = static_cast<char*>(out) + (size_t)((n * G.O + g * G.Og) * G.Pn) * osz;
-      err = G.Og <= 16 ? launch_gemv(A, col, G.Og, G.Pn, G.Kc16, e, o, st)
-                       : launch_gemm(A, col, G.Og, G.Pn, G.Kc16, e, o, st);
-      if (err != hipSuccess) return err;
-    }
-  return hipSuccess;
+  const bool aligned = ((reinterpret_cast<uintptr_t>(workspace) | (G.Kn > 1 && !w_taps ? reinterpret_cast<uintptr_t>(w) : 0)) & 15) == 0;
+  if (conv_frame_path(G, &F) && aligned)
+    return launch_conv_channel_last(x, w, w_taps, G, F, e, workspace, ws_bytes, out, st);
+  return launch_conv_im2col(x, w, G, e, workspace, ws_bytes, out, st);
 }
 
 }  // namespace q8

@@ -75,6 +75,15 @@ __device__ __forceinline__ int sum16(v4i v, int s) {
   return __builtin_amdgcn_sdot4(v.w, 0x01010101, s, false);
 }
 
+// The offset of every 16-byte chunk of a conv's contraction from its column's
+// frame position.
+__device__ __forceinline__ void fill_taps(int* taps, const GemmEpi& e, const AnyPlan& p, int K, int tid, int threads) {
+  for (int i = tid; i < (K >> 4); i += threads) {
+    const uint32_t t = 16u * (uint32_t)i / (uint32_t)p.conv_cg;
+    taps[i] = (int)(convb_tap(e.cb, t) * e.cb.Cg + (16u * (uint32_t)i - t * (uint32_t)p.conv_cg));
+  }
+}
+
 // One 128-byte stage: the wave's (32 TM) x (32 TN) sub-tile at (wm, wn).
 template <class C>
 __device__ __forceinline__ void mfma_stage(const int8_t* st, int wm, int wn, int lane, v16i (&acc)[C::TM][C::TN]) {
@@ -262,10 +271,7 @@ void k_qgemm_any(const int8_t* __restrict__ A, const int8_t* __restrict__ B, int
   B += blockIdx.y * p.b_step;
   const int64_t o_base = blockIdx.y * p.o_step;
   if constexpr (CONV) {
-    for (int i = tid; i < (K >> 4); i += 256 * KG) {
-      const uint32_t t = 16u * (uint32_t)i / (uint32_t)p.conv_cg;
-      taps[i] = (int)(convb_tap(e.cb, t) * e.cb.Cg + (16u * (uint32_t)i - t * (uint32_t)p.conv_cg));
-    }
+    fill_taps(taps, e, p, K, tid, 256 * KG);
     __syncthreads();
   }
 
@@ -408,6 +414,164 @@ void k_qgemm_any(const int8_t* __restrict__ A, const int8_t* __restrict__ B, int
   any_epilogue<C, KG, ZP>(acc, lds, s_rows, sum_a, sum_b, wave, grp, lane, m0, n0, wm, wn, M, N, o_base, e, z, p, out);
 }
 
+// The same product with the K range split over the 8 waves of a workgroup,
+// for up to one 32 x 32 tile per CU: each wave computes the whole tile over
+// its own 128-byte slices of K, its operands loaded straight into the MFMA
+// layout (16x16x64: lane l holds 16 bytes of row l % 16, chunk l / 16), two
+// 64-byte steps in flight.  No LDS staging and no barrier until the partial
+// tiles meet in LDS: with so few tiles the time is one workgroup's load
+// latencies, and a staged stage costs a barrier on top of its own.  (17 x 4096
+// x 4096: 16.5 us in four K groups of 64 x 64 tiles, 11.1 here; 512 x 49 x
+// 4608, a 7 x 7 x 512 conv of one image: 15.6 and 8.1 us.  Larger tiles of
+// this form lose: 64 x 11008 x 4096 takes 25 us with 64 x 64, 21 staged.)
+constexpr int WKT = 2, WKW = 8, WKB = 16 * WKT;       // 16-row blocks, waves, tile edge
+constexpr int WK_PITCH = WKB + 4;
+constexpr int WK_LDS = WKT * WKW * 16 * WK_PITCH * 4 + 8 * WKB + 8 * WKB;
+template <bool ZP, bool CONV>
+__global__ __launch_bounds__(64 * WKW, 2)
+void k_qgemm_wk(const int8_t* __restrict__ A, const int8_t* __restrict__ B, int M, int N, int K,
+                int tiles_m, int tiles_n, GemmEpi e, AffineDot z, AnyPlan p, void* __restrict__ out) {
+  extern __shared__ __attribute__((aligned(1024))) int8_t lds[];
+  int* red = reinterpret_cast<int*>(lds);                 // [strip][wave][16][WK_PITCH]
+  double* s_rows = reinterpret_cast<double*>(red + WKT * WKW * 16 * WK_PITCH);
+  int* sum_a = reinterpret_cast<int*>(s_rows + WKB);
+  int* sum_b = sum_a + WKB;
+  int* taps = sum_b + WKB;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r16 = lane & 15, g = lane >> 4;
+  int tm, tn;
+  tile_of((int)blockIdx.x, tiles_m, tiles_n, tm, tn);
+  const int m0 = tm * WKB, n0 = tn * WKB;
+  if (tid < WKB)
+    s_rows[tid] = e.mode == 1 && !e.out_i32 && m0 + tid < M ? e.sA[(int64_t)(m0 + tid) * e.sA_stride] : 0.0;
+  if (ZP && tid < 2 * WKB) sum_a[tid] = 0;
+  A += blockIdx.y * p.a_step;
+  B += blockIdx.y * p.b_step;
+  const int64_t o_base = blockIdx.y * p.o_step;
+  if constexpr (CONV) fill_taps(taps, e, p, K, tid, 64 * WKW);
+  if (CONV || ZP) __syncthreads();
+  const int xa = ZP ? z.xa : 0, xb = ZP ? z.xb : 0;
+  // rows past the edge repeat the last one: their results are never stored
+  const int8_t* pa[WKT];
+  const int8_t* pb[WKT];
+#pragma unroll
+  for (int i = 0; i < WKT; ++i) {
+    pa[i] = A + (int64_t)min(m0 + 16 * i + r16, M - 1) * p.lda;
+    const int n = min(n0 + 16 * i + r16, N - 1);
+    pb[i] = B + (CONV ? (int64_t)convb_row(e.cb, (uint32_t)n) : n * p.ldb);
+  }
+  int sa[WKT], sb[WKT];
+  v4i acc[WKT][WKT];
+#pragma unroll
+  for (int i = 0; i < WKT; ++i) {
+    sa[i] = sb[i] = 0;
+#pragma unroll
+    for (int j = 0; j < WKT; ++j) acc[i][j] = v4i{0, 0, 0, 0};
+  }
+  struct Frag {
+    v4i a[WKT], b[WKT];
+  };
+  // 64-byte step s of the contraction: steps 2 c and 2 c + 1 are slice c,
+  // wave w takes slices w, w + 8, ...  K >= 16.
+  const int KS = (K + 63) / 64;
+  auto load = [&](int s, Frag& f) {
+    const int kk = min(64 * s + 16 * g, K - 16);
+    const int kb = CONV ? taps[kk >> 4] : kk;
+#pragma unroll
+    for (int i = 0; i < WKT; ++i) {
+      f.a[i] = load16_any(pa[i] + kk);
+      f.b[i] = load16_any(pb[i] + kb);
+    }
+  };
+  auto mul = [&](int s, Frag& f) {
+    if constexpr (ZP) {
+#pragma unroll
+      for (int i = 0; i < WKT; ++i) {
+        f.a[i] ^= xa;
+        f.b[i] ^= xb;
+      }
+    }
+    if (s == KS - 1) {                                   // uniform: the tail moves down, zeros come in
+      const int kc = 64 * s + 16 * g, sh = kc - min(kc, K - 16);
+#pragma unroll
+      for (int i = 0; i < WKT; ++i) {
+        f.a[i] = shift_down(f.a[i], sh);
+        f.b[i] = shift_down(f.b[i], sh);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < WKT; ++i)
+#pragma unroll
+      for (int j = 0; j < WKT; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(f.a[i], f.b[j], acc[i][j], 0, 0, 0);
+    if constexpr (ZP) {
+#pragma unroll
+      for (int i = 0; i < WKT; ++i) {
+        sa[i] = sum16(f.a[i], sa[i]);
+        sb[i] = sum16(f.b[i], sb[i]);
+      }
+    }
+  };
+  Frag f0, f1;
+  int s = 2 * wave;
+  if (s < KS) load(s, f0);
+  while (s < KS) {
+    const bool two = s + 1 < KS;
+    if (two) load(s + 1, f1);
+    mul(s, f0);
+    const int nx = s + 2 * WKW;
+    if (nx < KS) load(nx, f0);
+    if (two) mul(s + 1, f1);
+    s = nx;
+  }
+  if constexpr (ZP) {
+    // lanes of one row differ in g
+#pragma unroll
+    for (int i = 0; i < WKT; ++i) {
+      int va = sa[i], vb = sb[i];
+      va += __shfl_xor(va, 16, 64);
+      va += __shfl_xor(va, 32, 64);
+      vb += __shfl_xor(vb, 16, 64);
+      vb += __shfl_xor(vb, 32, 64);
+      if (g == 0) {
+        atomicAdd(&sum_a[16 * i + r16], va);
+        atomicAdd(&sum_b[16 * i + r16], vb);
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < WKT; ++i)
+#pragma unroll
+    for (int j = 0; j < WKT; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) red[((i * WKW + wave) * 16 + 4 * g + r) * WK_PITCH + 16 * j + r16] = acc[i][j][r];
+  __syncthreads();
+  // two outputs per thread, consecutive columns over the lanes
+#pragma unroll
+  for (int t = tid; t < WKB * WKB; t += 64 * WKW) {
+    const int row = t / WKB, col = t % WKB, m = m0 + row, n = n0 + col;
+    uint32_t a = 0u;
+#pragma unroll
+    for (int w = 0; w < WKW; ++w) a += (uint32_t)red[((row / 16 * WKW + w) * 16 + row % 16) * WK_PITCH + col];
+    if (m >= M || n >= N) continue;
+    if constexpr (ZP) a += z.kcc + (uint32_t)z.cA * (uint32_t)sum_b[col] + (uint32_t)z.cB * (uint32_t)sum_a[row];
+    int64_t at = o_base + (int64_t)m * N + n;
+    if (e.col_blk > 0) {
+      const unsigned blk = (unsigned)n / (unsigned)e.col_blk;
+      at = o_base + blk * e.blk_stride + (int64_t)m * e.ld_out + (unsigned)n - blk * (unsigned)e.col_blk;
+    }
+    if (e.out_i32) {
+      static_cast<int32_t*>(out)[at] = (int32_t)a;
+    } else {
+      float y = e.mode == 0 ? (float)((double)(int32_t)a * e.s_out)
+                            : mul_acc_f32scale((int32_t)a, (float)(s_rows[row] * e.sB[(int64_t)n * e.sB_stride]));
+      y = epi_finish(y, n, e);
+      if (e.out_q8) static_cast<int8_t*>(out)[at] = (int8_t)requant(y, e);
+      else static_cast<float*>(out)[at] = y;
+    }
+  }
+}
+
 // One thread per output with byte loads: products of a few thousand outputs
 // over a short row are a launch and one load latency either way, and this
 // kernel's few instructions arrive sooner than the tiled kernel's.
@@ -421,6 +585,17 @@ __global__ __launch_bounds__(256) void k_qgemm_tiny(const int8_t* __restrict__ A
   store_out(out, idx, (int)s, m, n, e);
 }
 
+#define Q8_ANY_LAUNCH(KERN, ...)                                                                                   \
+  do {                                                                                                             \
+    if (p.conv_cg) {                                                                                               \
+      if (z) hipLaunchKernelGGL((KERN<__VA_ARGS__ true, true>), grid, block, lds, st, A, B, M, N, K, tm, tn, e, zz, p, out); \
+      else hipLaunchKernelGGL((KERN<__VA_ARGS__ false, true>), grid, block, lds, st, A, B, M, N, K, tm, tn, e, zz, p, out);  \
+    } else {                                                                                                       \
+      if (z) hipLaunchKernelGGL((KERN<__VA_ARGS__ true, false>), grid, block, lds, st, A, B, M, N, K, tm, tn, e, zz, p, out); \
+      else hipLaunchKernelGGL((KERN<__VA_ARGS__ false, false>), grid, block, lds, st, A, B, M, N, K, tm, tn, e, zz, p, out);  \
+    }                                                                                                              \
+  } while (0)
+
 template <int BM, int BN, int KG>
 hipError_t launch_any_tile(const int8_t* A, const int8_t* B, int M, int N, int K, const GemmEpi& e,
                            const AffineDot* z, const AnyPlan& p, void* out, hipStream_t st) {
@@ -428,15 +603,20 @@ hipError_t launch_any_tile(const int8_t* A, const int8_t* B, int M, int N, int K
   const dim3 grid((unsigned)(tm * tn), (unsigned)p.groups), block(256 * KG);
   const unsigned lds = AnyCfg<BM, BN, KG>::LDS + (p.conv_cg ? (unsigned)K / 4 : 0u);
   const AffineDot zz = z ? *z : AffineDot{};
-  if (p.conv_cg) {
-    if (z) hipLaunchKernelGGL((k_qgemm_any<BM, BN, KG, true, true>), grid, block, lds, st, A, B, M, N, K, tm, tn, e, zz, p, out);
-    else hipLaunchKernelGGL((k_qgemm_any<BM, BN, KG, false, true>), grid, block, lds, st, A, B, M, N, K, tm, tn, e, zz, p, out);
-  } else {
-    if (z) hipLaunchKernelGGL((k_qgemm_any<BM, BN, KG, true, false>), grid, block, lds, st, A, B, M, N, K, tm, tn, e, zz, p, out);
-    else hipLaunchKernelGGL((k_qgemm_any<BM, BN, KG, false, false>), grid, block, lds, st, A, B, M, N, K, tm, tn, e, zz, p, out);
-  }
+  Q8_ANY_LAUNCH(k_qgemm_any, BM, BN, KG, );
   return hipGetLastError();
 }
+
+hipError_t launch_wk(const int8_t* A, const int8_t* B, int M, int N, int K, const GemmEpi& e,
+                     const AffineDot* z, const AnyPlan& p, void* out, hipStream_t st) {
+  const int tm = (M + WKB - 1) / WKB, tn = (N + WKB - 1) / WKB;
+  const dim3 grid((unsigned)(tm * tn), (unsigned)p.groups), block(64 * WKW);
+  const unsigned lds = WK_LDS + (p.conv_cg ? (unsigned)K / 4 : 0u);
+  const AffineDot zz = z ? *z : AffineDot{};
+  Q8_ANY_LAUNCH(k_qgemm_wk, );
+  return hipGetLastError();
+}
+#undef Q8_ANY_LAUNCH
 
 }  // namespace
 
@@ -464,6 +644,8 @@ hipError_t launch_gemm_any(const int8_t* A, const int8_t* B, int64_t M, int64_t 
   // most one (2048 x 2048 x 8192: 76 -> 60 us).
   const int KT = (k + AK - 1) / AK;
   const bool big = M > 64 && N > 64 && KT >= 6;
+  const int64_t t32 = p.groups * ((M + 31) / 32) * ((N + 31) / 32);
+  if (t32 <= cus && K >= 16) return launch_wk(A, B, m, n, k, e, z, p, out, st);
   if (KT > 2) {
     if (t64 <= cus) return launch_any_tile<64, 64, 4>(A, B, m, n, k, e, z, p, out, st);
     if (t64 <= 2 * cus) return launch_any_tile<64, 64, 2>(A, B, m, n, k, e, z, p, out, st);
@@ -489,6 +671,10 @@ hipError_t setup_any_attributes() {
   Q8_SET_ANY(64, 64, 2)
   Q8_SET_ANY(64, 64, 4)
 #undef Q8_SET_ANY
+  set(reinterpret_cast<const void*>(k_qgemm_wk<false, false>), WK_LDS);
+  set(reinterpret_cast<const void*>(k_qgemm_wk<true, false>), WK_LDS);
+  set(reinterpret_cast<const void*>(k_qgemm_wk<false, true>), WK_LDS + ANY_CONV_MAX_K / 4);
+  set(reinterpret_cast<const void*>(k_qgemm_wk<true, true>), WK_LDS + ANY_CONV_MAX_K / 4);
   return err;
 }
 

@@ -63,26 +63,14 @@ struct GemmEpi {
     uint32_t K1, K2, Kn;       // kernel sizes of dims 1, 2; kernel positions
     uint32_t dl0, dl1, dl2;    // dilations
     uint32_t frame_bytes;      // bytes of the batch's frames
-    uint32_t kps;              // K stages per split (split-K), >= all stages for one split
   } cb;
 };
 
 // GEMM of quantized_conv's implicit form: A [M, K] (tap-major weight rows),
 // B the frames described by e.cb (N = images x Pn columns), column-blocked
-// output as set in e.  K a multiple of 64, at most 16384.  The plan picks
-// the tile and a split of K when the tiles alone would leave most of the
-// chip idle; the splits' int32 partial sums go to `part` (splits * M * N
-// words) and a finishing pass adds them (int32 addition does not depend on
-// the order) and applies the output mapping and dequant.
-struct ConvGemmPlan {
-  int bm;       // square tile edge, 128 or 64
-  int splits;   // K splits, >= 1
-  int kps;      // K stages (of 128) per split
-};
-ConvGemmPlan conv_gemm_plan(int64_t M, int64_t N, int64_t K, size_t part_cap_bytes);
+// output as set in e.  K a multiple of 64, at most 16384.
 hipError_t launch_gemm_conv(const int8_t* A, const int8_t* frame, int64_t M, int64_t N, int64_t K,
-                            const GemmEpi& e, const ConvGemmPlan& plan, int32_t* part, void* out,
-                            hipStream_t st);
+                            const GemmEpi& e, void* out, hipStream_t st);
 
 hipError_t launch_fill_normal(float* out, int64_t n, uint32_t seed, uint64_t offset,
                               double mean, double std, hipStream_t st);
@@ -207,15 +195,17 @@ struct ConvGeom {
   int zpx = 0, zpw = 0;          // input / kernel zero points
   int x_u8 = 0, w_u8 = 0;        // operands read as ui8 (else i8)
 };
-// Zero points and ui8 operands run the direct kernel (exact, one thread per
-// output); plain i8 convs with Cg * prod(K) >= 64 run im2col + GEMM.
-bool conv_direct(const ConvGeom& G);
+// Whether the conv runs the direct kernel (exact, one thread per output):
+// Cg * prod(K) < 64, or zero points / ui8 operands with less workspace than
+// the GEMM paths need or an input zero point outside its type.
+bool conv_direct(const ConvGeom& G, size_t workspace_bytes);
 bool conv_uses_gemm(const ConvGeom& G);
-size_t conv_workspace_bytes(const ConvGeom& G);
+size_t conv_workspace_need(const ConvGeom& G);    // the least a call is accepted with
+size_t conv_workspace_bytes(const ConvGeom& G);   // what a caller is told to bring
 // w_taps (may be null): the weight already in the channel-last path's
 // tap-major form (launch_conv_weight_taps), which then is not permuted per call.
 hipError_t launch_conv(const int8_t* x, const int8_t* w, const int8_t* w_taps, const ConvGeom& G,
-                       const GemmEpi& e, void* workspace, void* out, hipStream_t st);
+                       const GemmEpi& e, void* workspace, size_t ws_bytes, void* out, hipStream_t st);
 // Whether the tap-major weight form is used for weights of G's shape (Cg a
 // multiple of 16, 2 <= prod(K) <= 1024), and the permutation that makes it:
 // w_taps[o][t * Cg + c] = w[o][c][t], O * Cg * prod(K) bytes.

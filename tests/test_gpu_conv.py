@@ -185,3 +185,59 @@ def test_conv_workspace_is_reused(ops, oracle):
     b = ops.quantized_conv(dev(x[:, :, :5, :5].copy()), dev(w), [1, 1], [[0, 0], [0, 0]], workspace=ws)
     same_bits(host(a), oracle.quantized_conv(x, w, [1, 1], [[0, 0], [0, 0]]))
     same_bits(host(b), oracle.quantized_conv(x[:, :, :5, :5].copy(), w, [1, 1], [[0, 0], [0, 0]]))
+
+
+AFFINE = [
+    # x shape, w shape, strides, padding, dilation, groups
+    ((2, 64, 12, 11), (32, 64, 3, 3), [1, 1], [[1, 1], [1, 1]], [1, 1], 1),   # frame path
+    ((3, 96, 9, 9), (80, 32, 3, 3), [2, 1], [[1, 2], [0, 1]], [1, 2], 3),     # groups of one launch, 80 / 3 rows
+    ((5, 48, 7, 7), (9, 16, 5, 5), [1, 1], [[2, 2], [2, 2]], [1, 1], 3),      # 3 output channels per group
+    ((4, 32, 8, 8), (40, 32, 1, 1), [1, 1], [[0, 0], [0, 0]], [1, 1], 1),     # 1 x 1
+    ((2, 10, 11, 13), (48, 10, 3, 3), [1, 2], [[0, 2], [1, 0]], [1, 1], 1),   # im2col, Kc 90
+    ((2, 20, 11, 13), (6, 10, 3, 3), [1, 1], [[1, 1], [1, 1]], [1, 1], 2),    # im2col, groups
+    ((1, 16, 6, 5, 7), (24, 16, 2, 3, 2), [1, 2, 1], [[1, 0], [0, 1], [1, 1]], [1, 1, 2], 1),  # 3-D
+    ((8, 3, 56, 56), (32, 3, 3, 3), [1, 1], [[1, 1], [1, 1]], [1, 1], 1),     # Kc 27, large: im2col
+    ((2, 512, 7, 7), (80, 512, 3, 3), [1, 1], [[1, 1], [1, 1]], [1, 1], 1),   # 36 stages, few tiles
+    ((64, 64, 14, 14), (192, 64, 3, 3), [1, 1], [[1, 1], [1, 1]], [1, 1], 1),  # more tiles than 2 per CU
+]
+
+
+@pytest.mark.parametrize("case", AFFINE)
+@pytest.mark.parametrize("x_u8,w_u8,zpx,zpw", [(True, False, 117, 0), (False, False, -128, 0), (True, True, 3, 130),
+                                               (False, False, 0, 0), (True, False, 300, 0)])
+def test_quantized_conv_affine_paths(ops, oracle, case, x_u8, w_u8, zpx, zpw):
+    """The GEMM paths with zero points and ui8 operands (and, symmetric, the
+    same shapes), bit for bit; zpx = 300 has no ui8 code and runs direct."""
+    xs, ws, st, pd, dl, g = case
+    if np.prod(xs) * np.prod(ws) > 1 << 33 and zpx not in (117, 0):
+        pytest.skip("large shape: one affine and one symmetric run")
+    if ws[0] % g:
+        ws = (ws[0] // g * g, *ws[1:])
+    rng = np.random.default_rng(sum(xs) + zpx + 256 + 2 * x_u8)
+    x = rng.integers(0, 256, xs).astype(np.uint8)
+    w = rng.integers(0, 256, ws).astype(np.uint8)
+    x = x if x_u8 else x.view(np.int8)
+    w = w if w_u8 else w.view(np.int8)
+    print(f"conv affine {xs} {ws} g{g} u8=({x_u8},{w_u8}) zp=({zpx},{zpw})", flush=True)
+    want = oracle.quantized_conv(x, w, st, pd, dl, g, zpx, zpw)
+    same_bits(host(ops.quantized_conv(dev(x), dev(w), st, pd, dl, g, zpx=zpx, zpw=zpw)), want)
+    s_out = 1.7e-4
+    got = host(ops.quantized_conv(dev(x), dev(w), st, pd, dl, g, zpx=zpx, zpw=zpw, s_out=s_out))
+    same_bits(got, (want.astype(np.float64) * s_out).astype(np.float32))
+
+
+def test_conv_affine_without_workspace(ops, oracle):
+    """An affine conv still runs with no workspace (the direct kernel), as a
+    caller that never brought one expects, with the same bits."""
+    import ctypes as C
+    from mlfw_amd import _lib as L
+    rng = np.random.default_rng(5)
+    x = rng.integers(0, 256, (2, 64, 9, 9)).astype(np.uint8)
+    w = rng.integers(-128, 128, (24, 64, 3, 3)).astype(np.int8)
+    out = torch.empty((2, 24, 9, 9), dtype=torch.int32, device=DEV)
+    arr = lambda v: (C.c_int64 * len(v))(*v)  # noqa: E731
+    dx, dw = dev(x), dev(w)
+    L.call("q8_quantized_conv_ex", C.c_void_p(dx.data_ptr()), L.Q8_U8, C.c_void_p(dw.data_ptr()), L.Q8_I8, 2,
+           arr(x.shape), arr(w.shape), arr([1, 1]), arr([1, 1]), arr([1, 1]), arr([1, 1]), 1, 99, 0, L.Q8_I32, 0.0,
+           None, 0, C.c_void_p(out.data_ptr()), None)
+    same_bits(host(out), oracle.quantized_conv(x, w, [1, 1], [[1, 1], [1, 1]], [1, 1], 1, 99, 0))
