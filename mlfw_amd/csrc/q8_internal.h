@@ -181,6 +181,12 @@ hipError_t launch_gemv_w4(const int8_t* xq, const double* sx, int sx_stride, con
                           const double* sw, int64_t M, int64_t N, int64_t K, int64_t group,
                           const float* bias, int act, float* y, hipStream_t st);
 
+// The same for prompts: a tiled GEMM (q8_w4_gemm.hip), where it applies.
+bool gemm_w4_ok(const int8_t* xq, const uint8_t* wq4, int64_t M, int64_t N, int64_t K, int64_t group);
+hipError_t launch_gemm_w4(const int8_t* xq, const double* sx, int sx_stride, const uint8_t* wq4, const double* sw,
+                          int64_t M, int64_t N, int64_t K, int64_t group, const float* bias, int act, float* y,
+                          hipStream_t st);
+
 // Geometry of a quantized_conv (NC(spatial) input, OI(spatial) kernel);
 // unused trailing spatial dimensions have size 1.  Validated by the C ABI:
 // every int field and Cg * prod(K) below 2^31.

@@ -747,6 +747,8 @@ hipError_t launch_gemv_w4(const int8_t* xq, const double* sx, int sx_stride, con
                           const double* sw, int64_t M, int64_t N, int64_t K, int64_t group,
                           const float* bias, int act, float* y, hipStream_t st) {
   if (M == 0 || N == 0) return hipSuccess;
+  if (gemm_w4_ok(xq, wq4, M, N, K, group))
+    return launch_gemm_w4(xq, sx, sx_stride, wq4, sw, M, N, K, group, bias, act, y, st);
   W4Plan pl;
   const bool dot4 = w4_plan(M, K, group, &pl);
   W4MPlan mp;

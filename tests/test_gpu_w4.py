@@ -148,3 +148,25 @@ def test_gemv_w4_per_tensor_scale(ops, oracle, M, N, K, g):
     want = oracle.gemv_w4(xq, np.full(M, s), wq4, sw, K, g, act="silu")
     got = ops.qlinear_w4(dev(xq), dev(np.array([s])), dev(wq4), dev(sw), K, g, act="silu")
     same_bits(host(got), want)
+
+
+# The tiled GEMM (more than 16 tokens where it is the faster): its three tile
+# shapes with ragged token and row counts, groups that end inside a stage or
+# span several, a K that ends inside one, and more than one window of scales.
+@pytest.mark.parametrize("M,N,K,g", [(40, 2100, 256, 128), (33, 1999, 320, 64), (64, 2051, 352, 32),    # 32 x 32
+                                     (97, 4093, 512, 128), (96, 4096, 768, 384),                        # 32 x 64
+                                     (500, 4090, 256, 128), (511, 4096, 192, 64),                       # 64 x 64
+                                     (130, 700, 128 * 19, 128), (130, 600, 32 * 37, 32), (70, 900, 1536, 768)])
+def test_gemm_w4(ops, oracle, M, N, K, g):
+    rng = np.random.default_rng(M + N + K + g)
+    W = (rng.standard_normal((N, K)) * 0.02).astype(np.float32)
+    W[0] = 0.0                                                # scale 1e-10, all codes zero
+    xq = rng.integers(-128, 128, (M, K)).astype(np.int8)
+    sx = rng.uniform(1e-3, 0.05, M)
+    bias = rng.uniform(-1, 1, N).astype(np.float32)
+    wq, sw = ops.pack_weight_int4(dev(W), g)
+    print(f"gemm w4 M={M} N={N} K={K} g={g}", flush=True)
+    for b, act in ((None, "none"), (bias, "silu")):
+        got = host(ops.qlinear_w4(dev(xq), dev(sx), wq, sw, K, g, bias=None if b is None else dev(b), act=act))
+        want = oracle.gemv_w4(xq, sx, host(wq), host(sw), K, g, bias=b, act=act)
+        assert got.tobytes() == want.tobytes(), np.count_nonzero(got != want)
