@@ -71,6 +71,7 @@ int init_device(int dev) {
   e = q8::setup_kernel_attributes();
   if (e == hipSuccess) e = q8::setup_w4_attributes();
   if (e == hipSuccess) e = q8::setup_any_attributes();
+  if (e == hipSuccess) e = q8::setup_ring_attributes();
   (void)q8::cu_count();
   void* sp = nullptr;
   if (e == hipSuccess) e = hipGetSymbolAddress(&sp, HIP_SYMBOL(scratch));

@@ -1186,6 +1186,8 @@ hipError_t launch_gemm(const int8_t* A, const int8_t* B, int64_t M, int64_t N, i
     g_generic_gemm_launches.fetch_add(1, std::memory_order_relaxed);
     return launch_gemm_any(A, B, M, N, K, e, nullptr, out, st);
   }
+  const int ring = gemm_ring_tile(M, N, K);
+  if (ring >= 0) return launch_gemm_ring(A, B, M, N, K, e, ring, out, st);
   switch (gemm_tile_choice(M, N, epi_192_ok(e) ? 0x1Fu : 0xFu)) {
     case 0: return launch_qgemm_tile<256, 256>(A, B, (int)M, (int)N, (int)K, e, out, st);
     case 1: return launch_qgemm_tile<256, 128>(A, B, (int)M, (int)N, (int)K, e, out, st);

@@ -138,6 +138,13 @@ inline hipError_t launch_gemm_any(const int8_t* A, const int8_t* B, int64_t M, i
   p.lda = p.ldb = K;
   return launch_gemm_any(A, B, M, N, K, e, z, p, out, st);
 }
+// The aligned GEMM where every tile has a CU of its own (q8_gemm_ring.hip):
+// the tile to use, or -1; K a multiple of 16, 16-byte aligned operands,
+// 256 * K < 2^31.
+int gemm_ring_tile(int64_t M, int64_t N, int64_t K);
+hipError_t launch_gemm_ring(const int8_t* A, const int8_t* B, int64_t M, int64_t N, int64_t K,
+                            const GemmEpi& e, int tile, void* out, hipStream_t st);
+hipError_t setup_ring_attributes();  // dynamic LDS limits
 hipError_t setup_any_attributes();   // its dynamic LDS limits
 bool gemm_dq_fits(int64_t M, int64_t N);
 size_t gemm_dq_ws_bytes(int64_t M);
