@@ -450,8 +450,48 @@ __global__ __launch_bounds__(NT) void k_quant_tensor(const float* __restrict__ x
   }
 }
 
+// Small tensors in one launch: every workgroup takes the absmax of the whole
+// tensor (cached after the first), then quantizes its 4096 elements.  Bound
+// by one CU's read of the tensor, about 60 GB/s a CU beyond the launch; the
+// three dependent launches below take 7.2 us whatever the size.  (1000
+// elements 5.1 -> 2.3 us, 32768 7.2 -> 4.0, 65536 7.2 -> 5.1; 131072 7.3 both
+// ways, 262144 7.6 against 11.7 here.)
+constexpr int SMALL_TPB = 1024;
+constexpr int64_t QUANT_SMALL = 98304;
+__global__ __launch_bounds__(SMALL_TPB) void k_quant_tensor_small(const float* __restrict__ x, int n,
+                                                                  double* __restrict__ scale,
+                                                                  int8_t* __restrict__ q) {
+  __shared__ int red[SMALL_TPB / 64];
+  const int tid = threadIdx.x, n4 = n >> 2;
+  const float4* x4 = reinterpret_cast<const float4*>(x);
+  int key = -1;
+#pragma unroll 8
+  for (int i = tid; i < n4; i += SMALL_TPB) {
+    const int k = key4(x4[i]);
+    key = key > k ? key : k;
+  }
+  for (int i = (n4 << 2) + tid; i < n; i += SMALL_TPB) {
+    const int k = absmax_key(x[i]);
+    key = key > k ? key : k;
+  }
+  key = block_max_i32_n<SMALL_TPB>(key, red);
+  const double s = scale_from_key(key);
+  if (blockIdx.x == 0 && tid == 0) *scale = s;
+  const bool fast = fast_scale_ok(s);
+  const float r32 = (float)(1.0 / s);
+  const int i = blockIdx.x * SMALL_TPB + tid;
+  if (i < n4) reinterpret_cast<int*>(q)[i] = quant4_sym(x4[i], fast, r32, s);
+  const int t = (n4 << 2) + i;
+  if (t < n) q[t] = (int8_t)(fast ? quant_sym_fast(x[t], r32, s) : quant_exact(x[t], s, 0.0, -128, 127));
+}
+
 hipError_t launch_quant_tensor(const float* x, int64_t n, int8_t* q, double* scales,
                                hipStream_t st) {
+  if (n > 0 && n <= QUANT_SMALL && ((reinterpret_cast<uintptr_t>(x) & 15) | (reinterpret_cast<uintptr_t>(q) & 3)) == 0) {
+    const int64_t g = (n + 4 * SMALL_TPB - 1) / (4 * SMALL_TPB);
+    hipLaunchKernelGGL(k_quant_tensor_small, dim3((unsigned)g), dim3(SMALL_TPB), 0, st, x, (int)n, scales, q);
+    return hipGetLastError();
+  }
   // A fill kernel (not a memset) starts the key, so the sequence can be
   // captured in a HIP graph.
   long long* dkey = reinterpret_cast<long long*>(scales);

@@ -1,0 +1,50 @@
+"""The small-call routes against the oracle: the one-launch per-tensor
+quantize at the edges of its range (with zeros, NaN and infinities, and
+misaligned tensors on the general route) and the dot4 GEMV of long rows."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+@pytest.fixture(scope="module")
+def ops():
+    if not torch.cuda.is_available():
+        pytest.skip("no HIP device")
+    from mlfw_amd import ops as O
+    from mlfw_amd import _lib
+    _lib.call("q8_init", 0)
+    return O
+
+
+def host(t):
+    torch.cuda.synchronize()
+    return t.cpu().numpy()
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 255, 4096, 4097, 65537, 98304, 98305])
+@pytest.mark.parametrize("kind", ["normal", "zeros", "nan", "inf", "tiny"])
+def test_quantize_per_tensor_small(ops, oracle, n, kind):
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal(n).astype(np.float32)
+    if kind == "zeros":
+        x[:] = -0.0
+    elif kind == "nan":
+        x[::2] = np.nan
+    elif kind == "inf":
+        x[n // 2] = -np.inf
+    elif kind == "tiny":
+        x *= np.float32(1e-42)
+    s = oracle.scale_per_tensor(x)
+    want = oracle.quantize(x, s)
+    for shift in (0, 1):
+        buf = torch.empty(n + 1, device=DEV)
+        d = buf[shift:shift + n]
+        d.copy_(torch.from_numpy(x))
+        q, sc = ops.quantize_per_tensor(d)
+        assert host(sc)[0] == s or (np.isnan(s) and np.isnan(host(sc)[0])), (kind, n)
+        np.testing.assert_array_equal(host(q), want)
