@@ -250,8 +250,8 @@ int q8_gemm(const int8_t* A, const int8_t* B, int64_t M, int64_t N, int64_t K,
 
 /* The skinny (decode) form of q8_gemm for 1 <= M <= 16: same contract,
  * HBM-bound kernels that stream the weight once: packed int8 dot products
- * (v_dot4_i32_i8) for M <= 4, one 16x16x64 int8 MFMA per 16 weight rows x
- * 64 K-bytes for 4 < M <= 16. */
+ * (v_dot4_i32_i8) for M <= 4 and K <= 20480, one 16x16x64 int8 MFMA per 16
+ * weight rows x 64 K-bytes otherwise. */
 int q8_gemv(const int8_t* A, const int8_t* B, int64_t M, int64_t N, int64_t K,
             const double* sA, int sA_mode, const double* sB, int sB_mode,
             int epi, double s_out, const float* bias, int act,

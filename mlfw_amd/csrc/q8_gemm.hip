@@ -1870,11 +1870,17 @@ template <int MT>
 static hipError_t launch_gemv_mt(const int8_t* A, const int8_t* B, int M, int N, int K,
                                  const GemmEpi& e, void* out, hipStream_t st) {
   const dim3 grid((unsigned)((N + GV_ROWS - 1) / GV_ROWS)), block(256);
-  const int cpt = (K / 16 + 255) / 256;               // <= 2 (K <= 8192)
+  const int cpt = (K / 16 + 255) / 256;               // <= 5 (K <= 20480)
   if (cpt <= 1)
     hipLaunchKernelGGL((k_gemv_i8<MT, 1>), grid, block, 0, st, A, B, M, N, K, e, out);
-  else
+  else if (cpt == 2)
     hipLaunchKernelGGL((k_gemv_i8<MT, 2>), grid, block, 0, st, A, B, M, N, K, e, out);
+  else if (cpt == 3)
+    hipLaunchKernelGGL((k_gemv_i8<MT, 3>), grid, block, 0, st, A, B, M, N, K, e, out);
+  else if (cpt == 4)
+    hipLaunchKernelGGL((k_gemv_i8<MT, 4>), grid, block, 0, st, A, B, M, N, K, e, out);
+  else
+    hipLaunchKernelGGL((k_gemv_i8<MT, 5>), grid, block, 0, st, A, B, M, N, K, e, out);
   return hipGetLastError();
 }
 
@@ -1910,13 +1916,16 @@ hipError_t launch_gemv(const int8_t* A, const int8_t* B, int64_t M, int64_t N, i
                        const GemmEpi& e, void* out, hipStream_t st) {
   if (M == 0 || N == 0) return hipSuccess;
   // 16-byte chunks and aligned rows, else the GEMM kernels (which handle
-  // any M).  The dot4 kernel keeps 16 weight rows of K <= 2 * 256 * 16
-  // bytes in registers; the MFMA kernel walks any K in passes.
+  // any M).  The dot4 kernel keeps 4 weight rows of K <= 5 * 256 * 16
+  // bytes in registers (the MFMA kernel, which pads the tokens to 16 and
+  // walks K in passes, takes 13.0 us for 1 x 4096 x 11008, dot4 9.4; 4
+  // tokens 13.4 and 11.8; 1 x 5120 x 20480 28.3 and 18.6); beyond that and
+  // for more tokens the MFMA kernel runs, with any K.
   const bool vec = (K % 16 == 0) && K > 0 && K < (int64_t)1 << 30 &&
                    ((reinterpret_cast<uintptr_t>(A) & 15) == 0) &&
                    ((reinterpret_cast<uintptr_t>(B) & 15) == 0);
   if (!vec) return launch_gemm(A, B, M, N, K, e, out, st);
-  if (M > 4 || K > 8192) {
+  if (M > 4 || K > 20480) {
     if (16 * K >= (int64_t)OOB) return launch_gemm(A, B, M, N, K, e, out, st);
     return launch_gemv_mfma(A, B, (int)M, (int)N, (int)K, e, out, st);
   }

@@ -48,3 +48,13 @@ def test_quantize_per_tensor_small(ops, oracle, n, kind):
         q, sc = ops.quantize_per_tensor(d)
         assert host(sc)[0] == s or (np.isnan(s) and np.isnan(host(sc)[0])), (kind, n)
         np.testing.assert_array_equal(host(q), want)
+
+
+@pytest.mark.parametrize("M", [1, 2, 3, 4])
+@pytest.mark.parametrize("N,K", [(5, 8208), (70, 12288), (33, 12304), (10, 16400), (7, 20480), (9, 20496)])
+def test_gemv_long_rows(ops, oracle, M, N, K):
+    rng = np.random.default_rng(M + N + K)
+    A = rng.integers(-128, 128, (M, K)).astype(np.int8)
+    B = rng.integers(-128, 128, (N, K)).astype(np.int8)
+    got = ops.quantized_dot(torch.from_numpy(A).to(DEV), torch.from_numpy(B).to(DEV))
+    np.testing.assert_array_equal(host(got), oracle.quantized_dot(A, B, 1))
