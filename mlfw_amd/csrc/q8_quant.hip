@@ -797,10 +797,11 @@ hipError_t launch_pack_weight(const float* W, int64_t rows, int64_t cols, int ax
 }
 
 // ------------------------------------------------------------------ SiLU(g)*u + per-token quantize
-// TPB threads per row: 256, or 512 for long rows, where a 256-thread
+// TPB threads per row: 256; 512 for long rows, where a 256-thread
 // block would hold 8-12 float4 of g and of u per lane and run 2 waves per
 // SIMD; at 512 threads a lane holds 4-6 and the SIMD keeps more waves to
-// hide the f64 exp behind the loads of other rows.
+// hide the f64 exp behind the loads of other rows; 1024 where the rows are
+// too few to share the CUs or too long for 512.
 template <int VPT, int TPB>
 __global__ __launch_bounds__(TPB) void k_silu_mul_quant_rows(const float* __restrict__ g,
                                                              const float* __restrict__ u,
@@ -858,7 +859,7 @@ __global__ __launch_bounds__(TPB) void k_silu_mul_quant_rows(const float* __rest
 }
 
 // Fallback for K % 4 != 0, a row stride that is not a multiple of 4,
-// misaligned pointers or rows above 12 Ki elements: h is formed twice (scan,
+// misaligned pointers or rows above 20 Ki elements: h is formed twice (scan,
 // then quantize) from g and u.
 __global__ __launch_bounds__(NT) void k_silu_mul_quant_rows_scalar(
     const float* __restrict__ g, const float* __restrict__ u, int64_t ldg, int64_t ldu, int64_t M,
@@ -890,7 +891,7 @@ hipError_t launch_silu_mul_quant_rows(const float* g, int64_t ldg, const float* 
                                       float* h, int8_t* q, double* scales, hipStream_t st) {
   if (M == 0) return hipSuccess;
   const int grid = (int)(M < 1048576 ? M : 1048576);
-  const bool vec = (K % 4 == 0) && (ldg % 4 == 0) && (ldu % 4 == 0) && (K / 4 <= 6 * 512) &&
+  const bool vec = (K % 4 == 0) && (ldg % 4 == 0) && (ldu % 4 == 0) && (K / 4 <= 5 * 1024) &&
                    ((reinterpret_cast<uintptr_t>(g) & 15) == 0) &&
                    ((reinterpret_cast<uintptr_t>(u) & 15) == 0) &&
                    ((reinterpret_cast<uintptr_t>(h) & 15) == 0) &&
@@ -907,18 +908,25 @@ hipError_t launch_silu_mul_quant_rows(const float* g, int64_t ldg, const float* 
     return hipGetLastError();
   }
   const int workers = (int)(M < 8 * cu_count() ? M : 8 * cu_count());
-  // 256 threads per row up to 4 float4 per lane, then 512 (measured at
+  // Many rows: 256 threads per row up to 4 float4 per lane, then 512 (measured at
   // [2048, 8192] and [2048, 11008] against 256 threads x 8-12 and 1024
   // threads x 2-3 per lane, with and without occupancy limits)
-  if (K4 <= 4 * 256)
-    hipLaunchKernelGGL((k_silu_mul_quant_rows<4, 256>), dim3(workers), dim3(256), 0, st, g, u, ldg, ldu, M, K,
-                       h, q, scales);
-  else if (K4 <= 4 * 512)
-    hipLaunchKernelGGL((k_silu_mul_quant_rows<4, 512>), dim3(workers), dim3(512), 0, st, g, u, ldg, ldu, M, K,
-                       h, q, scales);
-  else
-    hipLaunchKernelGGL((k_silu_mul_quant_rows<6, 512>), dim3(workers), dim3(512), 0, st, g, u, ldg, ldu, M, K,
-                       h, q, scales);
+#define Q8_SILU(VPT, TPB)                                                                                     \
+  hipLaunchKernelGGL((k_silu_mul_quant_rows<VPT, TPB>), dim3(workers), dim3(TPB), 0, st, g, u, ldg, ldu, M, K, \
+                     h, q, scales)
+  // Up to a row per CU a row's f64 exps are one CU's work, and 16 waves get
+  // through them a little sooner than 8 (1 x 11008 7.4 -> 6.8 us, 64 x 11008
+  // 7.9 -> 7.2; rows of 4096 and below 0.3 us later).  Rows of more than 12288
+  // fit 1024 threads only (1 x 16320: 46.9 us with h formed twice from
+  // scalar loads, 9.4 us).
+  if (K4 > 6 * 512 || (M <= cu_count() && K4 > 1024)) {
+    if (K4 <= 2 * 1024) Q8_SILU(2, 1024);
+    else if (K4 <= 3 * 1024) Q8_SILU(3, 1024);
+    else Q8_SILU(5, 1024);
+  } else if (K4 <= 4 * 256) Q8_SILU(4, 256);
+  else if (K4 <= 4 * 512) Q8_SILU(4, 512);
+  else Q8_SILU(6, 512);
+#undef Q8_SILU
   return hipGetLastError();
 }
 

@@ -1,6 +1,7 @@
 """The small-call routes against the oracle: the one-launch per-tensor
 quantize at the edges of its range (with zeros, NaN and infinities, and
-misaligned tensors on the general route) and the dot4 GEMV of long rows."""
+misaligned tensors on the general route), the dot4 GEMV of long rows and
+SiLU * up + quantize on either side of its row-length limits."""
 import numpy as np
 import pytest
 
@@ -58,3 +59,22 @@ def test_gemv_long_rows(ops, oracle, M, N, K):
     B = rng.integers(-128, 128, (N, K)).astype(np.int8)
     got = ops.quantized_dot(torch.from_numpy(A).to(DEV), torch.from_numpy(B).to(DEV))
     np.testing.assert_array_equal(host(got), oracle.quantized_dot(A, B, 1))
+
+
+@pytest.mark.parametrize("M", [1, 3, 300])
+@pytest.mark.parametrize("K", [4096, 4100, 8192, 8196, 11008, 12288, 12292, 13376, 20480, 20484])
+def test_silu_rows(ops, oracle, M, K):
+    rng = np.random.default_rng(M + K)
+    gu = (rng.standard_normal((M, 2 * K)) * 4).astype(np.float32)
+    gu[0, K - 1] = np.inf
+    gu[M - 1, K // 2] = np.nan
+    h = oracle.silu_mul(np.ascontiguousarray(gu[:, :K]), np.ascontiguousarray(gu[:, K:]))
+    s = oracle.scales_per_token(h)
+    want = oracle.quantize_rows(h, s)
+    d = torch.from_numpy(gu).to(DEV)
+    h_out = torch.empty(M, K, device=DEV)
+    for g, u in ((d[:, :K], d[:, K:]), (d[:, :K].contiguous(), d[:, K:].contiguous())):
+        q, sc = ops.silu_mul_quantize(g, u, h_out)
+        np.testing.assert_array_equal(host(h_out), h)
+        np.testing.assert_array_equal(host(sc), s)
+        np.testing.assert_array_equal(host(q), want)
