@@ -372,8 +372,8 @@ CONV_LAYERS = [(32, 64, 56, 56, 64, 3, 1), (32, 128, 28, 28, 128, 3, 1), (32, 25
 
 def bench_conv():
     """quantized_conv with the fused per-tensor dequant (fp32 out), int8
-    operands: the whole call per launch (frame transpose, implicit GEMM,
-    split-K finish where planned), 8 calls per graph.  The constant weight
+    operands: the whole call per launch (frame transpose, implicit GEMM),
+    8 calls per graph.  The constant weight
     is prepacked once (conv_weight_taps); avg_us_unpacked_weight is the call
     that permutes the weight itself."""
     import torch

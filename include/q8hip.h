@@ -424,7 +424,8 @@ int q8_pack_weight_int4(const float* W, int64_t N, int64_t K, int64_t group_size
  * Kernels: packed dot products for M <= 2 (M <= 4 where K or the group
  * rule out the MFMA kernel) with a power-of-two group_size in [32, 2048]
  * and K <= 8192; the MFMA kernel for any M (blocks of 16 tokens) with K and
- * group_size multiples of 32; any other shape (a group that is not a
+ * group_size multiples of 32; a tiled GEMM for M > 16 where it is faster
+ * (groups of 32, 64 or a multiple of 128); any other shape (a group that is not a
  * multiple of 32) runs a simple exact kernel.  All give the same bits. */
 int q8_gemv_w4(const int8_t* xq, const double* sx, int sx_mode, const uint8_t* Wq4,
                const double* sw, int64_t M, int64_t N, int64_t K, int64_t group_size,
@@ -447,11 +448,12 @@ int q8_gemv_w4(const int8_t* xq, const double* sx, int sx_mode, const uint8_t* W
  *   (x[n, g*C/groups + ic, p*stride + k*dilation - pad_lo] - zp_x) * (w[o, ic, k] - zp_w),
  *   g = o / (O/groups); a tap in the padding adds 0; int32 wrap-around.
  * out_kind Q8_I32: out = acc; Q8_F32: out = fround(acc * s_out).
- * Zero points (the op's input_zero_point / kernel_zero_point) run the
- * direct kernel, exact for any value.
- * workspace: device memory of at least q8_quantized_conv_workspace bytes
- * (may be 0: then NULL is accepted); calls that share a workspace must be
- * ordered (same stream). */
+ * Zero points (the op's input_zero_point / kernel_zero_point) run the same
+ * kernels, exact for any value.
+ * workspace: device memory of q8_quantized_conv_workspace bytes (may be 0:
+ * then NULL is accepted).  A call with zero points is accepted with less and
+ * then takes a slower kernel, one thread per output.  Calls that share a
+ * workspace must be ordered (same stream). */
 int q8_quantized_conv_workspace(int spatial_dims, const int64_t* x_shape, const int64_t* w_shape,
                                 const int64_t* strides, const int64_t* pad_lo,
                                 const int64_t* pad_hi, const int64_t* dilation, int64_t groups,
@@ -463,7 +465,7 @@ int q8_quantized_conv(const int8_t* x, const int8_t* w, int spatial_dims, const 
                       size_t workspace_bytes, void* out, void* stream);
 /* The same with the operand types: x_dtype / w_dtype Q8_I8 or Q8_U8 (the
  * lowering reads Int8Array or Uint8Array elements; the op admits mixed
- * types, ops/quantization.ts:176-178).  ui8 operands run the direct kernel. */
+ * types, ops/quantization.ts:176-178).  The workspace rule is the one of zero points. */
 int q8_quantized_conv_ex(const void* x, int x_dtype, const void* w, int w_dtype, int spatial_dims,
                          const int64_t* x_shape, const int64_t* w_shape, const int64_t* strides,
                          const int64_t* pad_lo, const int64_t* pad_hi, const int64_t* dilation,

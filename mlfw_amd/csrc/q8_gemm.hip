@@ -1804,7 +1804,9 @@ void k_gemv_mfma(const int8_t* __restrict__ A, const int8_t* __restrict__ B, int
       // launch at N = 4096, K = 1024..4096).  With several blocks per
       // workgroup the loop below stays: walking balanced row ranges, or
       // issuing the next block's weights before this block's MFMAs, was
-      // slower there (N = 11008, M <= 8: 12.0 -> 12.5-13.5 us).
+      // slower there (N = 11008, M <= 8: 12.0 -> 12.5-13.5 us), also with
+      // two blocks' copies always in flight in a second LDS buffer (N = 22016,
+      // K = 4096, M = 16: 21.4 -> 22.0 us; N = 4096, K = 11008: 14.4 -> 15.3).
       load_x(0);
       const int n0 = (int)blockIdx.x * 16;
       const int rows = N - n0 < 16 ? N - n0 : 16;

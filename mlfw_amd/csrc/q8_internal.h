@@ -209,7 +209,7 @@ struct ConvGeom {
   int x_u8 = 0, w_u8 = 0;        // operands read as ui8 (else i8)
 };
 // Whether the conv runs the direct kernel (exact, one thread per output):
-// Cg * prod(K) < 64, or zero points / ui8 operands with less workspace than
+// short contractions of small products, zero points / ui8 operands with less workspace than
 // the GEMM paths need or an input zero point outside its type.
 bool conv_direct(const ConvGeom& G, size_t workspace_bytes);
 bool conv_uses_gemm(const ConvGeom& G);

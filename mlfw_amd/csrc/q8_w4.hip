@@ -25,7 +25,10 @@
 // acc_g * sw_g (f64) to LDS, and one lane per (row, token) adds the groups
 // in order from LDS.  HBM-bound on the K / 2 bytes per row: half the int8
 // weight traffic.
-// Generic kernel (any M, any group dividing K): one thread per output.
+// More than 16 tokens go to the tiled GEMM (q8_w4_gemm.hip) where it applies;
+// other M >= 3 to the MFMA kernel below, in blocks of 16 tokens.
+// Generic kernel (any M, any group dividing K): one thread per output, for
+// groups the others cannot split.
 #include <algorithm>
 
 #include "q8_device.h"
