@@ -492,6 +492,17 @@ int q8_quantized_conv_prepacked(const int8_t* x, const int8_t* w, const int8_t* 
                                 int64_t groups, int32_t zp_x, int32_t zp_w, int out_kind, double s_out,
                                 void* workspace, size_t workspace_bytes, void* out, void* stream);
 
+/* For tests and diagnosis, no counterpart in the reference: how a conv call
+ * of these arguments would run, launching nothing (the workspace's address is
+ * looked at, not its memory).  route: 0 one thread per output, 1 channel-last
+ * frame, 2 matrix of receptive fields; images and groups of one pass; bytes
+ * of the workspace, from its start, that no pass writes past (all three 0 for
+ * route 0).  Refuses what the call itself refuses. */
+int q8_debug_conv_plan(int spatial_dims, const int64_t* x_shape, const int64_t* w_shape, const int64_t* strides,
+                       const int64_t* pad_lo, const int64_t* pad_hi, const int64_t* dilation, int64_t groups,
+                       int x_dtype, int32_t zp_x, int w_dtype, int32_t zp_w, int prepacked, const void* workspace,
+                       size_t workspace_bytes, int* route, int64_t* images, int64_t* group_count, size_t* bytes);
+
 /* ---------------------------------------------------------------- fused */
 
 /* h = fround(silu(g) * u) for the gated MLP (SiLU decomposition

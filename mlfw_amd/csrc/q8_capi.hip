@@ -935,6 +935,25 @@ int q8_quantized_conv_workspace(int spatial_dims, const int64_t* x_shape, const 
   return Q8_OK;
 }
 
+// The operand types and the workspace of a conv call: its plan.
+static int conv_check(const char* who, int x_dtype, int w_dtype, int32_t zp_x, int32_t zp_w, bool prepacked,
+                      const void* workspace, size_t workspace_bytes, q8::ConvGeom* G, q8::ConvPlan* plan) {
+  Q8_REQUIRE((x_dtype == Q8_I8 || x_dtype == Q8_U8) && (w_dtype == Q8_I8 || w_dtype == Q8_U8),
+             "%s: operands must be Q8_I8 or Q8_U8 (got %d, %d)", who, x_dtype, w_dtype);
+  G->zpx = zp_x;
+  G->zpw = zp_w;
+  G->x_u8 = x_dtype == Q8_U8;
+  G->w_u8 = w_dtype == Q8_U8;
+  const bool empty = G->N * G->O * G->Pn == 0;
+  const size_t need = q8::conv_uses_gemm(*G) && !q8::conv_affine(*G) ? q8::conv_workspace_need(*G) : 0;
+  Q8_REQUIRE(empty || workspace_bytes >= need,
+             "%s: workspace of %zu bytes is smaller than the %zu bytes required "
+             "(q8_quantized_conv_workspace)", who, workspace_bytes, need);
+  Q8_REQUIRE(empty || need == 0 || workspace, "%s: workspace is NULL", who);
+  *plan = q8::conv_plan(*G, workspace, workspace_bytes, prepacked);
+  return Q8_OK;
+}
+
 static int conv_impl(const char* who, const void* x, int x_dtype, const void* w, int w_dtype,
                      const int8_t* w_taps, int spatial_dims, const int64_t* x_shape, const int64_t* w_shape,
                      const int64_t* strides, const int64_t* pad_lo, const int64_t* pad_hi,
@@ -946,19 +965,10 @@ static int conv_impl(const char* who, const void* x, int x_dtype, const void* w,
                      &G);
   if (rc != Q8_OK) return rc;
   Q8_REQUIRE(out_kind == Q8_F32 || out_kind == Q8_I32, "%s: out_kind must be Q8_F32 or Q8_I32", who);
-  Q8_REQUIRE((x_dtype == Q8_I8 || x_dtype == Q8_U8) && (w_dtype == Q8_I8 || w_dtype == Q8_U8),
-             "%s: operands must be Q8_I8 or Q8_U8 (got %d, %d)", who, x_dtype, w_dtype);
-  G.zpx = zp_x;
-  G.zpw = zp_w;
-  G.x_u8 = x_dtype == Q8_U8;
-  G.w_u8 = w_dtype == Q8_U8;
-  const bool empty = G.N * G.O * G.Pn == 0;
-  Q8_REQUIRE(empty || (x && w && out), "%s: NULL pointer", who);
-  const size_t need = q8::conv_direct(G, workspace ? workspace_bytes : 0) ? 0 : q8::conv_workspace_need(G);
-  Q8_REQUIRE(empty || workspace_bytes >= need,
-             "%s: workspace of %zu bytes is smaller than the %zu bytes required "
-             "(q8_quantized_conv_workspace)", who, workspace_bytes, need);
-  Q8_REQUIRE(empty || need == 0 || workspace, "%s: workspace is NULL", who);
+  Q8_REQUIRE(G.N * G.O * G.Pn == 0 || (x && w && out), "%s: NULL pointer", who);
+  q8::ConvPlan plan;
+  rc = conv_check(who, x_dtype, w_dtype, zp_x, zp_w, w_taps != nullptr, workspace, workspace_bytes, &G, &plan);
+  if (rc != Q8_OK) return rc;
   q8::GemmEpi e{};
   e.mode = 0;
   e.s_out = s_out;
@@ -970,8 +980,29 @@ static int conv_impl(const char* who, const void* x, int x_dtype, const void* w,
     Q8_REQUIRE((reinterpret_cast<uintptr_t>(w_taps) & 15) == 0, "%s: w_taps must be 16-byte aligned", who);
   }
   return launched(q8::launch_conv(static_cast<const int8_t*>(x), static_cast<const int8_t*>(w), w_taps, G,
-                                  e, workspace, workspace_bytes, out, as_stream(stream)),
+                                  e, plan, workspace, out, as_stream(stream)),
                   "quantized_conv launch");
+}
+
+int q8_debug_conv_plan(int spatial_dims, const int64_t* x_shape, const int64_t* w_shape, const int64_t* strides,
+                       const int64_t* pad_lo, const int64_t* pad_hi, const int64_t* dilation, int64_t groups,
+                       int x_dtype, int32_t zp_x, int w_dtype, int32_t zp_w, int prepacked, const void* workspace,
+                       size_t workspace_bytes, int* route, int64_t* images, int64_t* group_count, size_t* bytes) {
+  Q8_REQUIRE(route && images && group_count && bytes, "q8_debug_conv_plan: NULL pointer");
+  q8::ConvGeom G;
+  int rc = conv_geom("q8_debug_conv_plan", spatial_dims, x_shape, w_shape, strides, pad_lo, pad_hi, dilation,
+                     groups, &G);
+  if (rc != Q8_OK) return rc;
+  q8::ConvPlan p;
+  rc = conv_check("q8_debug_conv_plan", x_dtype, w_dtype, zp_x, zp_w, prepacked != 0, workspace, workspace_bytes, &G,
+                  &p);
+  if (rc != Q8_OK) return rc;
+  *route = p.route;
+  *images = p.nb;
+  *group_count = p.gc;
+  *bytes = p.bytes;
+  g_err[0] = '\0';
+  return Q8_OK;
 }
 
 int q8_conv_weight_taps(const int8_t* w, int spatial_dims, const int64_t* w_shape, int64_t groups,

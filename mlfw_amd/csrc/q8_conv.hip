@@ -241,8 +241,8 @@ __device__ __forceinline__ void weight_taps(const int8_t* __restrict__ w, int64_
   const int slices = Cg >> 4;
   const int64_t s0 = blk * ns;
   const int n = (int)(nslices - s0 < ns ? nslices - s0 : ns);      // slices of this workgroup
-  const v4i* src = reinterpret_cast<const v4i*>(w + s0 * 16 * Kn);   // 16-byte aligned
-  for (int i = threadIdx.x; i < n * Kn; i += 256) reinterpret_cast<v4i*>(buf)[i] = src[i];
+  const int8_t* src = w + s0 * 16 * Kn;                            // any byte address
+  for (int i = threadIdx.x; i < n * Kn; i += 256) reinterpret_cast<v4i*>(buf)[i] = load16_any(src + 16 * (int64_t)i);
   __syncthreads();
   for (int i = threadIdx.x; i < n * Kn; i += 256) {
     const int t = i / n, sl = i - t * n;
@@ -360,14 +360,7 @@ static bool conv_short_gemm(const ConvGeom& G) {
 // tap in the padding holds.  Zero points outside the type's range have none.
 static int64_t conv_fill(const ConvGeom& G) { return (int64_t)G.zpx - (G.x_u8 ? 128 : 0); }
 
-static bool conv_affine(const ConvGeom& G) { return G.zpx != 0 || G.zpw != 0 || G.x_u8 || G.w_u8; }
-
-bool conv_direct(const ConvGeom& G, size_t workspace_bytes) {
-  if (conv_uses_gemm(G) && !conv_affine(G)) return false;
-  if (conv_fill(G) < -128 || conv_fill(G) > 127) return true;
-  if (conv_uses_gemm(G)) return workspace_bytes < conv_workspace_need(G);
-  return !conv_short_gemm(G) || workspace_bytes < conv_workspace_bytes(G);
-}
+bool conv_affine(const ConvGeom& G) { return G.zpx != 0 || G.zpw != 0 || G.x_u8 || G.w_u8; }
 
 constexpr size_t CONV_BATCH_BYTES = (size_t)128 << 20;   // workspace per batch of images
 static size_t round256(size_t b) { return (b + 255) & ~(size_t)255; }
@@ -470,28 +463,55 @@ size_t conv_workspace_bytes(const ConvGeom& G) {
   return want > need ? want : need;
 }
 
-// Images and groups of one pass: `unit` bytes each, within `avail` and the
-// launch limits.
-struct ConvBatch {
-  int64_t nb;
-  int gc;
-};
-static ConvBatch conv_batch(const ConvGeom& G, size_t unit, size_t avail) {
-  int64_t units = unit ? (int64_t)(avail / unit) : 1;
-  ConvBatch b;
-  const int64_t fit = unit ? (((int64_t)1 << 31) - 1) / (int64_t)unit : units;   // one image's offsets in 31 bits
+// Images and groups of one pass over `unit` workspace bytes each, with the
+// weight rows' wt before or after them: as many as fit `avail` and the launch
+// limits.  False where not even one does.
+static bool conv_batch(const ConvGeom& G, size_t unit, size_t wt, size_t avail, ConvPlan* p) {
+  if (avail < wt || avail - wt < unit) return false;
+  const int64_t units = (int64_t)((avail - wt) / unit);
+  const int64_t fit = (((int64_t)1 << 31) - 1) / (int64_t)unit;           // one pass's offsets in 31 bits
   int64_t gc = units < G.groups ? units : G.groups;
   gc = gc < fit ? gc : fit;
   gc = gc < 65535 ? gc : 65535;
-  b.gc = (int)(gc < 1 ? 1 : gc);
-  b.nb = b.gc == G.groups ? units / b.gc : 1;
-  b.nb = b.nb > G.N ? G.N : b.nb;
-  b.nb = b.nb > 65535 ? 65535 : b.nb;                                     // grid.y of k_im2col
-  const int64_t cap = ((int64_t)1 << 31) / (G.Pn > 0 ? G.Pn : 1) - 1;     // GEMM N = nb * P in an int
-  b.nb = b.nb > cap ? cap : b.nb;
-  b.nb = b.nb > fit / b.gc ? fit / b.gc : b.nb;
-  b.nb = b.nb < 1 ? 1 : b.nb;
-  return b;
+  gc = gc < 1 ? 1 : gc;
+  int64_t nb = gc == G.groups ? units / gc : 1;
+  nb = nb > G.N ? G.N : nb;
+  nb = nb > 65535 ? 65535 : nb;                                           // grid.y of the per-image launches
+  const int64_t cap = ((int64_t)1 << 31) / G.Pn - 1;                      // GEMM N = nb * P in an int
+  nb = nb > cap ? cap : nb;
+  nb = nb > fit / gc ? fit / gc : nb;
+  p->gc = (int)gc;
+  p->nb = nb < 1 ? 1 : nb;
+  p->wt = wt;
+  p->bytes = p->skip + wt + (size_t)p->nb * (size_t)gc * unit;
+  return true;
+}
+
+// Symmetric int8 with more than two tiles per CU: weight rows padded to the
+// matrix's pitch for the direct-to-LDS GEMM (32 x 3 x 112 x 112, 7 x 7 at
+// stride 2: 48.4 us against 53.5 with the weight at its own pitch).
+static bool conv_im2col_many(const ConvGeom& G) {
+  const int64_t t64 = ((G.Og + 63) / 64) * ((G.N * G.Pn + 63) / 64);
+  return !conv_affine(G) && G.groups == 1 && t64 > 2 * (cu_count() > 0 ? cu_count() : 256) &&
+         (int64_t)G.Kc16 * 256 < ((int64_t)1 << 31);
+}
+
+ConvPlan conv_plan(const ConvGeom& G, const void* ws, size_t ws_bytes, bool prepacked) {
+  ConvPlan p;
+  if (ws == nullptr || G.N * G.O * G.Pn == 0 || !(conv_uses_gemm(G) || conv_short_gemm(G))) return p;
+  if (conv_fill(G) < -128 || conv_fill(G) > 127) return p;
+  if (conv_uses_gemm(G) ? conv_affine(G) && ws_bytes < conv_workspace_need(G) : ws_bytes < conv_workspace_bytes(G))
+    return p;
+  p.skip = (16 - (reinterpret_cast<uintptr_t>(ws) & 15)) & 15;
+  const size_t avail = ws_bytes > p.skip ? ws_bytes - p.skip : 0;
+  ConvFrame F;
+  const size_t unit = (size_t)G.Pn * (size_t)G.Kc16;
+  if (conv_frame_path(G, &F) && conv_batch(G, (size_t)F.Ep * (size_t)G.Cg, prepacked ? 0 : conv_wt_bytes(G), avail, &p))
+    p.route = ConvPlan::FRAME;
+  else if ((conv_im2col_many(G) && G.Kc16 != G.Kc && conv_batch(G, unit, (size_t)G.O * (size_t)G.Kc16, avail, &p)) ||
+           conv_batch(G, unit, 0, avail, &p))
+    p.route = ConvPlan::IM2COL;
+  return p;
 }
 
 // The affine correction of the conv's GEMM (A: weights, B: input).
@@ -506,11 +526,9 @@ static AffineDot conv_zp(const ConvGeom& G) {
 
 static hipError_t launch_conv_channel_last(const int8_t* x, const int8_t* w, const int8_t* w_taps,
                                            const ConvGeom& G, const ConvFrame& F, const GemmEpi& e,
-                                           void* workspace, size_t ws_bytes, void* out, hipStream_t st) {
-  const size_t wt_bytes = w_taps ? 0 : conv_wt_bytes(G);
-  int8_t* wt_ws = static_cast<int8_t*>(workspace);
-  int8_t* xp = wt_ws + wt_bytes;
-  const ConvBatch cb = conv_batch(G, (size_t)F.Ep * (size_t)G.Cg, ws_bytes - wt_bytes);
+                                           const ConvPlan& cb, int8_t* workspace, void* out, hipStream_t st) {
+  int8_t* wt_ws = workspace;
+  int8_t* xp = wt_ws + cb.wt;
   // a 1 x 1 kernel's weight is its own tap-major form; a prepacked one
   // (q8_conv_weight_taps) is used as given
   const int8_t* wt = G.Kn == 1 ? w : w_taps ? w_taps : wt_ws;
@@ -596,18 +614,10 @@ static hipError_t launch_conv_channel_last(const int8_t* x, const int8_t* w, con
 // Receptive fields as a matrix (k_im2col), every group of a batch of images
 // at once; the GEMM takes the weight rows at their own pitch.
 static hipError_t launch_conv_im2col(const int8_t* x, const int8_t* w, const ConvGeom& G, const GemmEpi& e,
-                                     void* workspace, size_t ws_bytes, void* out, hipStream_t st) {
-  int8_t* col = static_cast<int8_t*>(workspace);
-  // symmetric int8 with more than two tiles per CU: weight rows padded to the
-  // matrix's pitch for the direct-to-LDS GEMM (32 x 3 x 112 x 112, 7 x 7 at
-  // stride 2: 48.4 us against 53.5 with the weight at its own pitch)
-  const int64_t t64 = ((G.Og + 63) / 64) * ((G.N * G.Pn + 63) / 64);
-  const bool many = !conv_affine(G) && G.groups == 1 && t64 > 2 * (cu_count() > 0 ? cu_count() : 256) &&
-                    (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 && (int64_t)G.Kc16 * 256 < ((int64_t)1 << 31);
-  const size_t wp_bytes = many && G.Kc16 != G.Kc ? (size_t)G.O * (size_t)G.Kc16 : 0;
-  const ConvBatch cb = conv_batch(G, (size_t)G.Pn * (size_t)G.Kc16, ws_bytes - wp_bytes);
+                                     const ConvPlan& cb, int8_t* col, void* out, hipStream_t st) {
+  const bool many = conv_im2col_many(G);
   const int8_t* wmat = w;
-  if (wp_bytes) {
+  if (cb.wt) {
     int8_t* wp = col + (size_t)cb.nb * (size_t)G.Pn * (size_t)G.Kc16;   // Kc16 % 16 == 0: stays aligned
     const int64_t n = G.O * G.Kc16;
     hipLaunchKernelGGL(k_pad_rows, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, w, G.O, (int64_t)G.Kc,
@@ -636,7 +646,7 @@ static hipError_t launch_conv_im2col(const int8_t* x, const int8_t* w, const Con
       hipError_t err = hipGetLastError();
       if (err != hipSuccess) return err;
       void* o = static_cast<char*>(out) + (size_t)((n0 * G.O + g * G.Og) * G.Pn) * osz;
-      if (many && (reinterpret_cast<uintptr_t>(wmat) & 15) == 0) {
+      if (many && (cb.wt || G.Kc16 == G.Kc) && (reinterpret_cast<uintptr_t>(wmat) & 15) == 0) {
         err = launch_gemm(wmat, col, G.Og, nb * G.Pn, G.Kc16, eb, o, st);
         if (err != hipSuccess) return err;
         continue;
@@ -668,19 +678,19 @@ hipError_t launch_conv_weight_taps(const int8_t* w, const ConvGeom& G, int8_t* w
 }
 
 hipError_t launch_conv(const int8_t* x, const int8_t* w, const int8_t* w_taps, const ConvGeom& G,
-                       const GemmEpi& e, void* workspace, size_t ws_bytes, void* out, hipStream_t st) {
+                       const GemmEpi& e, const ConvPlan& p, void* workspace, void* out, hipStream_t st) {
   if (G.N * G.O * G.Pn == 0) return hipSuccess;
-  if (conv_direct(G, workspace ? ws_bytes : 0)) {
+  if (p.route == ConvPlan::DIRECT) {
     const int64_t total = G.N * G.O * G.Pn;
     hipLaunchKernelGGL(k_conv_direct, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, x,
                        w, G, e, out);
     return hipGetLastError();
   }
+  int8_t* ws = static_cast<int8_t*>(workspace) + p.skip;
+  if (p.route == ConvPlan::IM2COL) return launch_conv_im2col(x, w, G, e, p, ws, out, st);
   ConvFrame F;
-  const bool aligned = ((reinterpret_cast<uintptr_t>(workspace) | (G.Kn > 1 && !w_taps ? reinterpret_cast<uintptr_t>(w) : 0)) & 15) == 0;
-  if (conv_frame_path(G, &F) && aligned)
-    return launch_conv_channel_last(x, w, w_taps, G, F, e, workspace, ws_bytes, out, st);
-  return launch_conv_im2col(x, w, G, e, workspace, ws_bytes, out, st);
+  if (!conv_frame_path(G, &F)) return hipErrorInvalidValue;
+  return launch_conv_channel_last(x, w, w_taps, G, F, e, p, ws, out, st);
 }
 
 }  // namespace q8

@@ -17,6 +17,13 @@ typedef int v2i __attribute__((ext_vector_type(2)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 
+// 16 bytes from any byte address (one global_load_dwordx4).
+__device__ __forceinline__ v4i load16_any(const int8_t* p) {
+  v4i v;
+  __builtin_memcpy(&v, p, 16);
+  return v;
+}
+
 // ECMA-262 Math.round for an exact double.  y - floor(y) is exact.
 __device__ __forceinline__ double js_round(double y) {
   double r = floor(y);

@@ -61,12 +61,6 @@ __device__ __forceinline__ v4i shift_down(v4i v, int sh) {
              (int)__builtin_amdgcn_alignbyte(0u, (uint32_t)t.w, b)};
 }
 
-__device__ __forceinline__ v4i load16_any(const int8_t* p) {
-  v4i v;
-  __builtin_memcpy(&v, p, 16);   // global_load_dwordx4; any byte address
-  return v;
-}
-
 __device__ __forceinline__ int sum16(v4i v, int s) {
   s = __builtin_amdgcn_sdot4(v.x, 0x01010101, s, false);
   s = __builtin_amdgcn_sdot4(v.y, 0x01010101, s, false);

@@ -208,17 +208,30 @@ struct ConvGeom {
   int zpx = 0, zpw = 0;          // input / kernel zero points
   int x_u8 = 0, w_u8 = 0;        // operands read as ui8 (else i8)
 };
-// Whether the conv runs the direct kernel (exact, one thread per output):
-// short contractions of small products, zero points / ui8 operands with less workspace than
-// the GEMM paths need or an input zero point outside its type.
-bool conv_direct(const ConvGeom& G, size_t workspace_bytes);
+// How a conv runs with the workspace it is given: the direct kernel (exact,
+// one thread per output: short contractions of small products, an input zero
+// point outside its type, or nothing of the other two fits), the channel-last
+// frame or the matrix of receptive fields.  Everything that decides it is
+// here, so that what a launch writes is what was checked against the
+// workspace.
+struct ConvPlan {
+  enum Route { DIRECT, FRAME, IM2COL };
+  int route = DIRECT;
+  int gc = 0;         // groups and
+  int64_t nb = 0;     // images of one pass
+  size_t skip = 0;    // bytes up to the workspace's first 16-byte boundary
+  size_t wt = 0;      // bytes of the weight's form that the GEMM reads (tap-major, or padded rows)
+  size_t bytes = 0;   // of the workspace from its start: nothing past them is written
+};
+ConvPlan conv_plan(const ConvGeom& G, const void* ws, size_t ws_bytes, bool prepacked);
+bool conv_affine(const ConvGeom& G);
 bool conv_uses_gemm(const ConvGeom& G);
 size_t conv_workspace_need(const ConvGeom& G);    // the least a call is accepted with
 size_t conv_workspace_bytes(const ConvGeom& G);   // what a caller is told to bring
 // w_taps (may be null): the weight already in the channel-last path's
 // tap-major form (launch_conv_weight_taps), which then is not permuted per call.
 hipError_t launch_conv(const int8_t* x, const int8_t* w, const int8_t* w_taps, const ConvGeom& G,
-                       const GemmEpi& e, void* workspace, size_t ws_bytes, void* out, hipStream_t st);
+                       const GemmEpi& e, const ConvPlan& p, void* workspace, void* out, hipStream_t st);
 // Whether the tap-major weight form is used for weights of G's shape (Cg a
 // multiple of 16, 2 <= prod(K) <= 1024), and the permutation that makes it:
 // w_taps[o][t * Cg + c] = w[o][c][t], O * Cg * prod(K) bytes.

@@ -241,3 +241,62 @@ def test_conv_affine_without_workspace(ops, oracle):
            arr(x.shape), arr(w.shape), arr([1, 1]), arr([1, 1]), arr([1, 1]), arr([1, 1]), 1, 99, 0, L.Q8_I32, 0.0,
            None, 0, C.c_void_p(out.data_ptr()), None)
     same_bits(host(out), oracle.quantized_conv(x, w, [1, 1], [[1, 1], [1, 1]], [1, 1], 1, 99, 0))
+
+
+def conv_call(x, w, st, pd, g=1, s_out=None, zpx=0, ws_bytes=None, ws_shift=0, w_shift=0, taps=None):
+    """quantized_conv through the C ABI with a workspace of ws_bytes (the size
+    asked for when None) that starts ws_shift bytes past an aligned address,
+    the weight w_shift bytes past one; the bytes around the workspace are
+    checked afterwards."""
+    import ctypes as C
+    from mlfw_amd import _lib as L
+    d = x.ndim - 2
+    arr = lambda v: (C.c_int64 * len(v))(*v)  # noqa: E731
+    lo, hi = [p[0] for p in pd], [p[1] for p in pd]
+    geom = (d, arr(x.shape), arr(w.shape), arr(st), arr(lo), arr(hi), arr([1] * d), g)
+    if ws_bytes is None:
+        need = C.c_size_t(0)
+        L.call("q8_quantized_conv_workspace", *geom, C.byref(need))
+        ws_bytes = need.value
+    GUARD = 4096
+    buf = torch.full((GUARD + ws_shift + ws_bytes + GUARD,), 0x5a, dtype=torch.uint8, device=DEV)
+    wbuf = torch.zeros(w.size + 64, dtype=torch.uint8, device=DEV)
+    wbuf[w_shift:w_shift + w.size] = dev(w.view(np.uint8).reshape(-1))
+    shape = (x.shape[0], w.shape[0], *[(x.shape[2 + i] + lo[i] + hi[i] - w.shape[2 + i]) // st[i] + 1 for i in range(d)])
+    out = torch.empty(shape, dtype=torch.int32 if s_out is None else torch.float32, device=DEV)
+    dx = dev(x)
+    p = lambda t, off=0: C.c_void_p(t.data_ptr() + off)  # noqa: E731
+    kind, s = (L.Q8_I32, 0.0) if s_out is None else (L.Q8_F32, s_out)
+    code = {np.dtype(np.int8): L.Q8_I8, np.dtype(np.uint8): L.Q8_U8}
+    ws = p(buf, GUARD + ws_shift) if ws_bytes else None
+    print(f"conv C ABI x{x.shape} w{w.shape} g{g} ws={ws_bytes}+{ws_shift} w+{w_shift}", flush=True)
+    if taps is not None:
+        L.call("q8_quantized_conv_prepacked", p(dx), p(wbuf, w_shift), p(taps), *geom, zpx, 0, kind, s, ws, ws_bytes,
+               p(out), None)
+    else:
+        L.call("q8_quantized_conv_ex", p(dx), code[x.dtype], p(wbuf, w_shift), code[w.dtype], *geom, zpx, 0, kind, s, ws,
+               ws_bytes, p(out), None)
+    got = host(out)
+    b = host(buf)
+    assert (b[:GUARD + ws_shift] == 0x5a).all() and (b[GUARD + ws_shift + ws_bytes:] == 0x5a).all(), "workspace overrun"
+    return got
+
+
+@pytest.mark.parametrize("ws_shift,w_shift", [(0, 1), (0, 8), (1, 0), (15, 3)])
+@pytest.mark.parametrize("xs,ws,pd", [((1, 16, 112, 112), (64, 16, 1, 3), [[0, 0], [1, 1]]),   # short, frame
+                                      ((1, 16, 6000), (64, 16, 3), [[1, 1]]),
+                                      ((2, 16, 6000), (128, 16, 2), [[0, 0]]),
+                                      ((2, 64, 9, 9), (48, 64, 3, 3), [[1, 1], [1, 1]]),       # frame
+                                      ((3, 10, 9, 11), (24, 10, 3, 3), [[1, 1], [1, 0]])])     # matrix
+@pytest.mark.parametrize("u8", [False, True])
+def test_conv_misaligned_weight_and_workspace(ops, oracle, xs, ws, pd, u8, ws_shift, w_shift):
+    """A weight (a view into a larger blob) and a workspace at any byte
+    address: the same bits, and nothing written outside a workspace of exactly
+    the size asked for."""
+    rng = np.random.default_rng(sum(xs) + ws_shift)
+    x = rng.integers(0, 256, xs).astype(np.uint8)
+    x = x if u8 else x.view(np.int8)
+    w = rng.integers(-128, 128, ws).astype(np.int8)
+    st, zp = [1] * (len(xs) - 2), 77 if u8 else 0
+    got = conv_call(x, w, st, pd, zpx=zp, ws_shift=ws_shift, w_shift=w_shift)
+    same_bits(got, oracle.quantized_conv(x, w, st, pd, [1] * len(st), 1, zp, 0))
