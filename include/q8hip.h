@@ -290,6 +290,12 @@ int q8_gemm_glu(const int8_t* A, const int8_t* B, int64_t M, int64_t F, int64_t 
  * path); it makes the slow route visible to callers and tests. */
 int q8_generic_gemm_launches(int64_t* count);
 
+/* For tests and diagnosis, no counterpart in the reference: the matrix
+ * kernel the calling thread launched last ("qgemm 128x128", "ring 64x64 k2",
+ * "any 64x64 k4", "gemv dot4", ...: kernel, tile, groups a tile's K is split
+ * over), copied into buf (cap bytes, NUL-terminated). */
+int q8_debug_last_gemm(char* buf, size_t cap);
+
 /* quantized_dot as the reference defines it (src/compiler/ir/graph/ops/
  * quantization.ts:103-155, lowering rules/quantization.ts:23-42): operands
  * i8 or ui8 (Q8_I8 / Q8_U8: Int8Array or Uint8Array elements, the

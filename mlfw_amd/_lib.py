@@ -79,6 +79,7 @@ SIGNATURES = {
     "q8_gemv": [_vp, _vp, _i64, _i64, _i64, _vp, _int, _vp, _int, _int, _dbl, _vp, _int,
                 _int, _vp, _vp],
     "q8_generic_gemm_launches": [_vp],
+    "q8_debug_last_gemm": [_vp, C.c_size_t],
     "q8_glu_interleave": [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _vp, _vp, _vp, _vp],
     "q8_gemm_glu_workspace": [_i64, _i64, _i64, _vp],
     "q8_gemm_glu": [_vp, _vp, _i64, _i64, _i64, _vp, _int, _vp, _int, _vp, _vp, _vp, C.c_size_t, _vp],

@@ -528,6 +528,15 @@ int q8_generic_gemm_launches(int64_t* count) {
   return Q8_OK;
 }
 
+int q8_debug_last_gemm(char* buf, size_t cap) {
+  Q8_REQUIRE(buf != nullptr && cap > 0, "q8_debug_last_gemm: no buffer");
+  const q8::GemmRoute& r = q8::g_route;
+  if (r.bm == 0) snprintf(buf, cap, "%s", r.kernel);
+  else if (r.kg == 0) snprintf(buf, cap, "%s %dx%d", r.kernel, r.bm, r.bn);
+  else snprintf(buf, cap, "%s %dx%d k%d", r.kernel, r.bm, r.bn, r.kg);
+  return Q8_OK;
+}
+
 int q8_gemv(const int8_t* A, const int8_t* B, int64_t M, int64_t N, int64_t K, const double* sA,
             int sA_mode, const double* sB, int sB_mode, int epi, double s_out, const float* bias,
             int act, int out_kind, void* out, void* stream) {

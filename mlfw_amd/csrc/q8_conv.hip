@@ -682,6 +682,7 @@ hipError_t launch_conv(const int8_t* x, const int8_t* w, const int8_t* w_taps, c
   if (G.N * G.O * G.Pn == 0) return hipSuccess;
   if (p.route == ConvPlan::DIRECT) {
     const int64_t total = G.N * G.O * G.Pn;
+    note_route("conv direct");
     hipLaunchKernelGGL(k_conv_direct, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, x,
                        w, G, e, out);
     return hipGetLastError();

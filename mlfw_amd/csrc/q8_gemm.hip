@@ -1082,6 +1082,7 @@ static hipError_t launch_qgemm_tile(const int8_t* A, const int8_t* B, int M, int
   const int tm = (M + BM - 1) / BM, tn = (N + BN - 1) / BN;
   const dim3 grid((unsigned)(tm * tn)), block(GEMM_THREADS);
   constexpr int lds = qgemm_lds<BM, BN>();
+  note_route("qgemm", BM, BN);
 #define Q8_LAUNCH_EPI(code)                                                                  \
   case code:                                                                                 \
     hipLaunchKernelGGL((k_qgemm<BM, BN, code>), grid, block, lds, st, A, B, M, N, K, tm, tn, \
@@ -1110,6 +1111,7 @@ static hipError_t launch_qgemm_tile(const int8_t* A, const int8_t* B, int M, int
 #define Q8_EPI_CODES_CONV(X) X(384) X(400)
 
 std::atomic<long long> g_generic_gemm_launches{0};
+thread_local GemmRoute g_route;
 
 // Tile choice by a fill-aware cost of the launch's rounds.  A tile shape
 // has `slots` workgroups resident at once (CUs x the workgroups per CU its
@@ -1164,6 +1166,7 @@ hipError_t launch_gemm_conv(const int8_t* A, const int8_t* frame, int64_t M, int
   const int tm = (int)((M + bm - 1) / bm), tn = (int)((N + bm - 1) / bm);
   if ((int64_t)tm * tn >= ((int64_t)1 << 31) / GEMM_THREADS) return hipErrorInvalidValue;
   const dim3 grid((unsigned)(tm * tn)), block(GEMM_THREADS);
+  note_route("conv", bm, bm);
   const int code = epi_code(e) | 256;
   hipError_t err = hipErrorInvalidValue;
   constexpr int lds128 = qgemm_lds<128, 128>(), lds64 = qgemm_lds<64, 64>();
@@ -1878,6 +1881,7 @@ template <int MT>
 static hipError_t launch_gemv_mt(const int8_t* A, const int8_t* B, int M, int N, int K,
                                  const GemmEpi& e, void* out, hipStream_t st) {
   const dim3 grid((unsigned)((N + GV_ROWS - 1) / GV_ROWS)), block(256);
+  note_route("gemv dot4");
   const int cpt = (K / 16 + 255) / 256;               // <= 5 (K <= 20480)
   if (cpt <= 1)
     hipLaunchKernelGGL((k_gemv_i8<MT, 1>), grid, block, 0, st, A, B, M, N, K, e, out);
@@ -1902,6 +1906,7 @@ static hipError_t launch_gemv_mfma(const int8_t* A, const int8_t* B, int M, int 
   // M = 8: 12.2 -> 11.6 us; N = 14336: 16.1 -> 14.6 us.
   const int nblk = (N + 15) / 16;
   const int cus = cu_count() > 0 ? cu_count() : 256;
+  note_route("gemv mfma");
   if (K >= 4096) {
     hipLaunchKernelGGL((k_gemv_mfma<4, 16>), dim3((unsigned)(nblk < cus ? nblk : cus)), dim3(1024), 0, st,
                        A, B, M, N, K, e, out);

@@ -445,6 +445,7 @@ hipError_t launch_any_tile(const int8_t* A, const int8_t* B, int M, int N, int K
   const int tm = (M + BM - 1) / BM, tn = (N + BN - 1) / BN;
   const dim3 grid((unsigned)(tm * tn), (unsigned)p.groups), block(256 * KG);
   const unsigned lds = AnyCfg<BM, BN, KG>::LDS + (p.conv_cg ? (unsigned)K / 4 : 0u);
+  note_route(p.conv_cg ? "any conv" : "any", BM, BN, KG);
   const AffineDot zz = z ? *z : AffineDot{};
   Q8_ANY_LAUNCH(k_qgemm_any, BM, BN, KG, );
   return hipGetLastError();
@@ -455,6 +456,7 @@ hipError_t launch_wk(const int8_t* A, const int8_t* B, int M, int N, int K, cons
   const int tm = (M + WKB - 1) / WKB, tn = (N + WKB - 1) / WKB;
   const dim3 grid((unsigned)(tm * tn), (unsigned)p.groups), block(64 * WKW);
   const unsigned lds = WK_LDS + (p.conv_cg ? (unsigned)K / 4 : 0u);
+  note_route(p.conv_cg ? "any conv" : "any", WKB, WKB, WKW);
   const AffineDot zz = z ? *z : AffineDot{};
   Q8_ANY_LAUNCH(k_qgemm_wk, );
   return hipGetLastError();
@@ -474,6 +476,7 @@ hipError_t launch_gemm_any(const int8_t* A, const int8_t* B, int64_t M, int64_t 
   const int m = (int)M, n = (int)N, k = (int)K;
   // (355 x 10 x 33, the last layer of a small MLP: 2 us less than a tile)
   if (!z && !p.conv_cg && p.groups == 1 && p.lda == K && p.ldb == K && K < 64 && M * N <= (1 << 16)) {
+    note_route("tiny");
     hipLaunchKernelGGL(k_qgemm_tiny, dim3((unsigned)((M * N + 255) / 256)), dim3(256), 0, st, A, B, m, n, k, e, out);
     return hipGetLastError();
   }

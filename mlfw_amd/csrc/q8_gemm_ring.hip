@@ -144,6 +144,7 @@ template <int BM, int BN, int GM, int GN, int KG, int NB>
 hipError_t launch_ring_tile(const int8_t* A, const int8_t* B, int M, int N, int K, const GemmEpi& e, void* out,
                             hipStream_t st) {
   const int tm = (M + BM - 1) / BM, tn = (N + BN - 1) / BN;
+  note_route("ring", BM, BN, KG);
   hipLaunchKernelGGL((k_qgemm_ring<BM, BN, GM, GN, KG, NB>), dim3((unsigned)(tm * tn)), dim3(64 * GM * GN * KG),
                      (unsigned)(RingCfg<BM, BN, GM, GN, KG, NB>::LDS), st, A, B, M, N, K, tm, tn, e, out);
   return hipGetLastError();
@@ -160,23 +161,31 @@ hipError_t launch_ring_tile(const int8_t* A, const int8_t* B, int M, int N, int 
   X(64, 128, 2, 2, 2, 3)   \
   X(128, 128, 2, 2, 1, 4)
 
-// The smallest tile that leaves every tile a CU of its own, -1 where none
-// does: a second round costs a workgroup's whole time again, while more and
-// smaller tiles spread the weights' load over more CUs.  (us, best of the tiles
-// against k_qgemm: 64 x 4096 x 4096 32 x 32 9.4 / 26.5; 17 x 11008 x 4096 32 x
-// 64 13.2 / 28.2; 128 x 4096 x 4096 64 x 32 10.7 / 26.1; 256 x 4096 x 11008 64 x
-// 64 30.8 / 65.1; 128 x 11008 x 4096 128 x 64 21.6 / 30.0; 64 x 22016 x 4096 64 x
-// 128 26.3 / 35.2; 1024 x 4096 x 4096 128 x 128 31.3 / 33.4; with 1.3 rounds, 384
-// x 11008 x 4096, 128 x 128 56.1 / 37.5.)  The larger tiles' fill does not pay
-// over less than eight stages (512 x 2048 x 512: 64 x 64 5.55 / 5.37).
+// The smallest tile that leaves every tile a CU of its own (a second round
+// costs a workgroup's whole time again, while more and smaller tiles spread
+// the weights' load over more CUs), -1 where none does, and from the tile's
+// `stages` on: filling the ring and adding up the groups cost the same however
+// short K is, and the larger the tile the more MFMAs k_qgemm hides its copies
+// behind.  Time against k_qgemm with the weights in the MALL / in HBM, median
+// over 1 to 51 products of M 17..2048, N 64..32000 at K = 128 x stages:
+//   32 x 32     3: 1.00 / 1.01    4: 0.92 / 0.91    8: 0.72 / 0.72   32: 0.36 / 0.35
+//   64 x 32     4: 0.95 / 0.95    6: 0.89 / 0.88    8: 0.78 / 0.77   32: 0.47 / 0.40
+//   32 x 64     3: 0.99 / 0.97    4: 0.90 / 0.90    8: 0.79 / 0.68   32: 0.54 / 0.46
+//   64 x 64     6: 0.99 / 0.98    8: 0.93 / 0.92   16: 0.76 / 0.67   32: 0.64 / 0.52
+//   128 x 64   12: 1.04 / 0.92   16: 0.98 / 0.80   20: 0.92 / 0.83   32: 0.85 / 0.66
+//   64 x 128   12: 1.03 / 0.89   16: 0.98 / 0.87   20: 0.97 / 0.86   32: 0.77 / 0.78
+//   128 x 128  16: 1.38 / 1.14   32: 1.16 / 0.92   48: 1.03 / 0.86   86: 0.89 / 0.78
+// (64 x 32 waits for 6: weights still in L2 take 1.07 at 4.)  One row of 128 x
+// 128 tiles, 90 MB of weights and more, is bound by their load sooner: 128 x
+// 32000, 32 stages, 0.86 / 0.83.
 int gemm_ring_tile(int64_t M, int64_t N, int64_t K) {
-  static const struct { int bm, bn; } tiles[] = {{32, 32}, {64, 32}, {32, 64}, {64, 64}, {128, 64}, {64, 128}, {128, 128}};
+  static const struct { int bm, bn, stages; } tiles[] = {{32, 32, 4},   {64, 32, 6},    {32, 64, 4},  {64, 64, 8},
+                                                         {128, 64, 20}, {64, 128, 16}, {128, 128, 48}};
   const int64_t cus = cu_count() > 0 ? cu_count() : 256, KT = (K + AK - 1) / AK;
-  if (KT < 2) return -1;
   for (int t = 0; t < 7; ++t) {
-    if (t >= 3 && KT < 8) break;
-    if ((tiles[t].bm == 32 && t == 2 && M > 32) || (t == 4 && M <= 64)) continue;   // rows of padding
-    if (((M + tiles[t].bm - 1) / tiles[t].bm) * ((N + tiles[t].bn - 1) / tiles[t].bn) <= cus) return t;
+    if ((t == 2 && M > 32) || (t == 4 && M <= 64)) continue;   // rows of padding
+    if (((M + tiles[t].bm - 1) / tiles[t].bm) * ((N + tiles[t].bn - 1) / tiles[t].bn) > cus) continue;
+    return KT >= (t == 6 && M <= 128 ? 32 : tiles[t].stages) ? t : -1;
   }
   return -1;
 }

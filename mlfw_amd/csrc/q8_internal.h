@@ -111,6 +111,15 @@ extern std::atomic<long long> g_ewise_jit_compiled, g_ewise_jit_launches;
 // Copies why the last failed ewise compile failed into buf (truncated,
 // NUL-terminated; "" if none has) and returns the message's full length.
 size_t ewise_jit_error(char* buf, size_t cap);
+// The matrix kernel this thread launched last, its tile and its K groups (0:
+// none): what q8_debug_last_gemm reports.
+struct GemmRoute {
+  const char* kernel = "";
+  int bm = 0, bn = 0, kg = 0;
+};
+extern thread_local GemmRoute g_route;
+inline void note_route(const char* kernel, int bm = 0, int bn = 0, int kg = 0) { g_route = {kernel, bm, bn, kg}; }
+
 // The GEMM for any K and alignment (q8_gemm_any.hip); with `z` the affine
 // form: operand bytes flipped by xa / xb (0, or 0x80808080 for a ui8
 // operand), the int32 result corrected by cB * rowsum(A) + cA * rowsum(B) +

@@ -752,6 +752,7 @@ hipError_t launch_gemv_w4(const int8_t* xq, const double* sx, int sx_stride, con
   if (M == 0 || N == 0) return hipSuccess;
   if (gemm_w4_ok(xq, wq4, M, N, K, group))
     return launch_gemm_w4(xq, sx, sx_stride, wq4, sw, M, N, K, group, bias, act, y, st);
+  note_route("w4 gemv");
   W4Plan pl;
   const bool dot4 = w4_plan(M, K, group, &pl);
   W4MPlan mp;

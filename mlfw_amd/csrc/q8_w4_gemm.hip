@@ -265,6 +265,7 @@ hipError_t launch_tile(const int8_t* xq, const double* sx, int sx_stride, const 
                        int N, int K, int group, const float* bias, int act, float* y, hipStream_t st) {
   const int tm = (M + BM - 1) / BM, tn = (N + BN - 1) / BN, G = K / group;
   const dim3 grid((unsigned)(tm * tn)), block(256);
+  note_route("w4", BM, BN);
 #define Q8_W4G(GPS, spg)                                                                                            \
   hipLaunchKernelGGL((k_gemm_w4<BM, BN, GPS>), grid, block, 0, st, xq, sx, sx_stride, wq4, sw, M, N, K, spg, G, tm, \
                      tn, bias, act, y)

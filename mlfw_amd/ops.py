@@ -448,6 +448,14 @@ def generic_gemm_launches() -> int:
     return n.value
 
 
+def last_gemm() -> str:
+    """The matrix kernel this thread launched last, its tile and its K groups
+    ("ring 64x64 k2"): for tests and diagnosis."""
+    buf = C.create_string_buffer(64)
+    L.call("q8_debug_last_gemm", buf, len(buf))
+    return buf.value.decode()
+
+
 def requant_dynamic_workspace(M: int, N: int, K: int):
     """(bytes, fused) of q8_gemm_requant_dynamic for this shape."""
     nb, fused = C.c_size_t(0), C.c_int(0)

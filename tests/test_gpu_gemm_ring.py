@@ -81,3 +81,35 @@ def test_ring_under_capture(ops, oracle):
         graph.replay()
         np.testing.assert_array_equal(host(out), acc)
         np.testing.assert_array_equal(host(ops.quantized_dot(dA, dB)), acc)
+
+
+# Either side of each tile's least number of 128-byte stages (256 CUs), K
+# ending inside the last one
+ROUTES = [(256, 1024, 384, "qgemm"), (48, 1000, 400, "ring 32x32 k4"),
+          (96, 4090, 640, "qgemm"), (96, 4090, 656, "ring 64x32 k4"),
+          (20, 11000, 384, "qgemm"), (20, 11001, 400, "ring 32x64 k4"),
+          (64, 11008, 896, "qgemm"), (61, 11008, 1008, "ring 64x64 k2"),
+          (130, 5500, 2416, "qgemm"), (130, 5501, 2448, "ring 128x64 k2"),
+          (64, 16500, 1920, "qgemm"), (63, 16500, 2000, "ring 64x128 k2"),
+          (512, 4200, 6000, "qgemm"), (511, 4201, 6032, "ring 128x128 k1"),
+          (100, 16500, 3968, "qgemm"), (100, 16499, 4000, "ring 128x128 k1"), (1024, 4096, 4096, "qgemm")]
+
+
+@pytest.mark.parametrize("M,N,K,route", ROUTES)
+def test_ring_from_its_first_stages_on(ops, oracle, M, N, K, route):
+    rng = np.random.default_rng(M + N + K)
+    A = rng.integers(-128, 128, (M, K)).astype(np.int8)
+    B = rng.integers(-128, 128, (N, K)).astype(np.int8)
+    sA, sB = rng.uniform(1e-3, 0.05, M), rng.uniform(1e-4, 0.02, N)
+    bias = rng.uniform(-1, 1, N).astype(np.float32)
+    print(f"ring route M={M} N={N} K={K}", flush=True)
+    acc = (A.astype(np.float64) @ B.T.astype(np.float64)).astype(np.int32)   # exact: sums below 2^53
+    dA, dB, da, db, dbias = dev(A), dev(B), dev(sA), dev(sB), dev(bias)
+    np.testing.assert_array_equal(host(ops.quantized_dot(dA, dB)), acc)
+    assert ops.last_gemm().startswith(route)
+    y = oracle.epilogue(acc, "rowcol", sA, sB, bias=bias, act="relu")
+    got = host(ops.qlinear(dA, da, dB, db, bias=dbias, act="relu"))
+    np.testing.assert_array_equal(got.view(np.uint32), y.view(np.uint32))
+    s_next = float(np.abs(y).max() / 127.0)
+    q = host(ops.qlinear_requant(dA, da, dB, db, s_next, bias=dbias, act="relu"))
+    np.testing.assert_array_equal(q, oracle.quantize(y.reshape(-1), s_next).reshape(M, N))
