@@ -415,17 +415,48 @@ void k_qgemm_wk(const int8_t* __restrict__ A, const int8_t* __restrict__ B, int 
   }
 }
 
-// One thread per output with byte loads: products of a few thousand outputs
-// over a short row are a launch and one load latency either way, and this
-// kernel's few instructions arrive sooner than the tiled kernel's.
+// One thread per output with byte loads: short rows are a launch and a few
+// load latencies either way, and this kernel's few instructions arrive sooner
+// than the tiled kernel's (any_tiny has the line).  Affine operands term by
+// term: (a' + cA)(b' + cB) summed over k is the corrected sum.
+template <bool ZP>
 __global__ __launch_bounds__(256) void k_qgemm_tiny(const int8_t* __restrict__ A, const int8_t* __restrict__ B, int M,
-                                                    int N, int K, GemmEpi e, void* __restrict__ out) {
+                                                    int N, int K, GemmEpi e, AffineDot z, void* __restrict__ out) {
   const int64_t idx = blockIdx.x * 256LL + threadIdx.x;
   if (idx >= (int64_t)M * N) return;
   const int64_t m = idx / N, n = idx % N;
   uint32_t s = 0;
-  for (int k = 0; k < K; ++k) s += (uint32_t)((int)A[m * K + k] * (int)B[n * K + k]);
+  for (int k = 0; k < K; ++k) {
+    if constexpr (ZP) {
+      const int a = (int8_t)(A[m * K + k] ^ (int8_t)z.xa), b = (int8_t)(B[n * K + k] ^ (int8_t)z.xb);
+      s += ((uint32_t)a + (uint32_t)z.cA) * ((uint32_t)b + (uint32_t)z.cB);
+    } else {
+      s += (uint32_t)((int)A[m * K + k] * (int)B[n * K + k]);
+    }
+  }
   store_out(out, idx, (int)s, m, n, e);
+}
+
+// Whether one thread per output serves an M x N product over rows of K bytes
+// sooner than tiles.  A thread's chain is about 0.15 us a byte, the launch
+// 1.2e6 multiply-adds (0.75e6 over longer rows) and 4.2e5 outputs a us; a tile
+// is worth 5 ns where it is full, 3.5 with few rows and 6.6 with few columns (a
+// lane's loads and stores then go one row each), and rows shorter than 16
+// bytes are loaded byte by byte.  us, thread per output / tiles: 500000 x 3 x 3 8.9 / 64.8, 100000 x 1 x
+// 33 8.2 / 17.1, 60000 x 10 x 15 12.9 / 20.0 and x 17 14.1 / 11.3, 300 x 300 x
+// 15 5.6 / 13.4, 64 x 8192 x 15 9.7 / 13.4 and x 17 10.5 / 7.5, 4096 x 4096 x
+// 3 59 / 33.  Up to 2^16 outputs a symmetric product over rows of less
+// than 64 bytes stays here throughout (355 x 10 x 33, the last layer of a
+// small MLP: 2 us less than a tile).
+bool any_tiny(int64_t M, int64_t N, int64_t K, int64_t t64, bool affine) {
+  const double mn = (double)M * (double)N, k = (double)K, t = (double)t64;
+  if (mn <= 65536.0 && K < 64 && !affine) return true;
+  if (K > 256 || mn >= 0x1p31) return false;
+  const double chain = 3.0 + 0.15 * k, rate = mn * k / (K < 16 ? 1.2e6 : 0.75e6);
+  const double thread = (chain > 5.5 ? chain : 5.5) > rate ? (chain > 5.5 ? chain : 5.5) : rate;
+  const double tiles = K < 16 ? 7.0 + 0.4 * k + t * (0.0066 + 0.0006 * k)
+                              : 5.6 + t * (N < 64 ? 0.0066 : M < 64 ? 0.0035 : 0.0052);
+  return thread + mn / 4.2e5 < tiles;
 }
 
 #define Q8_ANY_LAUNCH(KERN, ...)                                                                                   \
@@ -474,10 +505,11 @@ hipError_t launch_gemm_any(const int8_t* A, const int8_t* B, int64_t M, int64_t 
   const int64_t t64 = p.groups * ((M + 63) / 64) * ((N + 63) / 64);
   if (t64 > INT32_MAX || p.groups > 65535) return hipErrorInvalidValue;
   const int m = (int)M, n = (int)N, k = (int)K;
-  // (355 x 10 x 33, the last layer of a small MLP: 2 us less than a tile)
-  if (!z && !p.conv_cg && p.groups == 1 && p.lda == K && p.ldb == K && K < 64 && M * N <= (1 << 16)) {
+  if (!p.conv_cg && p.groups == 1 && p.lda == K && p.ldb == K && any_tiny(M, N, K, t64, z != nullptr)) {
     note_route("tiny");
-    hipLaunchKernelGGL(k_qgemm_tiny, dim3((unsigned)((M * N + 255) / 256)), dim3(256), 0, st, A, B, m, n, k, e, out);
+    const dim3 grid((unsigned)((M * N + 255) / 256));
+    if (z) hipLaunchKernelGGL(k_qgemm_tiny<true>, grid, dim3(256), 0, st, A, B, m, n, k, e, *z, out);
+    else hipLaunchKernelGGL(k_qgemm_tiny<false>, grid, dim3(256), 0, st, A, B, m, n, k, e, AffineDot{}, out);
     return hipGetLastError();
   }
   // Up to one 64 x 64 tile per CU: four K groups each (512 x 7 x 7 conv, 200

@@ -93,3 +93,32 @@ def test_int8_output(ops, oracle, M, N, K):
     got = host(ops.qlinear_requant(dev(A), torch.from_numpy(sA).to(DEV), dev(B), torch.from_numpy(sB).to(DEV),
                                    s_next, act="relu"))
     np.testing.assert_array_equal(got, oracle.quantize(y.reshape(-1), s_next).reshape(M, N))
+
+
+# Short rows over many outputs, on either side of the line between one thread
+# per output and tiles: skinny and square, below and above a 16-byte chunk
+SHORT_ROWS = [(300, 300, 1, "tiny"), (300, 301, 15, "tiny"), (500, 400, 17, "any"), (20000, 10, 15, "tiny"),
+              (60000, 10, 17, "any"), (20000, 10, 17, "tiny"), (1, 90000, 33, "tiny"), (90000, 1, 33, "tiny"), (16, 9000, 3, "tiny"),
+              (64, 8192, 15, "tiny"), (64, 8192, 17, "any"), (50000, 3, 3, "tiny"), (2048, 2047, 3, "any"),
+              (5, 7, 9, "tiny")]
+
+
+@pytest.mark.parametrize("M,N,K,route", SHORT_ROWS)
+def test_short_rows(ops, oracle, M, N, K, route):
+    rng = np.random.default_rng(M + N + K)
+    A = rng.integers(0, 256, (M, K)).astype(np.uint8)
+    B = rng.integers(0, 256, (N, K)).astype(np.uint8)
+    print(f"short rows M={M} N={N} K={K}", flush=True)
+    i8 = A.view(np.int8), B.view(np.int8)
+    acc = oracle.quantized_dot(*i8, 1)
+    np.testing.assert_array_equal(host(ops.quantized_dot(dev(i8[0]), dev(i8[1]))), acc)
+    assert ops.last_gemm().startswith(route)
+    sA, sB = rng.uniform(1e-3, 0.05, M), rng.uniform(1e-4, 0.02, N)
+    bias = rng.uniform(-1, 1, N).astype(np.float32)
+    want = oracle.epilogue(acc, "rowcol", sA, sB, bias=bias, act="relu")
+    d = [torch.from_numpy(v).to(DEV) for v in (sA, sB, bias)]
+    got = host(ops.qlinear(dev(i8[0]), d[0], dev(i8[1]), d[1], bias=d[2], act="relu"))
+    np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
+    for a, b, za, zb in ((A, i8[1], 121, 0), (i8[0], B, -3, 128), (A, B, 7, 250), (i8[0], i8[1], 0, 5)):
+        np.testing.assert_array_equal(host(ops.quantized_dot(dev(a), dev(b), za, zb)),
+                                      oracle.quantized_dot(a, b, 1, za, zb))
