@@ -451,7 +451,7 @@ __global__ __launch_bounds__(256) void k_qgemm_tiny(const int8_t* __restrict__ A
 bool any_tiny(int64_t M, int64_t N, int64_t K, int64_t t64, bool affine) {
   const double mn = (double)M * (double)N, k = (double)K, t = (double)t64;
   if (mn <= 65536.0 && K < 64 && !affine) return true;
-  if (K > 256 || mn >= 0x1p31) return false;
+  if (K > 256 || mn >= 0x1p32 - 256) return false;
   const double chain = 3.0 + 0.15 * k, rate = mn * k / (K < 16 ? 1.2e6 : 0.75e6);
   const double thread = (chain > 5.5 ? chain : 5.5) > rate ? (chain > 5.5 ? chain : 5.5) : rate;
   const double tiles = K < 16 ? 7.0 + 0.4 * k + t * (0.0066 + 0.0006 * k)
@@ -503,9 +503,14 @@ hipError_t launch_gemm_any(const int8_t* A, const int8_t* B, int64_t M, int64_t 
   const int64_t cus = cu_count() > 0 ? cu_count() : 256;
   const int64_t t128 = p.groups * ((M + 127) / 128) * ((N + 127) / 128);
   const int64_t t64 = p.groups * ((M + 63) / 64) * ((N + 63) / 64);
-  if (t64 > INT32_MAX || p.groups > 65535) return hipErrorInvalidValue;
+  // a launch has fewer than 2^32 threads: 2^24 - 1 tiles of 256, or as many
+  // outputs of a thread each (one row by 2^30 columns); and the tiles count K
+  // in 31 bits, stages past its end included
+  const bool plain = !p.conv_cg && p.groups == 1 && p.lda == K && p.ldb == K;
+  const bool wide = t64 >= ((int64_t)1 << 24) || K > INT32_MAX - 4096;
+  if (p.groups > 65535 || (wide && !(plain && (double)M * (double)N < 0x1p32 - 256))) return hipErrorInvalidValue;
   const int m = (int)M, n = (int)N, k = (int)K;
-  if (!p.conv_cg && p.groups == 1 && p.lda == K && p.ldb == K && any_tiny(M, N, K, t64, z != nullptr)) {
+  if (plain && (wide || any_tiny(M, N, K, t64, z != nullptr))) {
     note_route("tiny");
     const dim3 grid((unsigned)((M * N + 255) / 256));
     if (z) hipLaunchKernelGGL(k_qgemm_tiny<true>, grid, dim3(256), 0, st, A, B, m, n, k, e, *z, out);

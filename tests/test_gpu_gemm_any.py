@@ -122,3 +122,17 @@ def test_short_rows(ops, oracle, M, N, K, route):
     for a, b, za, zb in ((A, i8[1], 121, 0), (i8[0], B, -3, 128), (A, B, 7, 250), (i8[0], i8[1], 0, 5)):
         np.testing.assert_array_equal(host(ops.quantized_dot(dev(a), dev(b), za, zb)),
                                       oracle.quantized_dot(a, b, 1, za, zb))
+
+
+def test_more_tiles_than_a_launch_holds(ops):
+    """One row by 2^30 columns and more: tiles of 64 columns would be 2^24
+    workgroups of 256 threads, a thread per output still fits a launch."""
+    N = (1 << 30) + 1000
+    g = torch.Generator(device=DEV).manual_seed(1)
+    B = torch.randint(-128, 128, (N, 1), device=DEV, generator=g, dtype=torch.int8)
+    A = torch.full((1, 1), -77, dtype=torch.int8, device=DEV)
+    print(f"one row by {N} columns", flush=True)
+    out = ops.quantized_dot(A, B)
+    assert ops.last_gemm() == "tiny"
+    for i in range(0, N, 1 << 28):                      # exact int32 products, a slice at a time
+        assert torch.equal(out[0, i:i + (1 << 28)], B[i:i + (1 << 28), 0].to(torch.int32) * -77)
