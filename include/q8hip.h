@@ -303,10 +303,10 @@ int q8_debug_last_gemm(char* buf, size_t cap);
  *   out[m,n] = ToInt32( sum_k (A[m,k] - zpA) * (B[n,k] - zpB) )
  * with B in the [N,K] layout (rhs_contracting = [1]).  The reference's
  * QuantizationPass sets non-zero zero points for affine schemes
- * (quantization_pass.ts:303-332, :415-425).  Runs the int8 GEMM on
+ * (quantization_pass.ts:303-332, :415-425).  Runs the int8 GEMM / GEMV on
  * operands made signed (ui8 bytes flipped by 128) and adds the exact
- * zero-point correction from row sums, in one launch, or for very large
- * products as separate passes in the device workspace of
+ * zero-point correction from row sums, in one launch, or where the aligned
+ * kernels' lead pays for it as separate passes in the device workspace of
  * q8_quantized_dot_workspace bytes that the caller passes (0 for i8 operands
  * with zero zero points, where this is q8_gemm with Q8_I32 output). */
 int q8_quantized_dot_workspace(int64_t M, int64_t N, int64_t K, int a_dtype, int b_dtype,

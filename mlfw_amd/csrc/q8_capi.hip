@@ -576,6 +576,49 @@ QdotPlan qdot_plan(int64_t M, int64_t N, int64_t K, int a_dtype, int b_dtype, in
   p.bytes = off;
   return p;
 }
+
+// Whether an affine product with aligned operands takes the direct-to-LDS
+// GEMM or the GEMV between passes of its own (flips, row sums, correction)
+// instead of the one launch that does all of it on the way through registers:
+// where the lead of those kernels, in us, exceeds what the passes cost.  A
+// pass over a bytes costs 2 us and a / 3.5e6 (reading and writing counted
+// apart, the correction on 8 bytes an output).
+//   More than 16 tokens, from 2^21 outputs on: the one launch runs about 5e-7
+// us an output and 5.5e-10 us a multiply-add behind.  ui8 A with zero point 128
+// (one flip): 2048 x 11008 x 4096 110 us in passes, 158 in one launch, 1024 x
+// 4096 x 1024 13.8 and 13.5; row sums and correction: 1024 x 11008 x 11008
+// 170 and 214, 4096 x 4096 x 4096 109 and 108, 2048 x 4096 x 4096 65 and 56.
+//   Up to 16 tokens the GEMV reads B once at about 6 TB/s; the one launch's 32
+// x 32 tiles (8192 columns and fewer) are a chain over K, its 64 x 64 ones
+// read 3.9 TB/s.  One flip of A, 4 x 4096 x 11008: 13.0 us in passes, 20.1 in
+// one launch; 4 x 256 x 256 4.2 and 3.0.  Row sums of B are a second read of
+// it: 4 x 4096 x 11008 27.1 and 20.1.  A call made by itself keeps the host
+// busy for 13 us and 2.7 more for each pass, so a product below that stays
+// with the one launch (4 x 1024 x 4096, one flip: replayed from a graph 4.9 us
+// in passes and 7.8 in one launch, called one by one 15.4 and 12.7).
+bool qdot_passes(const QdotPlan& p, int64_t M, int64_t N, int64_t K) {
+  const double m = (double)M, n = (double)N, k = (double)K, mn = m * n;
+  double lead, rate = 3.5e6, flip = 2.0, sums = 2.0;
+  if (M > 16) {
+    if (mn < 0x1p21) return false;
+    lead = 5e-7 * mn + 5.5e-10 * mn * k;
+  } else {
+    const double chain = N <= 8192 ? k * (1.2e-3 + 4e-5 * m) + 8e-8 * n * k : 0.0, read = n * k / 3.9e6;
+    const double one = 2.7 + (chain > read ? chain : read);
+    if (one < 13.0) return false;
+    lead = one - 2.2 - n * k / 6e6 - (M > 4 ? 5.5e-4 * k : 0.0);
+    rate = 4e6;
+    flip = 1.6;
+    sums = 2.2;
+  }
+  double cost = 0.0;
+  if (p.a_u8) cost += flip + 2.0 * m * k / rate;
+  if (p.b_u8) cost += flip + 2.0 * n * k / rate;
+  if (p.need_rs) cost += sums + m * k / rate;
+  if (p.need_cs) cost += sums + n * k / rate;
+  if (p.need_rs || p.need_cs) cost += sums + 8.0 * mn / rate;
+  return lead > cost;
+}
 }  // namespace
 
 int q8_quantized_dot_workspace(int64_t M, int64_t N, int64_t K, int a_dtype, int b_dtype,
@@ -608,14 +651,9 @@ int q8_quantized_dot(const void* A, int a_dtype, const void* B, int b_dtype, int
   if (M * N == 0) return Q8_OK;
   hipStream_t st = as_stream(stream);
   // Zero points and ui8 operands: one launch that flips, sums and corrects
-  // on the way through registers (788 x 1000 x 1500: 4350 -> 16.5 us; 256 x
-  // 4096 x 4096, which the tiled GEMM takes too: 34.2 -> 16.8).  Only very
-  // large aligned products gain more from the direct-to-LDS GEMM than its
-  // separate passes over the operands and the result cost: from 2^37
-  // multiply-adds (4096 x 4096 x 11008 takes 267 us here and 222 us in
-  // passes, 2048 x 11008 x 4096 158 and 178).
+  // on the way through registers, or passes around the symmetric kernels.
   const bool aligned = K % 16 == 0 && ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B)) & 15) == 0;
-  const bool passes = aligned && M > 16 && (double)M * (double)N * (double)K >= 0x1p37;
+  const bool passes = aligned && qdot_passes(p, M, N, K);
   if ((p.a_u8 || p.b_u8 || p.cA != 0 || p.cB != 0) && !passes) {
     if (!aligned) q8::g_generic_gemm_launches.fetch_add(1, std::memory_order_relaxed);
     const int flip = (int)0x80808080u;

@@ -10,8 +10,8 @@
 // where sum a'b' is the int8 GEMM of the flipped operands and the rest is a
 // rank-1 correction from row sums -- all exact modulo 2^32, which is the
 // ToInt32 of the exact sum.  The general GEMM (q8_gemm_any.hip) evaluates this
-// identity in one launch; the passes below serve only products so large that
-// the direct-to-LDS GEMM's lead pays for them (q8_quantized_dot has the line).
+// identity in one launch; the passes below serve where the lead of the
+// direct-to-LDS GEMM or the GEMV pays for them (qdot_passes has the line).
 #include "q8_device.h"
 #include "q8_internal.h"
 

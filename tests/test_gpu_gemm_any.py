@@ -136,3 +136,30 @@ def test_more_tiles_than_a_launch_holds(ops):
     assert ops.last_gemm() == "tiny"
     for i in range(0, N, 1 << 28):                      # exact int32 products, a slice at a time
         assert torch.equal(out[0, i:i + (1 << 28)], B[i:i + (1 << 28), 0].to(torch.int32) * -77)
+
+
+# Affine products with aligned operands on either side of the line between one
+# launch and passes around the symmetric kernels: flips, row sums of A and B,
+# the correction; a few tokens (GEMV) and many (GEMM)
+AFFINE_ROUTES = [(4, 256, 256, "A", "any"), (4, 256, 4096, "A", "any"), (1, 4096, 11008, "A", "gemv"),
+                 (16, 1024, 11008, "A", "gemv"), (4, 4096, 4096, "csB", "any"), (1, 1024, 11008, "B", "gemv"),
+                 (1, 32000, 4096, "rsA", "gemv"), (1, 1024, 11008, "csB", "gemv"), (8, 1024, 1024, "all", "any"),
+                 (17, 4096, 4096, "A", "any"), (512, 4096, 4096, "A", ("qgemm", "ring")), (512, 4096, 4096, "rsA", "any"),
+                 (2048, 1024, 1024, "A", "any"), (2048, 4096, 1024, "A", ("qgemm", "ring")),
+                 (1024, 4000, 16384, "csB", ("qgemm", "ring")),
+                 (1024, 4000, 8192, "all", "any"), (256, 8200, 4096, "B", "any")]
+AFFINE_KINDS = {"A": (1, 0, 128, 0), "B": (0, 1, 0, 128), "rsA": (0, 0, 0, 3), "csB": (0, 0, 3, 0), "all": (1, 1, 121, 7)}
+
+
+@pytest.mark.parametrize("M,N,K,kind,route", AFFINE_ROUTES)
+def test_affine_routes(ops, oracle, M, N, K, kind, route):
+    ua, ub, za, zb = AFFINE_KINDS[kind]
+    rng = np.random.default_rng(M + N + K)
+    A = rng.integers(0, 256, (M, K)).astype(np.uint8)
+    B = rng.integers(0, 256, (N, K)).astype(np.uint8)
+    A, B = (A if ua else A.view(np.int8)), (B if ub else B.view(np.int8))
+    print(f"affine {kind} M={M} N={N} K={K}", flush=True)
+    got = host(ops.quantized_dot(dev(A), dev(B), za, zb))
+    assert ops.last_gemm().startswith(route), ops.last_gemm()
+    want = (A.astype(np.float64) - za) @ (B.astype(np.float64) - zb).T      # exact: sums below 2^53
+    np.testing.assert_array_equal(got, want.astype(np.int64).astype(np.int32))
