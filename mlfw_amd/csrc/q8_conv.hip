@@ -365,19 +365,6 @@ bool conv_affine(const ConvGeom& G) { return G.zpx != 0 || G.zpw != 0 || G.x_u8 
 constexpr size_t CONV_BATCH_BYTES = (size_t)128 << 20;   // workspace per batch of images
 static size_t round256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-// Images per batch: as many as fit CONV_BATCH_BYTES of per-image workspace
-// (`per`), within the launch limits; 1 with 16 or fewer output channels per
-// group, which go through the GEMV kernel one image at a time.
-static int64_t conv_batch_of(const ConvGeom& G, size_t per) {
-  if (G.Og <= 16) return 1;
-  int64_t nb = per ? (int64_t)(CONV_BATCH_BYTES / per) : 1;
-  nb = nb > G.N ? G.N : nb;
-  nb = nb > 65535 ? 65535 : nb;                                 // grid.y of the per-image launches
-  const int64_t cap = ((int64_t)1 << 31) / (G.Pn > 0 ? G.Pn : 1) - 1;   // GEMM N = nb * P in an int
-  nb = nb > cap ? cap : nb;
-  return nb < 1 ? 1 : nb;
-}
-
 // The channel-last path: Cg a multiple of 16, at most WT_CHUNKS kernel
 // positions, frame and matrix offsets of one image within 31 bits.
 static bool conv_frame_of(const ConvGeom& G, ConvFrame* F) {
@@ -405,62 +392,45 @@ static size_t conv_wt_bytes(const ConvGeom& G) {   // 1 x 1: the weight as given
   return G.Kn == 1 ? 0 : round256((size_t)G.O * (size_t)G.Kc);
 }
 
-// What split partial sums of the GEMM took (conv_workspace_need counts them).
-static size_t conv_split_bytes(int64_t M, int64_t N, int64_t K) {
-  const int64_t cus = cu_count() > 0 ? cu_count() : 256;
-  const int64_t tiles64 = ((M + 63) / 64) * ((N + 63) / 64);
-  const int64_t bm = M >= 128 && tiles64 >= 2 * cus ? 128 : 64;
-  const int64_t tiles = ((M + bm - 1) / bm) * ((N + bm - 1) / bm), KT = (K + 127) / 128;
-  int64_t splits = 1;
-  if (tiles < cus && K >= 4096) {
-    splits = (2 * cus + tiles - 1) / tiles;
-    splits = splits < 8 ? splits : 8;
-    splits = splits < KT / 8 ? splits : KT / 8;
-    splits = splits > 1 ? splits : 1;
-  }
-  while (splits > 1 && splits * M * N * 4 > ((int64_t)1 << 30)) --splits;
-  const int64_t kps = (KT + splits - 1) / splits;
-  splits = (KT + kps - 1) / kps;
-  return splits > 1 ? round256((size_t)(splits * M * N * 4)) : 0;
+// Symmetric int8 with more than two tiles per CU: weight rows padded to the
+// matrix's pitch for the direct-to-LDS GEMM (32 x 3 x 112 x 112, 7 x 7 at
+// stride 2: 48.4 us against 53.5 with the weight at its own pitch).
+static bool conv_im2col_many(const ConvGeom& G) {
+  const int64_t t64 = ((G.Og + 63) / 64) * ((G.N * G.Pn + 63) / 64);
+  return !conv_affine(G) && G.groups == 1 && t64 > 2 * (cu_count() > 0 ? cu_count() : 256) &&
+         (int64_t)G.Kc16 * 256 < ((int64_t)1 << 31);
 }
 
-// The least workspace a symmetric int8 conv is accepted with.  (What each
-// path below needs for one image and one group is no more; it runs as many
-// at once as fit the workspace it is given.)
+// Workspace bytes of one image and group, and of the weight rows beside them.
+struct ConvUnit {
+  size_t unit, wt;
+};
+static ConvUnit conv_unit(const ConvGeom& G) {
+  ConvFrame F;
+  if (conv_frame_path(G, &F)) return {(size_t)F.Ep * (size_t)G.Cg, conv_wt_bytes(G)};
+  return {(size_t)G.Pn * (size_t)G.Kc16, conv_im2col_many(G) && G.Kc16 != G.Kc ? (size_t)G.O * (size_t)G.Kc16 : 0};
+}
+
+// The least workspace a symmetric int8 conv is accepted with: one image of
+// one group at a time (where its first bytes are skipped for alignment and
+// that no longer fits, the direct kernel runs).
 size_t conv_workspace_need(const ConvGeom& G) {
   if (!conv_uses_gemm(G)) return 0;
-  // the im2col form: batched matrices, then padded weight rows
-  size_t b = round256((size_t)conv_batch_of(G, (size_t)G.Pn * (size_t)G.Kc16) * (size_t)G.Pn *
-                      (size_t)G.Kc16);
-  if (G.Kc16 != G.Kc) b += (size_t)G.O * (size_t)G.Kc16;
+  const ConvUnit u = conv_unit(G);
   ConvFrame F;
-  if (conv_frame_of(G, &F)) {
-    // frames of a batch; receptive fields too where the GEMM once needed them
-    const bool impl = !conv_pointwise(G) && G.Cg % 64 == 0 && G.Kc <= 16384 && G.Og > 16;
-    const size_t col1 = conv_pointwise(G) || impl ? 0 : (size_t)G.Pn * (size_t)G.Kc;
-    const size_t fr1 = (size_t)F.Ep * (size_t)G.Cg;
-    const int64_t nb = conv_batch_of(G, col1 + fr1);
-    size_t cl = round256((size_t)nb * col1) + round256((size_t)nb * fr1) + conv_wt_bytes(G);
-    if (impl) {
-      cl += conv_split_bytes(G.Og, nb * G.Pn, G.Kc);
-    }
-    b = cl > b ? cl : b;
-  }
-  return b;
+  return u.unit + (conv_frame_path(G, &F) ? u.wt : 0);
 }
 
-// What q8_quantized_conv_workspace asks for: every group of as many images
-// as fit CONV_BATCH_BYTES.
+// What q8_quantized_conv_workspace asks for: as many groups, and images of
+// all groups, as fit CONV_BATCH_BYTES, and room to start at a 16-byte
+// boundary.
 size_t conv_workspace_bytes(const ConvGeom& G) {
-  const size_t need = conv_workspace_need(G);
-  if (need == 0 && !conv_short_gemm(G)) return 0;
-  ConvFrame F;
-  const bool fr = conv_frame_path(G, &F);
-  const size_t per = (size_t)G.groups * (fr ? (size_t)F.Ep * (size_t)G.Cg : (size_t)G.Pn * (size_t)G.Kc16);
-  size_t nb = per ? CONV_BATCH_BYTES / per : 1;
-  nb = nb < 1 ? 1 : nb > (size_t)G.N ? (size_t)G.N : nb;
-  const size_t want = round256(nb * per) + (fr ? conv_wt_bytes(G) : (size_t)G.O * (size_t)G.Kc16);
-  return want > need ? want : need;
+  if (!conv_uses_gemm(G) && !conv_short_gemm(G)) return 0;
+  const ConvUnit u = conv_unit(G);
+  size_t n = CONV_BATCH_BYTES / u.unit;
+  const size_t groups = (size_t)G.groups, images = n / groups;
+  n = images > 0 ? groups * (images < (size_t)G.N ? images : (size_t)(G.N > 0 ? G.N : 1)) : n > 0 ? n : 1;
+  return round256(n * u.unit + 15) + u.wt;
 }
 
 // Images and groups of one pass over `unit` workspace bytes each, with the
@@ -487,31 +457,25 @@ static bool conv_batch(const ConvGeom& G, size_t unit, size_t wt, size_t avail, 
   return true;
 }
 
-// Symmetric int8 with more than two tiles per CU: weight rows padded to the
-// matrix's pitch for the direct-to-LDS GEMM (32 x 3 x 112 x 112, 7 x 7 at
-// stride 2: 48.4 us against 53.5 with the weight at its own pitch).
-static bool conv_im2col_many(const ConvGeom& G) {
-  const int64_t t64 = ((G.Og + 63) / 64) * ((G.N * G.Pn + 63) / 64);
-  return !conv_affine(G) && G.groups == 1 && t64 > 2 * (cu_count() > 0 ? cu_count() : 256) &&
-         (int64_t)G.Kc16 * 256 < ((int64_t)1 << 31);
-}
-
 ConvPlan conv_plan(const ConvGeom& G, const void* ws, size_t ws_bytes, bool prepacked) {
   ConvPlan p;
   if (ws == nullptr || G.N * G.O * G.Pn == 0 || !(conv_uses_gemm(G) || conv_short_gemm(G))) return p;
   if (conv_fill(G) < -128 || conv_fill(G) > 127) return p;
-  if (conv_uses_gemm(G) ? conv_affine(G) && ws_bytes < conv_workspace_need(G) : ws_bytes < conv_workspace_bytes(G))
-    return p;
   p.skip = (16 - (reinterpret_cast<uintptr_t>(ws) & 15)) & 15;
   const size_t avail = ws_bytes > p.skip ? ws_bytes - p.skip : 0;
   ConvFrame F;
-  const size_t unit = (size_t)G.Pn * (size_t)G.Kc16;
+  const size_t mat = (size_t)G.Pn * (size_t)G.Kc16;
   if (conv_frame_path(G, &F) && conv_batch(G, (size_t)F.Ep * (size_t)G.Cg, prepacked ? 0 : conv_wt_bytes(G), avail, &p))
     p.route = ConvPlan::FRAME;
-  else if ((conv_im2col_many(G) && G.Kc16 != G.Kc && conv_batch(G, unit, (size_t)G.O * (size_t)G.Kc16, avail, &p)) ||
-           conv_batch(G, unit, 0, avail, &p))
+  else if ((conv_im2col_many(G) && G.Kc16 != G.Kc && conv_batch(G, mat, (size_t)G.O * (size_t)G.Kc16, avail, &p)) ||
+           conv_batch(G, mat, 0, avail, &p))
     p.route = ConvPlan::IM2COL;
-  return p;
+  if (p.route == ConvPlan::DIRECT) return p;
+  // A workspace that holds a part of the batch: a pass is two launches, about
+  // 8 us, and the direct kernel does about 1.2e12 multiply-adds a second.
+  const double passes = (double)((G.N + p.nb - 1) / p.nb) * (double)((G.groups + p.gc - 1) / p.gc);
+  const double macs = (double)G.N * (double)G.O * (double)G.Pn * (double)G.Kc;
+  return passes > 1.0 && 8.0 * passes > macs / 1.2e6 ? ConvPlan{} : p;
 }
 
 // The affine correction of the conv's GEMM (A: weights, B: input).

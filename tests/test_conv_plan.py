@@ -128,3 +128,50 @@ def test_short_contraction_with_the_workspace_it_asks_for(lib, case):
     for at in (0x1001, 0x1008, 0x100f):
         route, nb, gc, b = plan(lib, args, at, want)
         assert max(b, written(case, route, nb, gc, at, 0)) <= want
+
+
+def test_workspace_asked_for_and_least_accepted(lib):
+    """No more is asked for than one batch (128 MiB, or one image of one group
+    where that is larger) and the weight rows; a symmetric conv is accepted
+    with one image of one group, and refused below."""
+    rng = random.Random(11)
+    many_groups = ([2, 256, 512, 512], [256, 8, 3, 3], [1, 1], [1, 1], [1, 1], [1, 1], 32)
+    deep = ([4, 64, 12, 12], [32, 64, 3, 3], [1, 1], [1, 1], [1, 1], [1, 1], 1)      # long contraction, few tiles
+    for case in [many_groups, deep] + [random_case(rng) for _ in range(300)]:
+        args = geom(*case)
+        want = asked(lib, args)
+        xs, ws, g = case[0], case[1], case[6]
+        kc = ws[1]
+        for k in ws[2:]:
+            kc *= k
+        kn = kc // ws[1]
+        frame = ws[1] % 16 == 0 and kc <= 65536 and kn <= 1024
+        weight = ws[0] * (kc if frame and kn > 1 else -(-kc // 16) * 16)
+        unit = written(case, FRAME if frame else MATRIX, 1, 1, 0, 1)
+        assert want <= max(128 << 20, unit) + 512 + weight + 256, case
+        if kc < 64:
+            continue
+        least = unit + (ws[0] * kc + 255) // 256 * 256 * (frame and kn > 1)
+        assert least <= want, case
+        assert plan(lib, args, 0x1000, least) is not None, case
+        assert plan(lib, args, 0x1000, least - 1) is None, case
+    # every group of every image in one pass where that is within a batch
+    assert plan(lib, geom(*deep), 0x1000, asked(lib, geom(*deep)))[1:3] == (4, 1)
+    r, nb, gc, b = plan(lib, geom(*many_groups), 0x1000, asked(lib, geom(*many_groups)))
+    assert r == MATRIX and nb == 1 and 1 < gc < 32
+
+
+def test_part_of_a_batch_or_one_thread_per_output(lib):
+    """A workspace for part of the batch is used while its passes are fewer
+    than the one-thread kernel's time is worth; below one image the affine
+    call runs that kernel and the symmetric one is refused."""
+    big = geom([16, 64, 56, 56], [64, 64, 3, 3], [1, 1], [1, 1], [1, 1], [1, 1], 1)
+    one = 58 * 58 * 64 + 64 * 576
+    for kind in ((0, 0, 0, 0), (1, 117, 0, 0)):
+        assert plan(lib, big, 0x1000, one, *kind)[:3] == (FRAME, 1, 1)
+    assert plan(lib, big, 0x1000, one - 1) is None
+    assert plan(lib, big, 0x1000, one - 1, 1, 117)[0] == DIRECT
+    tiny = geom([1000, 16, 7, 7], [16, 16, 3, 3], [1, 1], [1, 1], [1, 1], [1, 1], 1)
+    one = 9 * 9 * 16 + 16 * 144
+    assert plan(lib, tiny, 0x1000, asked(lib, tiny), 1, 117)[:3] == (FRAME, 1000, 1)
+    assert plan(lib, tiny, 0x1000, one, 1, 117)[0] == DIRECT      # 1000 passes for 0.1 ms of work

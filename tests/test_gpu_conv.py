@@ -300,3 +300,32 @@ def test_conv_misaligned_weight_and_workspace(ops, oracle, xs, ws, pd, u8, ws_sh
     st, zp = [1] * (len(xs) - 2), 77 if u8 else 0
     got = conv_call(x, w, st, pd, zpx=zp, ws_shift=ws_shift, w_shift=w_shift)
     same_bits(got, oracle.quantized_conv(x, w, st, pd, [1] * len(st), 1, zp, 0))
+
+
+@pytest.mark.parametrize("xs,ws,pd,g,u8", [((5, 64, 28, 28), (64, 64, 3, 3), [[1, 1], [1, 1]], 1, False),
+                                           ((4, 96, 28, 28), (96, 32, 3, 3), [[1, 1], [1, 1]], 3, False),
+                                           ((4, 96, 28, 28), (96, 32, 3, 3), [[1, 1], [1, 1]], 3, True),
+                                           ((6, 20, 40, 40), (48, 10, 3, 3), [[1, 1], [1, 0]], 2, False),
+                                           ((6, 20, 40, 40), (48, 10, 3, 3), [[1, 1], [1, 0]], 2, True)])
+def test_conv_in_several_passes(ops, oracle, xs, ws, pd, g, u8):
+    """A workspace for one image of one group, for an odd share of the batch
+    and for all of it but a byte: the passes over images and groups give the
+    same bits and stay inside it."""
+    import ctypes as C
+    from mlfw_amd import _lib as L
+    rng = np.random.default_rng(sum(xs))
+    x = rng.integers(0, 256, xs).astype(np.uint8)
+    x = x if u8 else x.view(np.int8)
+    w = rng.integers(-128, 128, ws).astype(np.int8)
+    zp = 77 if u8 else 0
+    want = oracle.quantized_conv(x, w, [1, 1], pd, [1, 1], g, zp, 0)
+    arr = lambda v: (C.c_int64 * len(v))(*v)  # noqa: E731
+    need = C.c_size_t(0)
+    lo, hi = [p[0] for p in pd], [p[1] for p in pd]
+    L.call("q8_quantized_conv_workspace", 2, arr(xs), arr(ws), arr([1, 1]), arr(lo), arr(hi), arr([1, 1]), g, C.byref(need))
+    P = [xs[2 + i] + lo[i] + hi[i] - ws[2 + i] + 1 for i in range(2)]
+    kc = ws[1] * ws[2] * ws[3]
+    one = ((xs[2] + lo[0] + hi[0]) * (xs[3] + lo[1] + hi[1]) * ws[1] + (ws[0] * kc + 255) // 256 * 256
+           if ws[1] % 16 == 0 else P[0] * P[1] * ((kc + 15) // 16 * 16))
+    for size in (one, (one + need.value) // 2, need.value - 1):
+        same_bits(conv_call(x, w, [1, 1], pd, g, zpx=zp, ws_bytes=size), want)
