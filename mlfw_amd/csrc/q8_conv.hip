@@ -465,9 +465,17 @@ ConvPlan conv_plan(const ConvGeom& G, const void* ws, size_t ws_bytes, bool prep
   const size_t avail = ws_bytes > p.skip ? ws_bytes - p.skip : 0;
   ConvFrame F;
   const size_t mat = (size_t)G.Pn * (size_t)G.Kc16;
-  if (conv_frame_path(G, &F) && conv_batch(G, (size_t)F.Ep * (size_t)G.Cg, prepacked ? 0 : conv_wt_bytes(G), avail, &p))
+  if (conv_frame_path(G, &F) && conv_batch(G, (size_t)F.Ep * (size_t)G.Cg, prepacked ? 0 : conv_wt_bytes(G), avail, &p)) {
     p.route = ConvPlan::FRAME;
-  else if ((conv_im2col_many(G) && G.Kc16 != G.Kc && conv_batch(G, mat, (size_t)G.O * (size_t)G.Kc16, avail, &p)) ||
+    // the frame launch: 64 x 64 tiles of positions and channels in 2^23
+    // workgroups, the channel tiles in grid.z
+    const int64_t wide = (int64_t)64 * 65535 / G.Cg;
+    if (p.gc > wide) p.gc = (int)wide, p.nb = 1;
+    const int64_t tiles = ((F.Ep + 63) / 64) * (((int64_t)p.gc * G.Cg + 63) / 64);
+    const int64_t cap = ((int64_t)1 << 23) / tiles;
+    if (p.nb > cap) p.nb = cap;
+    p.bytes = p.skip + p.wt + (size_t)p.nb * (size_t)p.gc * (size_t)F.Ep * (size_t)G.Cg;
+  } else if ((conv_im2col_many(G) && G.Kc16 != G.Kc && conv_batch(G, mat, (size_t)G.O * (size_t)G.Kc16, avail, &p)) ||
            conv_batch(G, mat, 0, avail, &p))
     p.route = ConvPlan::IM2COL;
   if (p.route == ConvPlan::DIRECT) return p;

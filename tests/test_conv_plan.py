@@ -175,3 +175,14 @@ def test_part_of_a_batch_or_one_thread_per_output(lib):
     one = 9 * 9 * 16 + 16 * 144
     assert plan(lib, tiny, 0x1000, asked(lib, tiny), 1, 117)[:3] == (FRAME, 1000, 1)
     assert plan(lib, tiny, 0x1000, one, 1, 117)[0] == DIRECT      # 1000 passes for 0.1 ms of work
+
+
+def test_frame_launches_stay_within_the_grid(lib):
+    """More channel tiles than grid.z takes, and more 64 x 64 tiles than a
+    launch: fewer groups or images a pass, as a launch per group once did."""
+    wide = geom([1, 128 * 40000, 1], [40000 * 17, 128, 1], [1], [0], [0], [1], 40000)
+    r, nb, gc, b = plan(lib, wide, 0x1000, 1 << 33)
+    assert r == FRAME and 0 < gc * 128 <= 64 * 65535
+    points = geom([65535, 32768, 1], [17, 32768, 1], [1], [0], [0], [1], 1)
+    r, nb, gc, b = plan(lib, points, 0x1000, 1 << 33)
+    assert r == FRAME and 0 < nb * 512 <= 1 << 23
