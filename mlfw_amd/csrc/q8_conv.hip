@@ -401,6 +401,20 @@ static bool conv_im2col_many(const ConvGeom& G) {
          (int64_t)G.Kc16 * 256 < ((int64_t)1 << 31);
 }
 
+// Groups one after another, each through the direct-to-LDS GEMM, where a
+// group's product alone fills the chip with 128 x 128 tiles: that GEMM's lead
+// over the one launch for all groups then pays for a frame and a GEMM launch
+// a group (3 x 3: 64 x 512 x 28 x 28 -> 512 in two groups 122 us against 153,
+// 8 x 256 x 56 x 56 -> 512 45 and 55, 32 x 256 x 28 x 28 -> 256, 196 tiles a
+// group, 39 and 33; 1 x 1, from two tiles per CU on: 64 x 512 x 28 x 28 -> 512
+// 55 and 59, 64 x 256 x 14 x 14 -> 1024, 392 tiles, 33 and 31).
+static bool conv_by_group(const ConvGeom& G) {
+  if (G.groups == 1 || conv_affine(G) || G.Og < 128) return false;
+  if (!conv_pointwise(G) && (G.Cg % 64 != 0 || G.Kc > 16384)) return false;
+  const int64_t cus = cu_count() > 0 ? cu_count() : 256, t128 = ((G.Og + 127) / 128) * ((G.N * G.Pn + 127) / 128);
+  return t128 >= (conv_pointwise(G) ? 2 * cus : cus);
+}
+
 // Workspace bytes of one image and group, and of the weight rows beside them.
 struct ConvUnit {
   size_t unit, wt;
@@ -436,15 +450,15 @@ size_t conv_workspace_bytes(const ConvGeom& G) {
 // Images and groups of one pass over `unit` workspace bytes each, with the
 // weight rows' wt before or after them: as many as fit `avail` and the launch
 // limits.  False where not even one does.
-static bool conv_batch(const ConvGeom& G, size_t unit, size_t wt, size_t avail, ConvPlan* p) {
+static bool conv_batch(const ConvGeom& G, size_t unit, size_t wt, size_t avail, ConvPlan* p, bool by_group = false) {
   if (avail < wt || avail - wt < unit) return false;
   const int64_t units = (int64_t)((avail - wt) / unit);
   const int64_t fit = (((int64_t)1 << 31) - 1) / (int64_t)unit;           // one pass's offsets in 31 bits
   int64_t gc = units < G.groups ? units : G.groups;
   gc = gc < fit ? gc : fit;
   gc = gc < 65535 ? gc : 65535;
-  gc = gc < 1 ? 1 : gc;
-  int64_t nb = gc == G.groups ? units / gc : 1;
+  gc = gc < 1 || by_group ? 1 : gc;
+  int64_t nb = gc == G.groups || by_group ? units / gc : 1;
   nb = nb > G.N ? G.N : nb;
   nb = nb > 65535 ? 65535 : nb;                                           // grid.y of the per-image launches
   const int64_t cap = ((int64_t)1 << 31) / G.Pn - 1;                      // GEMM N = nb * P in an int
@@ -465,7 +479,8 @@ ConvPlan conv_plan(const ConvGeom& G, const void* ws, size_t ws_bytes, bool prep
   const size_t avail = ws_bytes > p.skip ? ws_bytes - p.skip : 0;
   ConvFrame F;
   const size_t mat = (size_t)G.Pn * (size_t)G.Kc16;
-  if (conv_frame_path(G, &F) && conv_batch(G, (size_t)F.Ep * (size_t)G.Cg, prepacked ? 0 : conv_wt_bytes(G), avail, &p)) {
+  if (conv_frame_path(G, &F) && conv_batch(G, (size_t)F.Ep * (size_t)G.Cg, prepacked ? 0 : conv_wt_bytes(G), avail, &p,
+                                          conv_by_group(G))) {
     p.route = ConvPlan::FRAME;
     // the frame launch: 64 x 64 tiles of positions and channels in 2^23
     // workgroups, the channel tiles in grid.z
@@ -561,7 +576,7 @@ static hipError_t launch_conv_channel_last(const int8_t* x, const int8_t* w, con
       // 14 x 1024 -> 256: 16.6 against 18.9); with fewer, K groups do (7 x 7 x
       // 512: 25.1, split over K in two launches, against 21.6 us).
       const int64_t t64 = ((G.Og + 63) / 64) * ((nb * G.Pn + 63) / 64);
-      const bool many = !affine && G.groups == 1 && t64 > (cu_count() > 0 ? cu_count() : 256);
+      const bool many = !affine && cb.gc == 1 && t64 > (cu_count() > 0 ? cu_count() : 256);
       if (many && !conv_pointwise(G) && G.Cg % 64 == 0 && G.Kc <= 16384) {
         err = launch_gemm_conv(A, xp, G.Og, nb * G.Pn, G.Kc, eb, o, st);
       } else if (many && conv_pointwise(G) && (reinterpret_cast<uintptr_t>(A) & 15) == 0) {

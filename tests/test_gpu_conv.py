@@ -329,3 +329,33 @@ def test_conv_in_several_passes(ops, oracle, xs, ws, pd, g, u8):
            if ws[1] % 16 == 0 else P[0] * P[1] * ((kc + 15) // 16 * 16))
     for size in (one, (one + need.value) // 2, need.value - 1):
         same_bits(conv_call(x, w, [1, 1], pd, g, zpx=zp, ws_bytes=size), want)
+
+
+# Symmetric convs in groups whose product fills the chip with 128 x 128 tiles
+# run a group at a time through the direct-to-LDS GEMM; smaller ones, and
+# affine ones, all groups in one launch
+GROUPED = [((44, 128, 28, 28), (256, 64, 3, 3), 2, False, "conv 128x128"),
+           ((43, 128, 28, 28), (300, 64, 3, 3), 2, False, "conv 128x128"),
+           ((20, 128, 28, 28), (256, 64, 3, 3), 2, False, "any conv"),
+           ((44, 128, 28, 28), (256, 64, 3, 3), 2, True, "any conv"),
+           ((44, 96, 28, 28), (256, 48, 3, 3), 2, False, "any conv"),
+           ((86, 128, 28, 28), (256, 64, 1, 1), 2, False, "qgemm"),
+           ((44, 128, 28, 28), (256, 64, 1, 1), 2, False, "any conv")]
+
+
+@pytest.mark.parametrize("xs,ws,g,u8,route", GROUPED)
+def test_conv_large_groups(ops, oracle, xs, ws, g, u8, route):
+    rng = np.random.default_rng(sum(xs) + sum(ws))
+    x = rng.integers(0, 256, xs).astype(np.uint8)
+    x = x if u8 else x.view(np.int8)
+    w = rng.integers(-128, 128, ws).astype(np.int8)
+    pad = ws[2] // 2
+    pd, zp = [[pad, pad]] * 2, 77 if u8 else 0
+    want = oracle.quantized_conv(x, w, [1, 1], pd, [1, 1], g, zp, 0)
+    wt = None if u8 or pad == 0 else ops.conv_weight_taps(dev(w), g)
+    for taps in {None, wt}:
+        got = ops.quantized_conv(dev(x), dev(w), [1, 1], pd, groups=g, zpx=zp, w_taps=taps)
+        assert ops.last_gemm().startswith(route), ops.last_gemm()
+        same_bits(host(got), want)
+    got = ops.quantized_conv(dev(x), dev(w), [1, 1], pd, groups=g, zpx=zp, s_out=1.7e-4)
+    same_bits(host(got), (want.astype(np.float64) * 1.7e-4).astype(np.float32))
