@@ -574,12 +574,16 @@ static hipError_t launch_conv_channel_last(const int8_t* x, const int8_t* w, con
       // With more than one 64 x 64 tile per CU the direct-to-LDS GEMM's
       // cheaper copies win (56 x 56 x 64: 24.3 against 25.7 us; 1 x 1 14 x
       // 14 x 1024 -> 256: 16.6 against 18.9); with fewer, K groups do (7 x 7 x
-      // 512: 25.1, split over K in two launches, against 21.6 us).
-      const int64_t t64 = ((G.Og + 63) / 64) * ((nb * G.Pn + 63) / 64);
-      const bool many = !affine && cb.gc == 1 && t64 > (cu_count() > 0 ? cu_count() : 256);
-      if (many && !conv_pointwise(G) && G.Cg % 64 == 0 && G.Kc <= 16384) {
+      // 512: 25.1, split over K in two launches, against 21.6 us).  A 1 x 1
+      // conv needs no more than a 32 x 32 tile per CU: its rows are short (16 x
+      // 256 x 28 x 28 -> 64, 196 64 x 64 tiles: 9.3 against 11.5; 8 x 64 x 14 x
+      // 14 -> 64, 98 of 32 x 32: 8.6 against 7.7).
+      const int64_t cus = cu_count() > 0 ? cu_count() : 256;
+      const int64_t t32 = ((G.Og + 31) / 32) * ((nb * G.Pn + 31) / 32), t64 = ((G.Og + 63) / 64) * ((nb * G.Pn + 63) / 64);
+      const bool aligned = !affine && cb.gc == 1;
+      if (aligned && t64 > cus && !conv_pointwise(G) && G.Cg % 64 == 0 && G.Kc <= 16384) {
         err = launch_gemm_conv(A, xp, G.Og, nb * G.Pn, G.Kc, eb, o, st);
-      } else if (many && conv_pointwise(G) && (reinterpret_cast<uintptr_t>(A) & 15) == 0) {
+      } else if (aligned && t32 > cus && conv_pointwise(G) && (reinterpret_cast<uintptr_t>(A) & 15) == 0) {
         err = launch_gemm(A, xp, G.Og, nb * G.Pn, G.Kc, eb, o, st);
       } else {
         AnyPlan p;

@@ -359,3 +359,23 @@ def test_conv_large_groups(ops, oracle, xs, ws, g, u8, route):
         same_bits(host(got), want)
     got = ops.quantized_conv(dev(x), dev(w), [1, 1], pd, groups=g, zpx=zp, s_out=1.7e-4)
     same_bits(host(got), (want.astype(np.float64) * 1.7e-4).astype(np.float32))
+
+
+# 1 x 1 convs on either side of one 32 x 32 tile per CU (256), whole and ragged
+POINTWISE = [((8, 64, 14, 14), 64, "any conv 32x32"), ((16, 256, 28, 28), 64, "qgemm 64x64"),
+             ((11, 80, 27, 29), 33, "qgemm 64x64"), ((1, 2048, 28, 28), 512, "ring"), ((5, 48, 30, 30), 96, "qgemm"),
+             ((2, 96, 45, 46), 65, "qgemm")]
+
+
+@pytest.mark.parametrize("xs,o,route", POINTWISE)
+@pytest.mark.parametrize("w_shift", [0, 1])
+def test_conv_pointwise(ops, oracle, xs, o, route, w_shift):
+    rng = np.random.default_rng(sum(xs) + o)
+    x = rng.integers(-128, 128, xs).astype(np.int8)
+    w = rng.integers(-128, 128, (o, xs[1], 1, 1)).astype(np.int8)
+    want = oracle.quantized_conv(x, w, [1, 1], [[0, 0], [0, 0]], [1, 1], 1)
+    got = conv_call(x, w, [1, 1], [[0, 0], [0, 0]], w_shift=w_shift)
+    assert ops.last_gemm().startswith("any conv" if w_shift else route), ops.last_gemm()
+    same_bits(got, want)
+    got = conv_call(x, w, [1, 1], [[0, 0], [0, 0]], w_shift=w_shift, s_out=1.7e-4)
+    same_bits(got, (want.astype(np.float64) * 1.7e-4).astype(np.float32))
