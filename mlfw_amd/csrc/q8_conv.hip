@@ -444,7 +444,10 @@ size_t conv_workspace_bytes(const ConvGeom& G) {
   size_t n = CONV_BATCH_BYTES / u.unit;
   const size_t groups = (size_t)G.groups, images = n / groups;
   n = images > 0 ? groups * (images < (size_t)G.N ? images : (size_t)(G.N > 0 ? G.N : 1)) : n > 0 ? n : 1;
-  return round256(n * u.unit + 15) + u.wt;
+  // (a batch of fewer images than this or of part of the groups splits K no
+  // further: a split is for fewer tiles than CUs)
+  const int64_t nb = images > 0 ? (int64_t)(n / groups) : 1, gc = images > 0 ? G.groups : (int64_t)n;
+  return round256(n * u.unit + 15) + round256(u.wt) + any_part_bytes(G.Og, nb * G.Pn, gc, any_splits(G.Og, nb * G.Pn, G.Kc, gc));
 }
 
 // Images and groups of one pass over `unit` workspace bytes each, with the
@@ -494,6 +497,14 @@ ConvPlan conv_plan(const ConvGeom& G, const void* ws, size_t ws_bytes, bool prep
            conv_batch(G, mat, 0, avail, &p))
     p.route = ConvPlan::IM2COL;
   if (p.route == ConvPlan::DIRECT) return p;
+  // few tiles over a long contraction: partial sums of a K split behind the rest
+  const int splits = any_splits(G.Og, p.nb * G.Pn, G.Kc, p.gc);
+  const size_t part = any_part_bytes(G.Og, p.nb * G.Pn, p.gc, splits);
+  if (splits > 1 && p.bytes + part <= ws_bytes) {
+    p.splits = splits;
+    p.part = p.bytes;
+    p.bytes += part;
+  }
   // A workspace that holds a part of the batch: a pass is two launches, about
   // 8 us, and the direct kernel does about 1.2e12 multiply-adds a second.
   const double passes = (double)((G.N + p.nb - 1) / p.nb) * (double)((G.groups + p.gc - 1) / p.gc);
@@ -513,7 +524,8 @@ static AffineDot conv_zp(const ConvGeom& G) {
 
 static hipError_t launch_conv_channel_last(const int8_t* x, const int8_t* w, const int8_t* w_taps,
                                            const ConvGeom& G, const ConvFrame& F, const GemmEpi& e,
-                                           const ConvPlan& cb, int8_t* workspace, void* out, hipStream_t st) {
+                                           const ConvPlan& cb, int8_t* workspace, int32_t* part, void* out,
+                                           hipStream_t st) {
   int8_t* wt_ws = workspace;
   int8_t* xp = wt_ws + cb.wt;
   // a 1 x 1 kernel's weight is its own tap-major form; a prepacked one
@@ -594,6 +606,8 @@ static hipError_t launch_conv_channel_last(const int8_t* x, const int8_t* w, con
         p.b_step = G.Cg;
         p.o_step = (int64_t)G.Og * G.Pn;
         p.conv_cg = G.Cg;
+        p.splits = cb.splits;
+        p.part = part;
         err = launch_gemm_any(A, xp, G.Og, nb * G.Pn, G.Kc, eb, zp, p, o, st);
       }
       if (err != hipSuccess) return err;
@@ -605,7 +619,7 @@ static hipError_t launch_conv_channel_last(const int8_t* x, const int8_t* w, con
 // Receptive fields as a matrix (k_im2col), every group of a batch of images
 // at once; the GEMM takes the weight rows at their own pitch.
 static hipError_t launch_conv_im2col(const int8_t* x, const int8_t* w, const ConvGeom& G, const GemmEpi& e,
-                                     const ConvPlan& cb, int8_t* col, void* out, hipStream_t st) {
+                                     const ConvPlan& cb, int8_t* col, int32_t* part, void* out, hipStream_t st) {
   const bool many = conv_im2col_many(G);
   const int8_t* wmat = w;
   if (cb.wt) {
@@ -649,6 +663,8 @@ static hipError_t launch_conv_im2col(const int8_t* x, const int8_t* w, const Con
       p.a_step = (int64_t)G.Og * G.Kc;
       p.b_step = nb * G.Pn * G.Kc16;
       p.o_step = (int64_t)G.Og * G.Pn;
+      p.splits = cb.splits;
+      p.part = part;
       err = launch_gemm_any(w + g * G.Og * G.Kc, col, G.Og, nb * G.Pn, G.Kc, eb, zp, p, o, st);
       if (err != hipSuccess) return err;
     }
@@ -679,10 +695,11 @@ hipError_t launch_conv(const int8_t* x, const int8_t* w, const int8_t* w_taps, c
     return hipGetLastError();
   }
   int8_t* ws = static_cast<int8_t*>(workspace) + p.skip;
-  if (p.route == ConvPlan::IM2COL) return launch_conv_im2col(x, w, G, e, p, ws, out, st);
+  int32_t* part = reinterpret_cast<int32_t*>(static_cast<int8_t*>(workspace) + p.part);
+  if (p.route == ConvPlan::IM2COL) return launch_conv_im2col(x, w, G, e, p, ws, part, out, st);
   ConvFrame F;
   if (!conv_frame_path(G, &F)) return hipErrorInvalidValue;
-  return launch_conv_channel_last(x, w, w_taps, G, F, e, p, ws, out, st);
+  return launch_conv_channel_last(x, w, w_taps, G, F, e, p, ws, part, out, st);
 }
 
 }  // namespace q8

@@ -269,6 +269,7 @@ void k_qgemm_any(const int8_t* __restrict__ A, const int8_t* __restrict__ B, int
 // this form lose: 64 x 11008 x 4096 takes 25 us with 64 x 64, 21 staged.)
 constexpr int WKT = 2, WKW = 8, WKB = 16 * WKT;       // 16-row blocks, waves, tile edge
 constexpr int WK_PITCH = WKB + 4;
+constexpr int ANY_SPLIT_K = 4096;
 constexpr int WK_LDS = WKT * WKW * 16 * WK_PITCH * 4 + 8 * WKB + 8 * WKB;
 template <bool ZP, bool CONV>
 __global__ __launch_bounds__(64 * WKW, 2)
@@ -355,14 +356,16 @@ void k_qgemm_wk(const int8_t* __restrict__ A, const int8_t* __restrict__ B, int 
       }
     }
   };
+  // blockIdx.z: the split; its waves take every 8 * splits-th slice
   Frag f0, f1;
-  int s = 2 * wave;
+  const int zs = (int)blockIdx.z, stride = 2 * WKW * (int)gridDim.z;
+  int s = 2 * (wave + WKW * zs);
   if (s < KS) load(s, f0);
   while (s < KS) {
     const bool two = s + 1 < KS;
     if (two) load(s + 1, f1);
     mul(s, f0);
-    const int nx = s + 2 * WKW;
+    const int nx = s + stride;
     if (nx < KS) load(nx, f0);
     if (two) mul(s + 1, f1);
     s = nx;
@@ -396,8 +399,12 @@ void k_qgemm_wk(const int8_t* __restrict__ A, const int8_t* __restrict__ B, int 
     uint32_t a = 0u;
 #pragma unroll
     for (int w = 0; w < WKW; ++w) a += (uint32_t)red[((row / 16 * WKW + w) * 16 + row % 16) * WK_PITCH + col];
+    if constexpr (ZP) a += (zs == 0 ? z.kcc : 0u) + (uint32_t)z.cA * (uint32_t)sum_b[col] + (uint32_t)z.cB * (uint32_t)sum_a[row];
+    if (p.splits > 1) {                                  // uniform
+      p.part[(((int64_t)zs * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x) * (WKB * WKB) + t] = (int32_t)a;
+      continue;
+    }
     if (m >= M || n >= N) continue;
-    if constexpr (ZP) a += z.kcc + (uint32_t)z.cA * (uint32_t)sum_b[col] + (uint32_t)z.cB * (uint32_t)sum_a[row];
     int64_t at = o_base + (int64_t)m * N + n;
     if (e.col_blk > 0) {
       const unsigned blk = (unsigned)n / (unsigned)e.col_blk;
@@ -412,6 +419,25 @@ void k_qgemm_wk(const int8_t* __restrict__ A, const int8_t* __restrict__ B, int 
       if (e.out_q8) static_cast<int8_t*>(out)[at] = (int8_t)requant(y, e);
       else static_cast<float*>(out)[at] = y;
     }
+  }
+}
+
+// The splits' partial sums of a 32 x 32 tile, stored as k_qgemm_wk does.
+__global__ __launch_bounds__(256) void k_wk_finish(int M, int N, int tiles_m, int tiles_n, GemmEpi e, AnyPlan p,
+                                                   void* __restrict__ out) {
+  int tm, tn;
+  tile_of((int)blockIdx.x, tiles_m, tiles_n, tm, tn);
+  const int64_t step = (int64_t)gridDim.y * gridDim.x * (WKB * WKB);
+  const int32_t* part = p.part + ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * (WKB * WKB);
+  void* o = static_cast<char*>(out) + blockIdx.y * p.o_step * (e.out_q8 ? 1 : 4);
+  for (int t = threadIdx.x; t < WKB * WKB; t += 256) {
+    const int m = tm * WKB + t / WKB, n = tn * WKB + t % WKB;
+    uint32_t a = 0u;
+    for (int s = 0; s < p.splits; s += 4) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) a += s + q < p.splits ? (uint32_t)part[(s + q) * step + t] : 0u;
+    }
+    if (m < M && n < N) store_out(o, (int64_t)m * N + n, (int)a, m, n, e);
   }
 }
 
@@ -485,16 +511,41 @@ hipError_t launch_any_tile(const int8_t* A, const int8_t* B, int M, int N, int K
 hipError_t launch_wk(const int8_t* A, const int8_t* B, int M, int N, int K, const GemmEpi& e,
                      const AffineDot* z, const AnyPlan& p, void* out, hipStream_t st) {
   const int tm = (M + WKB - 1) / WKB, tn = (N + WKB - 1) / WKB;
-  const dim3 grid((unsigned)(tm * tn), (unsigned)p.groups), block(64 * WKW);
+  const dim3 grid((unsigned)(tm * tn), (unsigned)p.groups, (unsigned)p.splits), block(64 * WKW);
   const unsigned lds = WK_LDS + (p.conv_cg ? (unsigned)K / 4 : 0u);
   note_route(p.conv_cg ? "any conv" : "any", WKB, WKB, WKW);
   const AffineDot zz = z ? *z : AffineDot{};
   Q8_ANY_LAUNCH(k_qgemm_wk, );
+  hipError_t err = hipGetLastError();
+  if (err != hipSuccess || p.splits == 1) return err;
+  note_route("any conv split", WKB, WKB, p.splits);
+  hipLaunchKernelGGL(k_wk_finish, dim3((unsigned)(tm * tn), (unsigned)p.groups), dim3(256), 0, st, M, N, tm, tn, e, p, out);
   return hipGetLastError();
 }
 #undef Q8_ANY_LAUNCH
 
 }  // namespace
+
+// With fewer tiles than CUs and a long K, the time is what one CU can load
+// (2, 4, 6 and 8 steps in flight take the same): the K of the tiles is spread
+// over up to 8 workgroups each, at least 8 slices of 128 bytes to one, whose
+// sums cost a second launch.  Whole convs of one image, us, unsplit / split: 512
+// x 7 x 7 -> 16, 7 x 7 (2 tiles, K 25088) 42.3 / 17.8; 256 x 13 x 13 -> 3, 7 x 7
+// (6, 12544) 21.8 / 15.1; 1024 x 14 x 14 -> 10, 3 x 3 (7, 9216) 19.2 / 15.5; 256
+// x 28 x 28 -> 3, 5 x 5 (25, 6400) 14.8 / 14.3; 512 x 7 x 7 -> 512, 3 x 3 (32,
+// 4608) 15.5 / 13.7; below, 192 x 13 x 13 -> 64, 5 x 5 (12, 4800) 12.8 / 13.9, 256
+// x 14 x 14 -> 256, 3 x 3 (56, 2304) 11.9 / 13.7.
+int any_splits(int64_t M, int64_t N, int64_t K, int64_t groups) {
+  const int64_t cus = cu_count() > 0 ? cu_count() : 256, t32 = groups * ((M + 31) / 32) * ((N + 31) / 32);
+  if (K < ANY_SPLIT_K || 2 * t32 > cus) return 1;
+  int64_t s = cus / t32;
+  s = s < 8 ? s : 8;
+  s = s < K / 1024 ? s : K / 1024;
+  return (int)s;
+}
+size_t any_part_bytes(int64_t M, int64_t N, int64_t groups, int splits) {
+  return splits > 1 ? (size_t)splits * (size_t)groups * (size_t)((M + 31) / 32) * (size_t)((N + 31) / 32) * WKB * WKB * 4 : 0;
+}
 
 hipError_t launch_gemm_any(const int8_t* A, const int8_t* B, int64_t M, int64_t N, int64_t K,
                            const GemmEpi& e, const AffineDot* z, const AnyPlan& p, void* out, hipStream_t st) {
@@ -528,6 +579,7 @@ hipError_t launch_gemm_any(const int8_t* A, const int8_t* B, int64_t M, int64_t 
   const int KT = (k + AK - 1) / AK;
   const bool big = M > 64 && N > 64 && KT >= 6;
   const int64_t t32 = p.groups * ((M + 31) / 32) * ((N + 31) / 32);
+  if (p.splits > 1 && (t32 > cus || K < 16 || p.part == nullptr)) return hipErrorInvalidValue;
   if (t32 <= cus && K >= 16) return launch_wk(A, B, m, n, k, e, z, p, out, st);
   if (KT > 2) {
     if (t64 <= cus) return launch_any_tile<64, 64, 4>(A, B, m, n, k, e, z, p, out, st);

@@ -138,7 +138,15 @@ struct AnyPlan {
   int groups = 1;
   int64_t a_step = 0, b_step = 0, o_step = 0;   // bytes, bytes, output elements
   int conv_cg = 0;
+  // K split over workgroups: `splits` partial sums of every 32 x 32 tile in
+  // `part` (any_part_bytes), added up by a second launch
+  int splits = 1;
+  int32_t* part = nullptr;
 };
+// How many ways the K of a product of few tiles is split (1: not), and the
+// bytes of its partial sums.
+int any_splits(int64_t M, int64_t N, int64_t K, int64_t groups);
+size_t any_part_bytes(int64_t M, int64_t N, int64_t groups, int splits);
 hipError_t launch_gemm_any(const int8_t* A, const int8_t* B, int64_t M, int64_t N, int64_t K,
                            const GemmEpi& e, const AffineDot* z, const AnyPlan& p, void* out, hipStream_t st);
 inline hipError_t launch_gemm_any(const int8_t* A, const int8_t* B, int64_t M, int64_t N, int64_t K,
@@ -230,6 +238,8 @@ struct ConvPlan {
   int64_t nb = 0;     // images of one pass
   size_t skip = 0;    // bytes up to the workspace's first 16-byte boundary
   size_t wt = 0;      // bytes of the weight's form that the GEMM reads (tap-major, or padded rows)
+  int splits = 1;     // of K, their partial sums
+  size_t part = 0;    // from this offset on
   size_t bytes = 0;   // of the workspace from its start: nothing past them is written
 };
 ConvPlan conv_plan(const ConvGeom& G, const void* ws, size_t ws_bytes, bool prepacked);

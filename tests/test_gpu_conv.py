@@ -379,3 +379,32 @@ def test_conv_pointwise(ops, oracle, xs, o, route, w_shift):
     same_bits(got, want)
     got = conv_call(x, w, [1, 1], [[0, 0], [0, 0]], w_shift=w_shift, s_out=1.7e-4)
     same_bits(got, (want.astype(np.float64) * 1.7e-4).astype(np.float32))
+
+
+# Few tiles over a long contraction: K split over workgroups, its partial sums
+# behind the rest of the workspace; without room for them, unsplit
+SPLIT_K = [((1, 256, 13, 13), (3, 256, 7, 7), 1), ((2, 1024, 7, 7), (66, 1024, 3, 3), 1),
+           ((1, 1024, 7, 9), (40, 512, 3, 3), 2), ((1, 2048, 7, 7), (16, 2048, 3, 3), 1),
+           ((1, 100, 9, 9), (17, 100, 7, 7), 1), ((3, 300, 6, 5), (34, 150, 5, 7), 2)]
+
+
+@pytest.mark.parametrize("xs,ws,g", SPLIT_K)
+@pytest.mark.parametrize("u8", [False, True])
+def test_conv_split_k(ops, oracle, xs, ws, g, u8):
+    import ctypes as C
+    from mlfw_amd import _lib as L
+    rng = np.random.default_rng(sum(xs) + u8)
+    x = rng.integers(0, 256, xs).astype(np.uint8)
+    x = x if u8 else x.view(np.int8)
+    w = rng.integers(-128, 128, ws).astype(np.int8)
+    pd, zp = [[ws[2] // 2] * 2, [ws[3] // 2] * 2], 77 if u8 else 0
+    want = oracle.quantized_conv(x, w, [1, 1], pd, [1, 1], g, zp, 0)
+    same_bits(conv_call(x, w, [1, 1], pd, g, zpx=zp), want)
+    assert ops.last_gemm().startswith("any conv split"), ops.last_gemm()
+    same_bits(conv_call(x, w, [1, 1], pd, g, zpx=zp, s_out=1.7e-4), (want.astype(np.float64) * 1.7e-4).astype(np.float32))
+    arr = lambda v: (C.c_int64 * len(v))(*v)  # noqa: E731
+    need = C.c_size_t(0)
+    p = arr([q[0] for q in pd])
+    L.call("q8_quantized_conv_workspace", 2, arr(xs), arr(ws), arr([1, 1]), p, p, arr([1, 1]), g, C.byref(need))
+    same_bits(conv_call(x, w, [1, 1], pd, g, zpx=zp, ws_bytes=need.value - 4096), want)
+    assert ops.last_gemm().startswith("any"), ops.last_gemm()
