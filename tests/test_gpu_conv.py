@@ -1,19 +1,14 @@
 """GPU parity of quantized_conv (q8_quantized_conv) against the CPU oracle.
 
 int32 accumulators and fp32 dequantized outputs are compared bit for bit.
-The cases cover both device paths (direct kernel for contractions shorter
-than 64, im2col + MFMA GEMM otherwise, with and without a contraction that
-is a multiple of 16), the GEMV and the GEMM kernels behind the latter
-(<= 16 and > 16 output channels per group), groups / depthwise, strides,
-asymmetric padding, dilation, batch > 1 (batches of images in one GEMM
-whose epilogue scatters columns to images, with 16-byte and with
-per-element stores; one image at a time for the GEMV), spatial ranks 1 to
-3, and the three GEMM forms of the contraction: the byte-gather im2col
-(channels per group not a multiple of 16), the channel-last frame with a
-tap-major im2col (1 x 1 kernels use the frame itself), and the implicit
-GEMM reading the frame (channels per group a multiple of 64), with and
-without a split of K; zero
-points and ui8 operands; then the whole pipeline QuantizationPass builds
+The cases cover the device paths (the direct kernel for short contractions
+of little work, else a GEMM), groups / depthwise, strides, asymmetric
+padding, dilation, batch > 1 (images in one GEMM whose epilogue scatters
+columns to images, with 16-byte and with per-element stores), spatial ranks
+1 to 3, the byte-gather im2col (channels per group not a multiple of 16) and
+the channel-last frame, each GEMM kernel and tile behind them (the route is
+asserted where a case is for one), passes over parts of a batch, a split of
+K, misaligned weights and workspaces; zero points and ui8 operands; then the whole pipeline QuantizationPass builds
 for a conv (quantize input, quantize kernel, quantized_conv, dequantize).
 """
 import numpy as np
@@ -66,7 +61,7 @@ CASES = [
     ((1, 64, 10), (64, 1, 3), [1], [[1, 1]], [2], 64),                       # depthwise 1-D
     ((2, 64, 12, 12), (32, 64, 3, 3), [1, 1], [[1, 1], [1, 1]], [1, 1], 1),  # GEMM (Kc 576)
     ((1, 20, 11, 13), (48, 10, 3, 3), [1, 2], [[0, 2], [1, 0]], [1, 1], 2),  # GEMM, Kc 90 -> 96, groups
-    ((3, 16, 7, 9), (8, 16, 2, 3), [1, 1], [[1, 0], [0, 0]], [2, 1], 1),     # GEMV (Og 8), Kc 96
+    ((3, 16, 7, 9), (8, 16, 2, 3), [1, 1], [[1, 0], [0, 0]], [2, 1], 1),     # 8 outputs, Kc 96
     ((1, 8, 6, 5, 7), (24, 8, 2, 3, 2), [1, 2, 1], [[1, 0], [0, 1], [1, 1]], [1, 1, 2], 1),  # 3-D
     ((1, 256, 14, 14), (300, 256, 1, 1), [1, 1], [[0, 0], [0, 0]], [1, 1], 1),  # 1x1, tile edges
     # batched im2col + column-blocked GEMM (N > 1, Og > 16)
@@ -80,9 +75,9 @@ CASES = [
     ((2, 16, 5, 6, 7), (32, 16, 2, 3, 2), [1, 2, 1], [[1, 0], [0, 1], [1, 1]], [1, 1, 2], 1),  # 3-D
     ((3, 64, 9, 9), (40, 64, 1, 1), [2, 2], [[0, 0], [0, 0]], [1, 1], 1),    # 1x1 at stride 2
     ((2, 48, 6, 6), (24, 48, 1, 1), [1, 1], [[1, 1], [0, 2]], [1, 1], 1),    # 1x1 padded: frame is B
-    # implicit GEMM split over K (few tiles, long contraction)
-    ((2, 64, 9, 9), (48, 64, 5, 5), [1, 1], [[2, 2], [2, 2]], [1, 1], 1),    # 3 splits, K % 128 = 64
-    ((2, 256, 6, 6), (96, 128, 3, 3), [1, 1], [[1, 1], [1, 1]], [1, 1], 2),  # 2 splits, groups
+    # few tiles, longer contractions
+    ((2, 64, 9, 9), (48, 64, 5, 5), [1, 1], [[2, 2], [2, 2]], [1, 1], 1),    # Kc 1600, K % 128 = 64
+    ((2, 256, 6, 6), (96, 128, 3, 3), [1, 1], [[1, 1], [1, 1]], [1, 1], 2),  # Kc 1152, groups
 ]
 
 
@@ -408,3 +403,37 @@ def test_conv_split_k(ops, oracle, xs, ws, g, u8):
     L.call("q8_quantized_conv_workspace", 2, arr(xs), arr(ws), arr([1, 1]), p, p, arr([1, 1]), g, C.byref(need))
     same_bits(conv_call(x, w, [1, 1], pd, g, zpx=zp, ws_bytes=need.value - 4096), want)
     assert ops.last_gemm().startswith("any"), ops.last_gemm()
+
+
+# Each GEMM kernel and tile behind a conv (256 CUs): x, outputs, kernel edge,
+# stride, pad, ui8 input, route
+TILES = [((21, 64, 28, 28), 64, 3, 1, 1, False, "conv 64x64"), ((43, 64, 28, 28), 130, 3, 1, 1, False, "conv 128x128"),
+         ((11, 3, 112, 112), 64, 7, 2, 3, False, "qgemm 64x64"), ((11, 3, 111, 113), 33, 7, 2, 3, False, "qgemm 64x64"),
+         ((11, 3, 112, 112), 64, 7, 2, 3, True, "any 64x64"), ((8, 64, 28, 28), 64, 3, 1, 1, True, "any conv 64x64 k4"),
+         ((9, 96, 27, 28), 61, 3, 1, 1, False, "any conv 64x64 k4"), ((21, 64, 28, 28), 64, 3, 1, 1, True, "any conv 64x64 k2"),
+         ((22, 96, 27, 28), 61, 3, 1, 1, False, "any conv 64x64 k2"), ((21, 16, 28, 28), 64, 3, 1, 1, False, "any conv 64x64 k1"),
+         ((21, 16, 28, 28), 63, 3, 1, 1, True, "any conv 64x64 k1"),
+         ((32, 128, 28, 28), 128, 3, 1, 1, True, "any conv 128x128 k2"), ((33, 96, 27, 28), 127, 3, 1, 1, False, "any conv 128x128 k2"),
+         ((42, 96, 28, 28), 128, 3, 1, 1, True, "any conv 128x128 k1"), ((44, 96, 27, 29), 125, 3, 1, 1, False, "any conv 128x128 k1")]
+
+
+@pytest.mark.parametrize("xs,o,k,st,pad,u8,route", TILES)
+def test_conv_tiles(ops, xs, o, k, st, pad, u8, route):
+    """int32 and fp32 outputs, weights as given and prepacked, against a
+    float64 convolution on the CPU (exact: sums below 2^53)."""
+    rng = np.random.default_rng(sum(xs) + o)
+    x = rng.integers(0, 256, xs).astype(np.uint8)
+    x = x if u8 else x.view(np.int8)
+    w = rng.integers(-128, 128, (o, xs[1], k, k)).astype(np.int8)
+    zp = 117 if u8 else 0
+    print(f"conv tiles {route} x{xs} o{o} k{k}", flush=True)
+    want = torch.nn.functional.conv2d(torch.from_numpy(x.astype(np.float64) - zp), torch.from_numpy(w.astype(np.float64)),
+                                      stride=st, padding=pad).numpy().astype(np.int32)
+    dx, dw, pd = dev(x), dev(w), [[pad, pad]] * 2
+    wt = None if u8 else ops.conv_weight_taps(dw)
+    for taps in {None, wt}:
+        got = ops.quantized_conv(dx, dw, [st, st], pd, zpx=zp, w_taps=taps)
+        assert ops.last_gemm().startswith(route), ops.last_gemm()
+        same_bits(host(got), want)
+        got = ops.quantized_conv(dx, dw, [st, st], pd, zpx=zp, w_taps=taps, s_out=1.7e-4)
+        same_bits(host(got), (want.astype(np.float64) * 1.7e-4).astype(np.float32))

@@ -38,8 +38,9 @@ def host(t):
 
 # K: below a chunk, a chunk and one past, stage edges, several stages with a remainder
 KS = [1, 3, 15, 17, 31, 127, 129, 255, 300, 1001]
-# M, N: one element, tile edges, one tile column; 17 x 17 tiles of 64 take the
-# two-group form, 33 x 17 the 128-wide tile
+# M, N: one element, tile edges, one tile column: K of 64 and more takes a 32 x
+# 32 tile with K split over 8 waves, shorter rows a thread per output (the
+# tiled kernel: test_tiled)
 MNS = [(1, 1), (16, 65), (17, 64), (63, 129), (130, 68)]
 
 
@@ -163,3 +164,37 @@ def test_affine_routes(ops, oracle, M, N, K, kind, route):
     assert ops.last_gemm().startswith(route), ops.last_gemm()
     want = (A.astype(np.float64) - za) @ (B.astype(np.float64) - zb).T      # exact: sums below 2^53
     np.testing.assert_array_equal(got, want.astype(np.int64).astype(np.int32))
+
+
+# The tiled kernel in each of its forms (256 CUs): K below a chunk, just past a
+# stage, with remainders; quads and single columns stored
+TILED = [(4096, 2047, 1, "any 64x64 k1"), (2048, 2048, 15, "any 64x64 k1"), (700, 801, 129, "any 64x64 k1"),
+         (2100, 1071, 300, "any 64x64 k1"), (700, 804, 257, "any 64x64 k4"), (701, 801, 300, "any 64x64 k4"),
+         (640, 900, 1001, "any 64x64 k4"), (1030, 1072, 257, "any 64x64 k2"), (1030, 1071, 1001, "any 64x64 k2"),
+         (2100, 1072, 769, "any 128x128 k2"), (2099, 1071, 901, "any 128x128 k2"),
+         (2100, 2300, 769, "any 128x128 k1"), (2101, 2303, 1001, "any 128x128 k1")]
+
+
+@pytest.mark.parametrize("M,N,K,route", TILED)
+def test_tiled(ops, oracle, M, N, K, route):
+    rng = np.random.default_rng(M + N + K)
+    A = rng.integers(0, 256, (M, K)).astype(np.uint8)
+    B = rng.integers(0, 256, (N, K)).astype(np.uint8)
+    dot = lambda a, b, za=0, zb=0: ((a.astype(np.float64) - za) @ (b.astype(np.float64) - zb).T).astype(np.int64).astype(np.int32)  # noqa: E731  exact: sums below 2^53
+    Ai, Bi = A.view(np.int8), B.view(np.int8)
+    print(f"tiled {route} M={M} N={N} K={K}", flush=True)
+    for a, b, za, zb in ((Ai, Bi, 0, 0), (A, Bi, 121, 0), (Ai, B, -3, 130), (A, B, 7, 250)):
+        np.testing.assert_array_equal(host(ops.quantized_dot(dev(a), dev(b), za, zb)), dot(a, b, za, zb))
+        assert ops.last_gemm() == route, ops.last_gemm()
+    acc = dot(Ai, Bi)
+    sA, sB = rng.uniform(1e-3, 0.05, M), rng.uniform(1e-4, 0.02, N)
+    bias = rng.uniform(-1, 1, N).astype(np.float32)
+    da, db, dbias = (torch.from_numpy(v).to(DEV) for v in (sA, sB, bias))
+    for act in ("none", "relu", "silu"):
+        want = oracle.epilogue(acc, "rowcol", sA, sB, bias=bias, act=act)
+        got = host(ops.qlinear(dev(Ai), da, dev(Bi), db, bias=dbias, act=act))
+        np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
+    y = oracle.epilogue(acc, "rowcol", sA, sB, act="relu")
+    s_next = float(np.abs(y).max() / 127.0)
+    got = host(ops.qlinear_requant(dev(Ai), da, dev(Bi), db, s_next, act="relu"))
+    np.testing.assert_array_equal(got, oracle.quantize(y.reshape(-1), s_next).reshape(M, N))

@@ -170,3 +170,23 @@ def test_gemm_w4(ops, oracle, M, N, K, g):
         got = host(ops.qlinear_w4(dev(xq), dev(sx), wq, sw, K, g, bias=None if b is None else dev(b), act=act))
         want = oracle.gemv_w4(xq, sx, host(wq), host(sw), K, g, bias=b, act=act)
         assert got.tobytes() == want.tobytes(), np.count_nonzero(got != want)
+
+
+# The tiled GEMM over several windows of 16 groups' scales, with an odd number
+# of 128-code steps: groups of one step, of half and a quarter of one, and of
+# two and three; each of the three tiles.  The route is asserted.
+@pytest.mark.parametrize("M,N,K,g,tile", [(130, 4100, 128 * 19, 128, "32x32"), (130, 4099, 32 * 37, 32, "32x32"),
+                                          (100, 3001, 64 * 39, 64, "32x32"), (130, 4100, 256 * 19, 256, "32x32"),
+                                          (129, 4097, 384 * 17, 384, "32x32"), (97, 9001, 32 * 69, 32, "32x64"), (130, 6001, 256 * 19, 256, "32x64"),
+                                          (500, 4090, 128 * 35, 128, "64x64"), (501, 4091, 64 * 37, 64, "64x64")])
+def test_gemm_w4_scale_windows(ops, oracle, M, N, K, g, tile):
+    rng = np.random.default_rng(M + N + K + g)
+    W = (rng.standard_normal((N, K)) * 0.02).astype(np.float32)
+    xq = rng.integers(-128, 128, (M, K)).astype(np.int8)
+    sx = rng.uniform(1e-3, 0.05, M)
+    wq, sw = ops.pack_weight_int4(dev(W), g)
+    print(f"gemm w4 windows M={M} N={N} K={K} g={g}", flush=True)
+    got = host(ops.qlinear_w4(dev(xq), dev(sx), wq, sw, K, g))
+    assert ops.last_gemm() == "w4 " + tile, ops.last_gemm()
+    want = oracle.gemv_w4(xq, sx, host(wq), host(sw), K, g)
+    assert got.tobytes() == want.tobytes(), np.count_nonzero(got != want)
