@@ -457,9 +457,10 @@ int q8_gemv_w4(const int8_t* xq, const double* sx, int sx_mode, const uint8_t* W
  * Zero points (the op's input_zero_point / kernel_zero_point) run the same
  * kernels, exact for any value.
  * workspace: device memory of q8_quantized_conv_workspace bytes (may be 0:
- * then NULL is accepted).  A call with zero points is accepted with less and
- * then takes a slower kernel, one thread per output.  Calls that share a
- * workspace must be ordered (same stream). */
+ * then NULL is accepted), at any address.  With less the call runs in several
+ * passes over images and groups, or in a slower kernel, one thread per output;
+ * symmetric convs with prod(K) * C / groups >= 64 are refused below one image
+ * of one group.  Calls that share a workspace must be ordered (same stream). */
 int q8_quantized_conv_workspace(int spatial_dims, const int64_t* x_shape, const int64_t* w_shape,
                                 const int64_t* strides, const int64_t* pad_lo,
                                 const int64_t* pad_hi, const int64_t* dilation, int64_t groups,

@@ -16,7 +16,8 @@
 //     q8_gemm.  Images go in batches: one GEMM computes [Og, nb * P], its
 //     epilogue storing column n * P + p of the product at image n, position
 //     p (column-blocked output), and the groups are a second grid dimension,
-//     so a grouped conv is two launches, not two per group.  The receptive
+//     so a grouped conv is two launches, not two per group (two per group
+//     where each group's product fills the chip by itself).  The receptive
 //     fields come one of two ways:
 //       - channels per group a multiple of 16: the input is transposed to a
 //         padded channel-last frame and the contraction is taken tap-major
@@ -31,11 +32,13 @@
 //     the way (u - 128), padding holds the input's zero point, and the GEMM
 //     corrects its sums with the operands' row sums (q8_zp.hip states the
 //     identity).  28 x 28 x 128 at batch 32 with ui8 input: 2700 us one
-//     thread per output, 23.6 us here.
+//     thread per output, 21.4 us here.
 //   * a direct kernel (one thread per output element) for other short
 //     contractions -- depthwise and other small-group convolutions -- for an
-//     input zero point outside its type, and for affine calls that bring
-//     less workspace than the GEMM needs.
+//     input zero point outside its type, and for calls whose workspace is so
+//     small that the GEMM's passes do not fit or pay.
+// conv_plan decides the route, the images and groups of a pass and every byte
+// of the workspace that is written.
 // Spatial ranks 1..3 share the code: unused trailing dimensions have size 1,
 // stride 1, no padding and dilation 1.
 #include "q8_device.h"
@@ -349,7 +352,7 @@ bool conv_uses_gemm(const ConvGeom& G) { return G.Kc >= 64 && conv_gemm_fits(G);
 // Short contractions (Cg * prod(K) < 64) that the GEMM still serves better
 // than one thread per output: from 2^24 multiply-adds on (the direct kernel
 // does about 1.2e12 a second: 32 x 3 x 112 x 112 -> 32, 3 x 3, takes 299 us
-// direct and 44 us as im2col + GEMM; 8 x 3 x 56 x 56 -> 32 26 and 13 us)
+// direct and 72 us as im2col + GEMM; 8 x 3 x 56 x 56 -> 32 26 and 12 us)
 // with at least 8 output channels per group in a 64-row tile.
 static bool conv_short_gemm(const ConvGeom& G) {
   return G.Kc < 64 && G.Og >= 8 && conv_gemm_fits(G) &&

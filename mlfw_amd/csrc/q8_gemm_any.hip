@@ -21,9 +21,9 @@
 // passes the flips, row sums and correction were up to four more launches.
 //
 // Measured (MI355X, whole calls, before: one thread per output with byte
-// loads): quantized_dot 788 x 1000 x 1500 with ui8 activations 4350 -> 16.5
-// us (the host's share of the call is about 12); dynamic linear 42 x 3777 x
-// 7986 5400 -> 51 us, 1183 x 3917 x 3001 59300 -> 79 us.
+// loads): quantized_dot 788 x 1000 x 1500 with ui8 activations 4350 -> 12.9
+// us (the host's share of the call; 9.1 replayed from a graph); dynamic linear
+// 42 x 3777 x 7986 5400 -> 57 us, 1183 x 3917 x 3001 59300 -> 72 us.
 #include <type_traits>
 
 #include "q8_device.h"
