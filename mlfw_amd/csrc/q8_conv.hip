@@ -405,17 +405,21 @@ static bool conv_im2col_many(const ConvGeom& G) {
 }
 
 // Groups one after another, each through the direct-to-LDS GEMM, where a
-// group's product alone fills the chip with 128 x 128 tiles: that GEMM's lead
-// over the one launch for all groups then pays for a frame and a GEMM launch
-// a group (3 x 3: 64 x 512 x 28 x 28 -> 512 in two groups 122 us against 153,
-// 8 x 256 x 56 x 56 -> 512 45 and 55, 32 x 256 x 28 x 28 -> 256, 196 tiles a
-// group, 39 and 33; 1 x 1, from two tiles per CU on: 64 x 512 x 28 x 28 -> 512
-// 55 and 59, 64 x 256 x 14 x 14 -> 1024, 392 tiles, 33 and 31).
+// group's product alone fills the chip with 128 x 128 tiles.  That GEMM's lead
+// over the one launch for all groups grows with the contraction, and the frame
+// and GEMM launches of every group and the all-groups launch's fuller rounds
+// count against it with every group more: up to one group per 288 of Kc.  Time
+// by group against all at once, 3 x 3, 392 to 784 tiles a group: 256 channels a
+// group 0.80-0.87 in two groups, 0.85-0.95 in four, 0.91-1.01 in eight, 1.04-1.08
+// in sixteen; 128 channels 0.83-0.92, 0.95-1.00, 0.99-1.11; 64 channels 0.89-1.02
+// in two, 0.98-1.13 in three.  Outputs that leave 128-row tiles a quarter empty
+// (192: 0.97-1.01 in two groups, 1.04-1.12 in three), fewer tiles than CUs (32 x
+// 256 x 28 x 28 -> 256 in two groups: 39 against 33 us) and 1 x 1 kernels
+// (0.92-1.08 in two groups, 1.03-1.27 in three) stay with the one launch.
 static bool conv_by_group(const ConvGeom& G) {
-  if (G.groups == 1 || conv_affine(G) || G.Og < 128) return false;
-  if (!conv_pointwise(G) && (G.Cg % 64 != 0 || G.Kc > 16384)) return false;
-  const int64_t cus = cu_count() > 0 ? cu_count() : 256, t128 = ((G.Og + 127) / 128) * ((G.N * G.Pn + 127) / 128);
-  return t128 >= (conv_pointwise(G) ? 2 * cus : cus);
+  if (G.groups == 1 || conv_affine(G) || conv_pointwise(G) || G.Cg % 64 != 0 || G.Kc > 16384 || G.Og < 128) return false;
+  const int64_t cus = cu_count() > 0 ? cu_count() : 256, rows = (G.Og + 127) / 128;
+  return G.groups * 288 <= G.Kc && G.Og * 8 >= rows * 128 * 7 && rows * ((G.N * G.Pn + 127) / 128) >= cus;
 }
 
 // Workspace bytes of one image and group, and of the weight rows beside them.
