@@ -183,6 +183,7 @@ struct Epi {
   static constexpr bool COLBLK = (EPI & 128) != 0;   // GemmEpi::col_blk addressing
   static constexpr bool IMPL = (EPI & 256) != 0;     // B is a conv frame (GemmEpi::cb)
   static constexpr bool GLU = (EPI & 512) != 0;      // gate|up interleaved, h = silu(g) * u out
+  static constexpr bool LONGK = (EPI & 1024) != 0;   // conv over 16 K stages or more
   static constexpr int MODE = (EPI >> 3) & 1;
   static constexpr bool BIAS = (EPI & 4) != 0;
   static constexpr int ACT = EPI & 3;
@@ -397,12 +398,14 @@ void k_qgemm(const int8_t* __restrict__ A, const int8_t* __restrict__ B, int M, 
   stage_sync_keep<NV>();                          // stage 0 landed
   v4i fa0[C::TM], fb0[C::TN], fa1[C::TM], fb1[C::TN];
   read_frags(buf(0), 0, fa0, fb0);
-  // The conv form must not have its first iteration peeled: the loop is then
-  // one basic block in which every fragment read waits right before its MFMA
-  // (1280 channels at 32 x 32, one image: 64 x 64 tile 63.9 us peeled, 60.5
-  // not), so its first stage is a number the compiler does not know.
+  // The conv form over many stages must not have its first iteration peeled:
+  // the loop is then one basic block in which every fragment read waits right
+  // before its MFMA (1280 channels at 32 x 32, one image, 90 stages: 64 x 64
+  // tile 63.9 us peeled, 60.5 not; 256 at 14 x 14, 18 stages: 22.1 and 21.4), so
+  // its first stage is a number the compiler does not know.  Over few stages
+  // the peeled one saves more (128 at 28 x 28, 9 stages: 19.2 and 19.8).
   int first = 0;
-  if constexpr (IMPL) asm volatile("" : "+s"(first));
+  if constexpr (Epi<EPI>::LONGK) asm volatile("" : "+s"(first));
   for (int kt = first; kt < KT; ++kt) {
     int8_t* cur = buf(kt);
     // sub-step 0; the second half of stage kt+1's copies (stage 1 went out
@@ -1108,7 +1111,7 @@ static hipError_t launch_qgemm_tile(const int8_t* A, const int8_t* B, int M, int
 // Implicit conv GEMM (B a conv frame): column-blocked i32 and per-tensor f32
 // dequant outputs, on the tiles whose register budget has room for the
 // per-column frame offsets.
-#define Q8_EPI_CODES_CONV(X) X(384) X(400)
+#define Q8_EPI_CODES_CONV(X) X(384) X(400) X(1408) X(1424)
 
 std::atomic<long long> g_generic_gemm_launches{0};
 thread_local GemmRoute g_route;
@@ -1167,7 +1170,7 @@ hipError_t launch_gemm_conv(const int8_t* A, const int8_t* frame, int64_t M, int
   if ((int64_t)tm * tn >= ((int64_t)1 << 31) / GEMM_THREADS) return hipErrorInvalidValue;
   const dim3 grid((unsigned)(tm * tn)), block(GEMM_THREADS);
   note_route("conv", bm, bm);
-  const int code = epi_code(e) | 256;
+  const int code = epi_code(e) | 256 | (K >= 16 * BK ? 1024 : 0);
   hipError_t err = hipErrorInvalidValue;
   constexpr int lds128 = qgemm_lds<128, 128>(), lds64 = qgemm_lds<64, 64>();
 #define Q8_CONV_LAUNCH(BMV, codev)                                                                \
