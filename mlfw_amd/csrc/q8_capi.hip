@@ -590,7 +590,7 @@ QdotPlan qdot_plan(int64_t M, int64_t N, int64_t K, int a_dtype, int b_dtype, in
 // 170 and 214, 4096 x 4096 x 4096 109 and 108, 2048 x 4096 x 4096 65 and 56.
 //   Up to 16 tokens the GEMV reads B once at about 6 TB/s; the one launch's 32
 // x 32 tiles (8192 columns and fewer) are a chain over K, its 64 x 64 ones
-// read 3.9 TB/s.  One flip of A, 4 x 4096 x 11008: 13.0 us in passes, 20.1 in
+// read 3.9 TB/s from HBM and 5.4 from the MALL.  One flip of A, 4 x 4096 x 11008: 13.0 us in passes, 20.1 in
 // one launch; 4 x 256 x 256 4.2 and 3.0.  Row sums of B are a second read of
 // it: 4 x 4096 x 11008 27.1 and 20.1.  A call made by itself keeps the host
 // busy for 13 us and 2.7 more for each pass, so a product below that stays
@@ -603,13 +603,13 @@ bool qdot_passes(const QdotPlan& p, int64_t M, int64_t N, int64_t K) {
     if (mn < 0x1p21) return false;
     lead = 5e-7 * mn + 5.5e-10 * mn * k;
   } else {
-    const double chain = N <= 8192 ? k * (1.2e-3 + 4e-5 * m) + 8e-8 * n * k : 0.0, read = n * k / 3.9e6;
+    const double chain = N <= 8192 ? k * (1.2e-3 + 4e-5 * m) + 8e-8 * n * k : 0.0, read = n * k / 4.4e6;
     const double one = 2.7 + (chain > read ? chain : read);
-    if (one < 13.0) return false;
+    if (one < 12.5) return false;
     lead = one - 2.2 - n * k / 6e6 - (M > 4 ? 5.5e-4 * k : 0.0);
     rate = 4e6;
     flip = 1.6;
-    sums = 2.2;
+    sums = 4.5;
   }
   double cost = 0.0;
   if (p.a_u8) cost += flip + 2.0 * m * k / rate;

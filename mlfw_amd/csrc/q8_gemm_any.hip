@@ -269,9 +269,9 @@ void k_qgemm_any(const int8_t* __restrict__ A, const int8_t* __restrict__ B, int
 // this form lose: 64 x 11008 x 4096 takes 25 us with 64 x 64, 21 staged.)
 constexpr int WKT = 2, WKW = 8, WKB = 16 * WKT;       // 16-row blocks, waves, tile edge
 constexpr int WK_PITCH = WKB + 4;
-constexpr int ANY_SPLIT_K = 4096;
+constexpr int ANY_SPLIT_K = 5120;
 constexpr int WK_LDS = WKT * WKW * 16 * WK_PITCH * 4 + 8 * WKB + 8 * WKB;
-template <bool ZP, bool CONV>
+template <bool SPLIT, bool ZP, bool CONV>
 __global__ __launch_bounds__(64 * WKW, 2)
 void k_qgemm_wk(const int8_t* __restrict__ A, const int8_t* __restrict__ B, int M, int N, int K,
                 int tiles_m, int tiles_n, GemmEpi e, AffineDot z, AnyPlan p, void* __restrict__ out) {
@@ -356,9 +356,10 @@ void k_qgemm_wk(const int8_t* __restrict__ A, const int8_t* __restrict__ B, int 
       }
     }
   };
-  // blockIdx.z: the split; its waves take every 8 * splits-th slice
+  // SPLIT: split blockIdx.z of gridDim.z, whose waves take every 8 * splits-th
+  // slice (a form of its own: 3% on products of a few microseconds)
   Frag f0, f1;
-  const int zs = (int)blockIdx.z, stride = 2 * WKW * (int)gridDim.z;
+  const int zs = SPLIT ? (int)blockIdx.z : 0, stride = 2 * WKW * (SPLIT ? (int)gridDim.z : 1);
   int s = 2 * (wave + WKW * zs);
   if (s < KS) load(s, f0);
   while (s < KS) {
@@ -400,7 +401,7 @@ void k_qgemm_wk(const int8_t* __restrict__ A, const int8_t* __restrict__ B, int 
 #pragma unroll
     for (int w = 0; w < WKW; ++w) a += (uint32_t)red[((row / 16 * WKW + w) * 16 + row % 16) * WK_PITCH + col];
     if constexpr (ZP) a += (zs == 0 ? z.kcc : 0u) + (uint32_t)z.cA * (uint32_t)sum_b[col] + (uint32_t)z.cB * (uint32_t)sum_a[row];
-    if (p.splits > 1) {                                  // uniform
+    if constexpr (SPLIT) {
       p.part[(((int64_t)zs * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x) * (WKB * WKB) + t] = (int32_t)a;
       continue;
     }
@@ -515,9 +516,13 @@ hipError_t launch_wk(const int8_t* A, const int8_t* B, int M, int N, int K, cons
   const unsigned lds = WK_LDS + (p.conv_cg ? (unsigned)K / 4 : 0u);
   note_route(p.conv_cg ? "any conv" : "any", WKB, WKB, WKW);
   const AffineDot zz = z ? *z : AffineDot{};
-  Q8_ANY_LAUNCH(k_qgemm_wk, );
+  if (p.splits == 1) {
+    Q8_ANY_LAUNCH(k_qgemm_wk, false, );
+    return hipGetLastError();
+  }
+  Q8_ANY_LAUNCH(k_qgemm_wk, true, );
   hipError_t err = hipGetLastError();
-  if (err != hipSuccess || p.splits == 1) return err;
+  if (err != hipSuccess) return err;
   note_route("any conv split", WKB, WKB, p.splits);
   hipLaunchKernelGGL(k_wk_finish, dim3((unsigned)(tm * tn), (unsigned)p.groups), dim3(256), 0, st, M, N, tm, tn, e, p, out);
   return hipGetLastError();
@@ -533,7 +538,7 @@ hipError_t launch_wk(const int8_t* A, const int8_t* B, int M, int N, int K, cons
 // x 7 x 7 -> 16, 7 x 7 (2 tiles, K 25088) 42.3 / 17.8; 256 x 13 x 13 -> 3, 7 x 7
 // (6, 12544) 21.8 / 15.1; 1024 x 14 x 14 -> 10, 3 x 3 (7, 9216) 19.2 / 15.5; 256
 // x 28 x 28 -> 3, 5 x 5 (25, 6400) 14.8 / 14.3; 512 x 7 x 7 -> 512, 3 x 3 (32,
-// 4608) 15.5 / 13.7; below, 192 x 13 x 13 -> 64, 5 x 5 (12, 4800) 12.8 / 13.9, 256
+// 4608) 15.5 / 13.7, but 192 x 13 x 13 -> 64, 5 x 5 (12, 4800) 12.8 / 13.9 and 256
 // x 14 x 14 -> 256, 3 x 3 (56, 2304) 11.9 / 13.7.
 int any_splits(int64_t M, int64_t N, int64_t K, int64_t groups) {
   const int64_t cus = cu_count() > 0 ? cu_count() : 256, t32 = groups * ((M + 31) / 32) * ((N + 31) / 32);
@@ -606,10 +611,14 @@ hipError_t setup_any_attributes() {
   Q8_SET_ANY(64, 64, 2)
   Q8_SET_ANY(64, 64, 4)
 #undef Q8_SET_ANY
-  set(reinterpret_cast<const void*>(k_qgemm_wk<false, false>), WK_LDS);
-  set(reinterpret_cast<const void*>(k_qgemm_wk<true, false>), WK_LDS);
-  set(reinterpret_cast<const void*>(k_qgemm_wk<false, true>), WK_LDS + ANY_CONV_MAX_K / 4);
-  set(reinterpret_cast<const void*>(k_qgemm_wk<true, true>), WK_LDS + ANY_CONV_MAX_K / 4);
+#define Q8_SET_WK(SPLIT)                                                                     \
+  set(reinterpret_cast<const void*>(k_qgemm_wk<SPLIT, false, false>), WK_LDS);                   \
+  set(reinterpret_cast<const void*>(k_qgemm_wk<SPLIT, true, false>), WK_LDS);                    \
+  set(reinterpret_cast<const void*>(k_qgemm_wk<SPLIT, false, true>), WK_LDS + ANY_CONV_MAX_K / 4); \
+  set(reinterpret_cast<const void*>(k_qgemm_wk<SPLIT, true, true>), WK_LDS + ANY_CONV_MAX_K / 4);
+  Q8_SET_WK(false)
+  Q8_SET_WK(true)
+#undef Q8_SET_WK
   return err;
 }
 
