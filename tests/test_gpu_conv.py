@@ -326,16 +326,16 @@ def test_conv_in_several_passes(ops, oracle, xs, ws, pd, g, u8):
         same_bits(conv_call(x, w, [1, 1], pd, g, zpx=zp, ws_bytes=size), want)
 
 
-# Symmetric convs in groups whose product fills the chip with 128 x 128 tiles
-# run a group at a time through the direct-to-LDS GEMM; smaller ones, and
-# affine ones, all groups in one launch
+# Symmetric convs in few groups whose product fills the chip with 128 x 128 tiles
+# run a group at a time through the direct-to-LDS GEMM; smaller ones, more
+# groups, ragged outputs, 1 x 1 kernels and affine ones all groups in one launch
 GROUPED = [((44, 128, 28, 28), (256, 64, 3, 3), 2, False, "conv 128x128"),
-           ((43, 128, 28, 28), (300, 64, 3, 3), 2, False, "conv 128x128"),
+           ((22, 128, 27, 29), (480, 64, 3, 3), 2, False, "conv 128x128"),
+           ((43, 128, 28, 28), (300, 64, 3, 3), 2, False, "any conv"),
            ((20, 128, 28, 28), (256, 64, 3, 3), 2, False, "any conv"),
+           ((43, 192, 28, 28), (384, 64, 3, 3), 3, False, "any conv"),
            ((44, 128, 28, 28), (256, 64, 3, 3), 2, True, "any conv"),
-           ((44, 96, 28, 28), (256, 48, 3, 3), 2, False, "any conv"),
-           ((86, 128, 28, 28), (256, 64, 1, 1), 2, False, "qgemm"),
-           ((44, 128, 28, 28), (256, 64, 1, 1), 2, False, "any conv")]
+           ((86, 128, 28, 28), (256, 64, 1, 1), 2, False, "any conv")]
 
 
 @pytest.mark.parametrize("xs,ws,g,u8,route", GROUPED)
@@ -379,8 +379,8 @@ def test_conv_pointwise(ops, oracle, xs, o, route, w_shift):
 # Few tiles over a long contraction: K split over workgroups, its partial sums
 # behind the rest of the workspace; without room for them, unsplit
 SPLIT_K = [((1, 256, 13, 13), (3, 256, 7, 7), 1), ((2, 1024, 7, 7), (66, 1024, 3, 3), 1),
-           ((1, 1024, 7, 9), (40, 512, 3, 3), 2), ((1, 2048, 7, 7), (16, 2048, 3, 3), 1),
-           ((1, 100, 9, 9), (17, 100, 7, 7), 1), ((3, 300, 6, 5), (34, 150, 5, 7), 2)]
+           ((1, 1280, 7, 9), (40, 640, 3, 3), 2), ((1, 2048, 7, 7), (16, 2048, 3, 3), 1),
+           ((1, 108, 9, 9), (17, 108, 7, 7), 1), ((3, 300, 6, 5), (34, 150, 5, 7), 2)]
 
 
 @pytest.mark.parametrize("xs,ws,g", SPLIT_K)
@@ -407,7 +407,8 @@ def test_conv_split_k(ops, oracle, xs, ws, g, u8):
 
 # Each GEMM kernel and tile behind a conv (256 CUs): x, outputs, kernel edge,
 # stride, pad, ui8 input, route
-TILES = [((21, 64, 28, 28), 64, 3, 1, 1, False, "conv 64x64"), ((43, 64, 28, 28), 130, 3, 1, 1, False, "conv 128x128"),
+TILES = [((21, 64, 28, 28), 64, 3, 1, 1, False, "conv 64x64"), ((21, 256, 28, 28), 64, 3, 1, 1, False, "conv 64x64"),
+         ((43, 256, 28, 28), 130, 3, 1, 1, False, "conv 128x128"), ((43, 64, 28, 28), 130, 3, 1, 1, False, "conv 128x128"),
          ((11, 3, 112, 112), 64, 7, 2, 3, False, "qgemm 64x64"), ((11, 3, 111, 113), 33, 7, 2, 3, False, "qgemm 64x64"),
          ((11, 3, 112, 112), 64, 7, 2, 3, True, "any 64x64"), ((8, 64, 28, 28), 64, 3, 1, 1, True, "any conv 64x64 k4"),
          ((9, 96, 27, 28), 61, 3, 1, 1, False, "any conv 64x64 k4"), ((21, 64, 28, 28), 64, 3, 1, 1, True, "any conv 64x64 k2"),

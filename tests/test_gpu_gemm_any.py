@@ -144,7 +144,7 @@ def test_more_tiles_than_a_launch_holds(ops):
 # the correction; a few tokens (GEMV) and many (GEMM)
 AFFINE_ROUTES = [(4, 256, 256, "A", "any"), (4, 256, 4096, "A", "any"), (1, 4096, 11008, "A", "gemv"),
                  (16, 1024, 11008, "A", "gemv"), (4, 4096, 4096, "csB", "any"), (1, 1024, 11008, "B", "gemv"),
-                 (1, 32000, 4096, "rsA", "gemv"), (1, 1024, 11008, "csB", "gemv"), (8, 1024, 1024, "all", "any"),
+                 (1, 32000, 4096, "rsA", "any"), (1, 4096, 11008, "rsA", "gemv"), (1, 1024, 11008, "csB", "gemv"), (8, 1024, 1024, "all", "any"),
                  (17, 4096, 4096, "A", "any"), (512, 4096, 4096, "A", ("qgemm", "ring")), (512, 4096, 4096, "rsA", "any"),
                  (2048, 1024, 1024, "A", "any"), (2048, 4096, 1024, "A", ("qgemm", "ring")),
                  (1024, 4000, 16384, "csB", ("qgemm", "ring")),
